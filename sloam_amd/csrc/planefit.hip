@@ -20,7 +20,8 @@
 //    reference, which fits each cell by SVD without RANSAC): Philox4x32-10
 //    samples of 3 points, plane through them in FP32, inlier |n.p + d| < thr
 //    counted by wavefront ballot; best = max count, lowest index; FP64 PCA
-//    refit over the inliers.  Predicate: Plane::distance(const PointT&)
+//    refit over the inliers.  Large sets are cut into chunks that several
+//    workgroups score and refit.  Predicate: Plane::distance(const PointT&)
 //    (sloam/src/objects/plane.cpp:136-151) for a unit normal.
 #include <cstring>
 
@@ -277,7 +278,12 @@ __global__ __launch_bounds__(kGB) void ground_fit_kernel(
 constexpr int kPlB = 256;
 constexpr int kPlW = kPlB / 64;
 constexpr int kPlHB = 8;
-constexpr int kPlTile = 2048;
+constexpr int kPlTile = 1024;
+constexpr int kPlHyps = 64;         // hypotheses per score workgroup
+constexpr int kPlScore = 1024;      // points per score chunk
+constexpr int kPlScoreMax = 65536;  // score workgroups a batch is cut into at most
+constexpr int kPlRefit = 2048;      // points per refit chunk
+constexpr int kPlMaxChunks = 256;   // refit chunks per set at most
 
 struct PlFrame {
   float m[3];
@@ -332,23 +338,44 @@ __device__ inline bool plane_inlier(float x, float y, float z, const PlHyp& h, f
   return fabsf(t) < thr;
 }
 
-__global__ __launch_bounds__(kPlB) void plane_seed_kernel(const float* __restrict__ xyz,
-                                                          const int32_t* __restrict__ offsets,
-                                                          int n_sets, PlFrame* __restrict__ frames) {
+// The sets are cut twice: into score chunks (the points one workgroup scores
+// kPlHyps hypotheses on) and into refit chunks (kPlRefit points or more, at
+// most kPlMaxChunks a set).  A chunk is {set, first point, points, chunks of
+// the set << 16 | chunk index} with the points relative to the set; an empty
+// set has one empty chunk.
+struct PlChunk {
+  int set, first, n, of;
+  __device__ int count() const { return (int)((uint32_t)of >> 16); }
+  __device__ int index() const { return of & 0xffff; }
+};
+
+// Bounding box of a refit chunk (6 floats per chunk); zeroes what the next
+// kernels accumulate into: the set's counts (its first chunk's workgroup),
+// the arrival counters of the refit and the mask words.
+__global__ __launch_bounds__(kPlB) void plane_box_kernel(
+    const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
+    const PlChunk* __restrict__ chunks, int n_hyp, float* __restrict__ box,
+    int32_t* __restrict__ counts, int2* __restrict__ arrived, uint32_t* __restrict__ mask,
+    long long mask_words) {
   __shared__ float red[kPlW][6];
-  const int c = blockIdx.x;
-  if (c >= n_sets) return;
-  const int off = offsets[c];
-  const int n = offsets[c + 1] - off;
-  const float* P = xyz + 3 * (size_t)off;
+  const PlChunk ck = chunks[blockIdx.x];
+  const float* P = xyz + 3 * ((size_t)offsets[ck.set] + ck.first);
   float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-  for (int i = threadIdx.x; i < n; i += kPlB)
+  for (int i = threadIdx.x; i < ck.n; i += kPlB)
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const float q = P[3 * (size_t)i + k];
       mn[k] = fminf(mn[k], q);
       mx[k] = fmaxf(mx[k], q);
     }
+  if (ck.index() == 0) {
+    for (int h = threadIdx.x; h < n_hyp; h += kPlB) counts[(size_t)ck.set * n_hyp + h] = 0;
+    if (threadIdx.x == 0) arrived[ck.set] = make_int2(0, 0);
+  }
+  if (mask)
+    for (long long w = (long long)blockIdx.x * kPlB + threadIdx.x; w < mask_words;
+         w += (long long)gridDim.x * kPlB)
+      mask[w] = 0u;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
@@ -363,8 +390,38 @@ __global__ __launch_bounds__(kPlB) void plane_seed_kernel(const float* __restric
       red[wave][3 + k] = mx[k];
     }
   __syncthreads();
-  if (threadIdx.x != 0) return;
+  if (threadIdx.x < 6) {
+    const int k = threadIdx.x;
+    float a = red[0][k];
+    for (int w = 1; w < kPlW; ++w) a = k < 3 ? fminf(a, red[w][k]) : fmaxf(a, red[w][k]);
+    box[6 * (size_t)blockIdx.x + k] = a;
+  }
+}
+
+// The set's frame from the boxes of its R refit chunks (minima and maxima:
+// the order does not matter), by every thread of the workgroup.
+__device__ inline PlFrame plane_frame(const float* __restrict__ box, int R, int n,
+                                      float (*red)[6]) {
+  float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  for (int r = threadIdx.x; r < R; r += kPlB)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      const float q = box[6 * (size_t)r + k];
+      v[k] = k < 3 ? fminf(v[k], q) : fmaxf(v[k], q);
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      const float q = __shfl_xor(v[k], o, 64);
+      v[k] = k < 3 ? fminf(v[k], q) : fmaxf(v[k], q);
+    }
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) red[threadIdx.x >> 6][k] = v[k];
+  __syncthreads();
   PlFrame f;
+#pragma unroll
   for (int k = 0; k < 3; ++k) {
     float a = red[0][k], b = red[0][3 + k];
     for (int w = 1; w < kPlW; ++w) {
@@ -374,27 +431,37 @@ __global__ __launch_bounds__(kPlB) void plane_seed_kernel(const float* __restric
     f.m[k] = n > 0 ? 0.5f * (a + b) : 0.0f;
   }
   f.n = n;
-  frames[c] = f;
+  return f;
 }
 
+// Inlier counts of kPlHyps hypotheses (blockIdx.y) over one score chunk.
+// A set's chunks add their counts with integer atomics (any order gives the
+// same counts); a set of one chunk stores them.  A workgroup per set and 256
+// hypotheses, as before, left a scan's ground (one set) on one CU: 457 us at
+// 27,001 points x 200 hypotheses, and the largest patch of a batch set its
+// time (339 us at 300 sets of 40..20,000 points); in chunks of 1,024 points x
+// 64 hypotheses the two take 10.7 us (launch and gather latency) and 29 us
+// (16 us of VALU issue: 3 FMA + 1 compare per point and hypothesis).
 __global__ __launch_bounds__(kPlB) void plane_score_kernel(
     const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
-    const PlFrame* __restrict__ frames, const int4* __restrict__ work, int n_hyp, int hcap,
-    float thr, uint32_t k0, uint32_t k1, uint32_t tag, int32_t* __restrict__ counts,
+    const float* __restrict__ box, const int2* __restrict__ set_chunks,
+    const PlChunk* __restrict__ chunks, int n_hyp, float thr, uint32_t k0, uint32_t k1,
+    uint32_t tag, PlFrame* __restrict__ frames, int32_t* __restrict__ counts,
     int32_t* __restrict__ samples) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  float4* hp = reinterpret_cast<float4*>(smem_raw);
-  int* cnt = reinterpret_cast<int*>(hp + hcap);
-  float* sx = reinterpret_cast<float*>(cnt + hcap);
-  float* sy = sx + kPlTile;
-  float* sz = sy + kPlTile;
-  const int4 w = work[blockIdx.x];
-  const int c = w.x, h0 = w.y, hc = w.z;
+  __shared__ float4 hp[kPlHyps];
+  __shared__ float sx[kPlTile], sy[kPlTile], sz[kPlTile];
+  __shared__ int cnt[kPlHyps];
+  __shared__ float red[kPlW][6];
+  const PlChunk ck = chunks[blockIdx.x];
+  const int c = ck.set, h0 = blockIdx.y * kPlHyps, hc = min(kPlHyps, n_hyp - h0);
   const int off = offsets[c];
   const int n = offsets[c + 1] - off;
   const float* P = xyz + 3 * (size_t)off;
-  const PlFrame f = frames[c];
-  for (int t = threadIdx.x; t < hcap; t += kPlB) {
+  const int2 sc = set_chunks[c];
+  const PlFrame f = plane_frame(box + 6 * (size_t)sc.x, sc.y, n, red);
+  if (ck.index() == 0 && blockIdx.y == 0 && threadIdx.x == 0) frames[c] = f;
+  if (threadIdx.x < kPlHyps) {
+    const int t = threadIdx.x;
     float4 prm = make_float4(0.f, 0.f, 0.f, INFINITY);
     if (t < hc) {
       int32_t idx[3] = {-1, -1, -1};
@@ -402,7 +469,7 @@ __global__ __launch_bounds__(kPlB) void plane_score_kernel(
         const PlHyp h = plane_hyp_for(P, n, c, h0 + t, f, k0, k1, tag, idx);
         prm = make_float4(h.nx, h.ny, h.nz, h.d);
       }
-      if (samples) {
+      if (samples && ck.index() == 0) {
         int32_t* o = samples + 3 * ((size_t)c * n_hyp + h0 + t);
         o[0] = idx[0];
         o[1] = idx[1];
@@ -413,15 +480,15 @@ __global__ __launch_bounds__(kPlB) void plane_score_kernel(
     cnt[t] = 0;
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int hpw = hcap / kPlW;
-  for (int t0 = 0; t0 < n; t0 += kPlTile) {
-    const int tn = min(kPlTile, n - t0);
+  constexpr int hpw = kPlHyps / kPlW;  // hypotheses per wave
+  for (int t0 = 0; t0 < ck.n; t0 += kPlTile) {
+    const int tn = min(kPlTile, ck.n - t0);
     const int tn64 = (tn + 63) & ~63;
     __syncthreads();
     for (int i = threadIdx.x; i < tn64; i += kPlB) {
       float x = NAN, y = 0.f, z = 0.f;
       if (i < tn) {
-        const float* q = P + 3 * (size_t)(t0 + i);
+        const float* q = P + 3 * ((size_t)ck.first + t0 + i);
         x = q[0] - f.m[0];
         y = q[1] - f.m[1];
         z = q[2] - f.m[2];
@@ -431,6 +498,7 @@ __global__ __launch_bounds__(kPlB) void plane_score_kernel(
       sz[i] = z;
     }
     __syncthreads();
+#pragma unroll
     for (int hb = 0; hb < hpw; hb += kPlHB) {
       const int hbase = wave * hpw + hb;
       if (hbase >= hc) break;
@@ -461,30 +529,42 @@ __global__ __launch_bounds__(kPlB) void plane_score_kernel(
     }
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < hc; t += kPlB) counts[(size_t)c * n_hyp + h0 + t] = cnt[t];
+  if ((int)threadIdx.x < hc) {
+    int32_t* o = counts + (size_t)c * n_hyp + h0 + threadIdx.x;
+    const int v = cnt[threadIdx.x];
+    if (ck.count() == 1)
+      *o = v;
+    else if (v)
+      atomicAdd(o, v);
+  }
 }
 
-// model: plane[4] (unit normal, z >= 0 orientation), centroid[3], inliers of
-// the refitted plane
-__global__ __launch_bounds__(kPlB) void plane_refit_kernel(
-    const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
-    const PlFrame* __restrict__ frames, const int32_t* __restrict__ counts, int n_hyp, float thr,
-    uint32_t k0, uint32_t k1, uint32_t tag, uint32_t* __restrict__ mask,
-    int32_t* __restrict__ best_out, double* __restrict__ model) {
-  __shared__ double red[kPlW * 6];
-  __shared__ long long redk[kPlW];
-  __shared__ PlHyp best_h;
-  const int c = blockIdx.x;
-  const int off = offsets[c];
-  const int n = offsets[c + 1] - off;
-  const float* P = xyz + 3 * (size_t)off;
-  const PlFrame f = frames[c];
+// Sum of K doubles per thread over the workgroup, every thread gets it
+// (waves, then the waves in order).
+template <int K>
+__device__ inline void plane_sum(double (&v)[K], double* red) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  double* out = model + 8 * (size_t)c;
+#pragma unroll
+  for (int k = 0; k < K; ++k) v[k] = sl_wave_sum(v[k]);
+  __syncthreads();
+  if (lane == 0)
+#pragma unroll
+    for (int k = 0; k < K; ++k) red[wave * K + k] = v[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    double t = red[k];
+    for (int w = 1; w < kPlW; ++w) t += red[w * K + k];
+    v[k] = t;
+  }
+}
+
+// Best hypothesis of a set (max count, lowest index), by every thread.
+__device__ inline int plane_best(const int32_t* __restrict__ counts, int n_hyp, int n,
+                                 long long* redk) {
   long long key = -1;
   for (int h = threadIdx.x; h < n_hyp; h += kPlB) {
-    const long long kk = ((long long)counts[(size_t)c * n_hyp + h] << 32) |
-                         (long long)(0xFFFFFFFFu - (uint32_t)h);
+    const long long kk = ((long long)counts[h] << 32) | (long long)(0xFFFFFFFFu - (uint32_t)h);
     key = kk > key ? kk : key;
   }
 #pragma unroll
@@ -492,105 +572,53 @@ __global__ __launch_bounds__(kPlB) void plane_refit_kernel(
     const long long other = __shfl_xor(key, o, 64);
     key = other > key ? other : key;
   }
-  if (lane == 0) redk[wave] = key;
+  if ((threadIdx.x & 63) == 0) redk[threadIdx.x >> 6] = key;
   __syncthreads();
   key = redk[0];
   for (int w = 1; w < kPlW; ++w) key = redk[w] > key ? redk[w] : key;
-  const int best = (n >= 3) ? (int)(0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFll)) : -1;
-  if (threadIdx.x == 0) {
-    if (best >= 0) {
-      int32_t idx[3];
-      best_h = plane_hyp_for(P, n, c, best, f, k0, k1, tag, idx);
-    } else {
-      best_h.valid = 0;
-      best_h.nx = best_h.ny = best_h.nz = 0.f;
-      best_h.d = INFINITY;
-    }
-    if (best_out) best_out[c] = best;
-  }
-  __syncthreads();
-  const PlHyp h = best_h;
-  // mask + centroid (FP64, relative to m)
-  double acc[4] = {0, 0, 0, 0};
-  const int gend = off + n;
-  for (int gb = (off & ~63); gb < gend; gb += kPlB) {
-    const int g = gb + (int)threadIdx.x;
-    bool in = false;
-    double d3[3] = {0, 0, 0};
-    if (g >= off && g < gend) {
-      const float* q = xyz + 3 * (size_t)g;
-      const float x = q[0] - f.m[0], y = q[1] - f.m[1], z = q[2] - f.m[2];
-      in = plane_inlier(x, y, z, h, thr);
-      if (in) {
-        d3[0] = (double)q[0] - (double)f.m[0];
-        d3[1] = (double)q[1] - (double)f.m[1];
-        d3[2] = (double)q[2] - (double)f.m[2];
-      }
-    }
-    const uint64_t b = __builtin_amdgcn_ballot_w64(in);
-    if (mask && lane == 0 && b) {
-      const int w0 = (gb + wave * 64) >> 5;
-      if ((uint32_t)b) atomicOr(mask + w0, (uint32_t)b);
-      if ((uint32_t)(b >> 32)) atomicOr(mask + w0 + 1, (uint32_t)(b >> 32));
-    }
-    if (in) {
-      acc[0] += d3[0];
-      acc[1] += d3[1];
-      acc[2] += d3[2];
-      acc[3] += 1.0;
-    }
-  }
-  {
-    double a4[4] = {acc[0], acc[1], acc[2], acc[3]};
+  return n >= 3 ? (int)(0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFll)) : -1;
+}
+
+// kPlAhead points per thread, loaded before any is used (the loads overlap),
+// from i0 on in strides of the workgroup; NaN past n.
+constexpr int kPlAhead = 4;
+__device__ inline void plane_load(const float* __restrict__ P, int i0, int n,
+                                  float (&q)[kPlAhead][3]) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) a4[k] = sl_wave_sum(a4[k]);
-    __syncthreads();
-    if (lane == 0)
-      for (int k = 0; k < 4; ++k) red[wave * 4 + k] = a4[k];
-    __syncthreads();
-    for (int k = 0; k < 4; ++k) {
-      double t = red[k];
-      for (int w = 1; w < kPlW; ++w) t += red[w * 4 + k];
-      acc[k] = t;
-    }
-    __syncthreads();
-  }
-  const double k = acc[3];
-  if (k < 3.0 || !h.valid) {
-    if (threadIdx.x == 0) {
-      for (int i = 0; i < 7; ++i) out[i] = 0.0;
-      out[7] = k;
-    }
-    return;
-  }
-  const double mu[3] = {acc[0] / k, acc[1] / k, acc[2] / k};
-  double S[6] = {0, 0, 0, 0, 0, 0};
-  for (int i = threadIdx.x; i < n; i += kPlB) {
-    const float* q = P + 3 * (size_t)i;
-    if (!plane_inlier(q[0] - f.m[0], q[1] - f.m[1], q[2] - f.m[2], h, thr)) continue;
-    const double x = ((double)q[0] - (double)f.m[0]) - mu[0];
-    const double y = ((double)q[1] - (double)f.m[1]) - mu[1];
-    const double z = ((double)q[2] - (double)f.m[2]) - mu[2];
-    S[0] += x * x;
-    S[1] += x * y;
-    S[2] += x * z;
-    S[3] += y * y;
-    S[4] += y * z;
-    S[5] += z * z;
-  }
-  {
+  for (int j = 0; j < kPlAhead; ++j) {
+    const int i = i0 + j * kPlB + (int)threadIdx.x;
 #pragma unroll
-    for (int kk = 0; kk < 6; ++kk) S[kk] = sl_wave_sum(S[kk]);
-    __syncthreads();
-    if (lane == 0)
-      for (int kk = 0; kk < 6; ++kk) red[wave * 6 + kk] = S[kk];
-    __syncthreads();
-    for (int kk = 0; kk < 6; ++kk) {
-      double t = red[kk];
-      for (int w = 1; w < kPlW; ++w) t += red[w * 6 + kk];
-      S[kk] = t;
+    for (int k = 0; k < 3; ++k) q[j][k] = i >= 0 && i < n ? P[3 * (size_t)i + k] : NAN;
+  }
+}
+
+// Covariance (FP64, about mu) of the inliers of h among a chunk's points.
+__device__ inline void plane_cov(const float* __restrict__ P, int n, const PlFrame& f,
+                                 const PlHyp& h, float thr, const double mu[3], double (&S)[6]) {
+#pragma unroll
+  for (int k = 0; k < 6; ++k) S[k] = 0.0;
+  for (int i0 = 0; i0 < n; i0 += kPlAhead * kPlB) {
+    float q[kPlAhead][3];
+    plane_load(P, i0, n, q);
+#pragma unroll
+    for (int j = 0; j < kPlAhead; ++j) {
+      if (!plane_inlier(q[j][0] - f.m[0], q[j][1] - f.m[1], q[j][2] - f.m[2], h, thr)) continue;
+      const double x = ((double)q[j][0] - (double)f.m[0]) - mu[0];
+      const double y = ((double)q[j][1] - (double)f.m[1]) - mu[1];
+      const double z = ((double)q[j][2] - (double)f.m[2]) - mu[2];
+      S[0] += x * x;
+      S[1] += x * y;
+      S[2] += x * z;
+      S[3] += y * y;
+      S[4] += y * z;
+      S[5] += z * z;
     }
   }
+}
+
+// Unit normal, offset and centroid of the plane of covariance S about mu.
+__device__ inline void plane_solve(const double (&S)[6], const double mu[3], const PlFrame& f,
+                                   double pl[7]) {
   double w3[3], V[3][3], nrm[3];
   sl_eig3(S, w3, V);
   const int kmin = sl_argmin3(w3);
@@ -604,30 +632,216 @@ __global__ __launch_bounds__(kPlB) void plane_refit_kernel(
   }
   if (nrm[2] == 0.0) sl_sign_normalise(nrm);
   const double cxyz[3] = {(double)f.m[0] + mu[0], (double)f.m[1] + mu[1], (double)f.m[2] + mu[2]};
-  const double dd = -(nrm[0] * cxyz[0] + nrm[1] * cxyz[1] + nrm[2] * cxyz[2]);
-  // inliers of the refitted plane (FP64)
-  double cnt[1] = {0.0};
-  for (int i = threadIdx.x; i < n; i += kPlB) {
-    const float* q = P + 3 * (size_t)i;
-    const double t = nrm[0] * (double)q[0] + nrm[1] * (double)q[1] + nrm[2] * (double)q[2] + dd;
-    if (fabs(t) < (double)thr) cnt[0] += 1.0;
+  pl[0] = nrm[0];
+  pl[1] = nrm[1];
+  pl[2] = nrm[2];
+  pl[3] = -(nrm[0] * cxyz[0] + nrm[1] * cxyz[1] + nrm[2] * cxyz[2]);
+  pl[4] = cxyz[0];
+  pl[5] = cxyz[1];
+  pl[6] = cxyz[2];
+}
+
+// The refitted plane of covariance S about mu: unit normal, offset, centroid,
+// by the first wave (the FP64 eigen-solve of four waves at once held the
+// SIMDs longer than its own latency), every thread gets it.
+__device__ inline void plane_from_cov(const double (&S)[6], const double mu[3], const PlFrame& f,
+                                      double* lds, double pl[7]) {
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    plane_solve(S, mu, f, pl);
+    if (threadIdx.x == 0)
+      for (int i = 0; i < 7; ++i) lds[i] = pl[i];
   }
-  cnt[0] = sl_wave_sum(cnt[0]);
   __syncthreads();
-  if (lane == 0) red[wave] = cnt[0];
+  for (int i = 0; i < 7; ++i) pl[i] = lds[i];
+}
+
+// Inliers of the refitted plane (FP64) among a chunk's points, this thread's.
+__device__ inline int plane_recount(const float* __restrict__ P, int n, const double pl[7],
+                                    float thr) {
+  int k = 0;
+  for (int i0 = 0; i0 < n; i0 += kPlAhead * kPlB) {
+    float q[kPlAhead][3];
+    plane_load(P, i0, n, q);
+#pragma unroll
+    for (int j = 0; j < kPlAhead; ++j) {
+      const double t = pl[0] * (double)q[j][0] + pl[1] * (double)q[j][1] +
+                       pl[2] * (double)q[j][2] + pl[3];
+      k += fabs(t) < (double)thr ? 1 : 0;  // false for the NaN past n
+    }
+  }
+  return k;
+}
+
+__device__ inline int plane_sum_int(int v, int* red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
+  int t = red[0];
+  for (int w = 1; w < kPlW; ++w) t += red[w];
+  return t;
+}
+
+// What the refit's kernels hand on for a set of several chunks.
+struct PlState {
+  PlHyp h;  // the best hypothesis
+};
+
+// model: plane[4] (unit normal, z >= 0 orientation), centroid[3], inliers of
+// the refitted plane.
+//
+// Mask, centroid and covariance sums of one refit chunk.  A set of one chunk (up to
+// kPlRefit points) is finished here; of a larger one each chunk's sums go to
+// part, for plane_finish.  90 us by one workgroup
+// for a 27,001-point set, 9 + 11 us by fourteen.
+__global__ __launch_bounds__(kPlB) void plane_refit_kernel(
+    const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
+    const PlFrame* __restrict__ frames, const PlChunk* __restrict__ chunks,
+    const int32_t* __restrict__ counts, int n_hyp, float thr, uint32_t k0, uint32_t k1,
+    uint32_t tag, double* __restrict__ part, PlState* __restrict__ state,
+    uint32_t* __restrict__ mask, int32_t* __restrict__ best_out, double* __restrict__ model) {
+  __shared__ double red[kPlW * 6];
+  __shared__ long long redk[kPlW];
+  __shared__ int redi[kPlW];
+  __shared__ PlHyp best_h;
+  const PlChunk ck = chunks[blockIdx.x];
+  const int c = ck.set;
+  const int off = offsets[c];
+  const int n = offsets[c + 1] - off;
+  const float* P = xyz + 3 * (size_t)off;
+  const PlFrame f = frames[c];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double* out = model + 8 * (size_t)c;
+  const int best = plane_best(counts + (size_t)c * n_hyp, n_hyp, n, redk);
   if (threadIdx.x == 0) {
-    double t = red[0];
-    for (int w = 1; w < kPlW; ++w) t += red[w];
-    out[0] = nrm[0];
-    out[1] = nrm[1];
-    out[2] = nrm[2];
-    out[3] = dd;
-    out[4] = cxyz[0];
-    out[5] = cxyz[1];
-    out[6] = cxyz[2];
-    out[7] = t;
+    if (best >= 0) {
+      int32_t idx[3];
+      best_h = plane_hyp_for(P, n, c, best, f, k0, k1, tag, idx);
+    } else {
+      best_h.valid = 0;
+      best_h.nx = best_h.ny = best_h.nz = 0.f;
+      best_h.d = INFINITY;
+    }
+    if (ck.index() == 0) {
+      if (best_out) best_out[c] = best;
+      state[c].h = best_h;
+    }
   }
+  __syncthreads();
+  const PlHyp h = best_h;
+  // mask + centroid (FP64, relative to m)
+  double acc[4] = {0, 0, 0, 0};
+  const int gs = off + ck.first, gend = gs + ck.n;
+  for (int gb = (gs & ~63); gb < gend; gb += kPlAhead * kPlB) {
+    float q[kPlAhead][3];
+    plane_load(xyz + 3 * (size_t)gs, gb - gs, ck.n, q);
+#pragma unroll
+    for (int j = 0; j < kPlAhead; ++j) {
+      const bool in =
+          plane_inlier(q[j][0] - f.m[0], q[j][1] - f.m[1], q[j][2] - f.m[2], h, thr);
+      const uint64_t b = __builtin_amdgcn_ballot_w64(in);
+      if (mask && lane == 0 && b) {
+        const int w0 = (gb + j * kPlB + wave * 64) >> 5;
+        if ((uint32_t)b) atomicOr(mask + w0, (uint32_t)b);
+        if ((uint32_t)(b >> 32)) atomicOr(mask + w0 + 1, (uint32_t)(b >> 32));
+      }
+      if (in) {
+        acc[0] += (double)q[j][0] - (double)f.m[0];
+        acc[1] += (double)q[j][1] - (double)f.m[1];
+        acc[2] += (double)q[j][2] - (double)f.m[2];
+        acc[3] += 1.0;
+      }
+    }
+  }
+  plane_sum<4>(acc, red);
+  const double k = acc[3];
+  const bool whole = ck.count() == 1;
+  if (whole && (k < 3.0 || !h.valid)) {
+    if (threadIdx.x == 0) {
+      for (int i = 0; i < 7; ++i) out[i] = 0.0;
+      out[7] = k;
+    }
+    return;
+  }
+  const double mu[3] = {acc[0] / k, acc[1] / k, acc[2] / k};
+  double S[6], pl[7];
+  plane_cov(P + 3 * (size_t)ck.first, ck.n, f, h, thr, mu, S);
+  plane_sum<6>(S, red);
+  if (!whole) {
+    double* o = part + 10 * (size_t)blockIdx.x;
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = acc[i];
+#pragma unroll
+      for (int i = 0; i < 6; ++i) o[4 + i] = k > 0.0 ? S[i] : 0.0;
+    }
+    return;
+  }
+  plane_from_cov(S, mu, f, red, pl);
+  const int t = plane_sum_int(plane_recount(P, n, pl, thr), redi);
+  if (threadIdx.x == 0) {
+    for (int i = 0; i < 7; ++i) out[i] = pl[i];
+    out[7] = (double)t;
+  }
+}
+
+// The sets of several chunks: the plane of the chunks' sums (the covariance
+// about the common mean is the sum over the chunks of their own, each about
+// its own mean, plus n_r d_r d_r' with d_r the distance of the means; FP64,
+// in chunk order of a fixed tree), solved by every chunk's workgroup, and
+// each chunk's share of its inliers; the chunk that arrives last writes the
+// record.
+__global__ __launch_bounds__(kPlB) void plane_finish_kernel(
+    const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
+    const PlFrame* __restrict__ frames, const int2* __restrict__ set_chunks,
+    const PlChunk* __restrict__ chunks, float thr, const PlState* __restrict__ state,
+    const double* __restrict__ part, int2* __restrict__ arrived, double* __restrict__ model) {
+  __shared__ double red[kPlW * 6];
+  __shared__ int redi[kPlW];
+  static_assert(kPlMaxChunks <= kPlB, "one thread per chunk");
+  const PlChunk ck = chunks[blockIdx.x];
+  if (ck.count() == 1) return;
+  const int R = ck.count();
+  const double* sp = part + 10 * ((size_t)set_chunks[ck.set].x + threadIdx.x);
+  const bool mine = (int)threadIdx.x < R;
+  double* out = model + 8 * (size_t)ck.set;
+  double own[4], acc[4], S[6], pl[7];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = own[i] = mine ? sp[i] : 0.0;
+#pragma unroll
+  for (int i = 0; i < 6; ++i) S[i] = mine ? sp[4 + i] : 0.0;
+  plane_sum<4>(acc, red);
+  const double k = acc[3];
+  if (k < 3.0 || !state[ck.set].h.valid) {
+    if (ck.index() == 0 && threadIdx.x == 0) {
+      for (int i = 0; i < 7; ++i) out[i] = 0.0;
+      out[7] = k;
+    }
+    return;
+  }
+  const double mu[3] = {acc[0] / k, acc[1] / k, acc[2] / k};
+  if (own[3] > 0.0) {
+    const double x = own[0] / own[3] - mu[0], y = own[1] / own[3] - mu[1],
+                 z = own[2] / own[3] - mu[2];
+    S[0] += own[3] * (x * x);
+    S[1] += own[3] * (x * y);
+    S[2] += own[3] * (x * z);
+    S[3] += own[3] * (y * y);
+    S[4] += own[3] * (y * z);
+    S[5] += own[3] * (z * z);
+  }
+  plane_sum<6>(S, red);
+  plane_from_cov(S, mu, frames[ck.set], red, pl);
+  const int t = plane_sum_int(
+      plane_recount(xyz + 3 * ((size_t)offsets[ck.set] + ck.first), ck.n, pl, thr), redi);
+  if (threadIdx.x != 0) return;
+  atomicAdd(&arrived[ck.set].x, t);
+  __threadfence();
+  if (atomicAdd(&arrived[ck.set].y, 1) != R - 1) return;
+  __threadfence();
+  for (int i = 0; i < 7; ++i) out[i] = pl[i];
+  out[7] = (double)atomicAdd(&arrived[ck.set].x, 0);
 }
 
 }  // namespace
@@ -637,14 +851,19 @@ struct sloam_plane_plan {
   sloam_plane_fit_cfg cfg{};
   int32_t n_sets = 0;
   int64_t n_points = 0;
-  int hcap = 0;
-  int n_work = 0;
-  int4* d_work = nullptr;
+  int n_score = 0, n_refit = 0;  // chunks
+  bool multi = false;            // some set has several refit chunks
+  void* d_mem = nullptr;         // holds the tables and buffers below
+  PlChunk* d_score = nullptr;    // largest sets first
+  PlChunk* d_refit = nullptr;    // in set order
+  int2* d_sets = nullptr;        // per set {first refit chunk, refit chunks}
+  float* d_box = nullptr;        // 6 per refit chunk
+  double* d_part = nullptr;      // 10 per refit chunk: centroid sums, covariance
+  PlState* d_state = nullptr;
+  int2* d_arrived = nullptr;     // per set {inliers, chunks done}
   PlFrame* d_frames = nullptr;
   int32_t* d_counts = nullptr;
 };
-
-static int pl_round_up(int x, int m) { return (x + m - 1) / m * m; }
 
 extern "C" {
 
@@ -761,42 +980,82 @@ int sloam_plane_plan_create(sloam_ctx* ctx, const int32_t* h_offsets, int32_t n_
   p->cfg = *cfg;
   p->n_sets = n_sets;
   p->n_points = h_offsets[n_sets];
-  p->hcap = pl_round_up(std::min(256, pl_round_up(cfg->n_hyp, kPlW * kPlHB)), kPlW * kPlHB);
+  const int n_y = (cfg->n_hyp + kPlHyps - 1) / kPlHyps;
+  // set c's chunks of `chunk` points (one empty chunk for an empty set)
+  auto cut = [&](std::vector<PlChunk>& v, int c, int64_t chunk) {
+    const int len = h_offsets[c + 1] - h_offsets[c];
+    const int R = (int)std::max<int64_t>(1, (len + chunk - 1) / chunk);
+    for (int r = 0; r < R; ++r) {
+      const int64_t b = r * chunk, e = std::min<int64_t>(len, b + chunk);
+      v.push_back(PlChunk{c, (int)b, (int)(e - b), (R << 16) | r});
+    }
+    return R;
+  };
+  std::vector<PlChunk> refit, score;
+  std::vector<int2> sets(n_sets);
+  for (int c = 0; c < n_sets; ++c) {
+    const int64_t len = h_offsets[c + 1] - h_offsets[c];
+    const int64_t even = (len + kPlMaxChunks - 1) / kPlMaxChunks;
+    const int first = (int)refit.size();
+    const int R = cut(refit, c, std::max<int64_t>(kPlRefit, (even + 63) / 64 * 64));
+    sets[c] = make_int2(first, R);
+    p->multi = p->multi || R > 1;
+  }
+  // score chunks of kPlScore points, of more where that would cut the batch
+  // into over kPlScoreMax workgroups (the hypotheses are made once per chunk)
+  // or a set into over 2^15 - 1 chunks
+  int64_t chunk = kPlScore;
+  while ((p->n_points / chunk) * n_y > kPlScoreMax || p->n_points / chunk > 32766) chunk *= 2;
   std::vector<int> order(n_sets);
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
     return (h_offsets[a + 1] - h_offsets[a]) > (h_offsets[b + 1] - h_offsets[b]);
   });
-  std::vector<int4> work;
-  for (int c : order)
-    for (int h0 = 0; h0 < cfg->n_hyp; h0 += p->hcap)
-      work.push_back(make_int4(c, h0, std::min(p->hcap, cfg->n_hyp - h0), 0));
-  p->n_work = (int)work.size();
-  int st = SLOAM_OK;
-  if (p->n_work > 0) {
-    st = sloam_dev_alloc(ctx, (void**)&p->d_work, sizeof(int4) * work.size());
-    if (!st) {
-      hipError_t e = hipMemcpy(p->d_work, work.data(), sizeof(int4) * work.size(),
-                               hipMemcpyHostToDevice);
-      if (e != hipSuccess) st = sloam_record_hip_error(ctx, e, "hipMemcpy(plane work)");
-    }
+  for (int c : order) cut(score, c, chunk);
+  p->n_score = (int)score.size();
+  p->n_refit = (int)refit.size();
+  // one allocation: the three tables (uploaded in one copy), then the rest
+  auto al = [](size_t x) { return (x + 255) / 256 * 256; };
+  const size_t sb = al(sizeof(PlChunk) * score.size()), rb = al(sizeof(PlChunk) * refit.size()),
+               tb = al(sizeof(int2) * sets.size()), bb = al(sizeof(float) * 6 * refit.size()),
+               pb = al(sizeof(double) * 10 * refit.size()), hb = al(sizeof(PlState) * n_sets),
+               ab = al(sizeof(int2) * n_sets), fb = al(sizeof(PlFrame) * n_sets),
+               cb = al(sizeof(int32_t) * (size_t)n_sets * cfg->n_hyp);
+  int st = sloam_dev_alloc(ctx, &p->d_mem, sb + rb + tb + bb + pb + hb + ab + fb + cb);
+  if (!st && n_sets > 0) {
+    std::vector<char> tables(sb + rb + tb);
+    std::memcpy(tables.data(), score.data(), sizeof(PlChunk) * score.size());
+    std::memcpy(tables.data() + sb, refit.data(), sizeof(PlChunk) * refit.size());
+    std::memcpy(tables.data() + sb + rb, sets.data(), sizeof(int2) * sets.size());
+    const hipError_t e = hipMemcpy(p->d_mem, tables.data(), tables.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) st = sloam_record_hip_error(ctx, e, "hipMemcpy(plane chunks)");
   }
-  if (!st && n_sets > 0) st = sloam_dev_alloc(ctx, (void**)&p->d_frames, sizeof(PlFrame) * n_sets);
-  if (!st && n_sets > 0)
-    st = sloam_dev_alloc(ctx, (void**)&p->d_counts, sizeof(int32_t) * (size_t)n_sets * cfg->n_hyp);
   if (st) {
     sloam_plane_plan_destroy(p);
     return st;
   }
+  char* q = static_cast<char*>(p->d_mem);
+  auto take = [&](size_t bytes) {
+    char* r = q;
+    q += bytes;
+    return (void*)r;
+  };
+  p->d_score = (PlChunk*)take(sb);
+  p->d_refit = (PlChunk*)take(rb);
+  p->d_sets = (int2*)take(tb);
+  p->d_box = (float*)take(bb);
+  p->d_part = (double*)take(pb);
+  p->d_state = (PlState*)take(hb);
+  p->d_arrived = (int2*)take(ab);
+  p->d_frames = (PlFrame*)take(fb);
+  p->d_counts = (int32_t*)take(cb);
   *out = p;
   return SLOAM_OK;
 }
 
 void sloam_plane_plan_destroy(sloam_plane_plan* p) {
   if (!p) return;
-  sloam_dev_free(p->d_work);
-  sloam_dev_free(p->d_frames);
-  sloam_dev_free(p->d_counts);
+  sloam_dev_free(p->d_mem);
   delete p;
 }
 
@@ -810,29 +1069,32 @@ int sloam_plane_plan_exec(sloam_plane_plan* p, const float* d_xyz, const int32_t
   const uint32_t k0 = (uint32_t)p->cfg.seed, k1 = (uint32_t)(p->cfg.seed >> 32);
   const uint32_t tag = (uint32_t)p->cfg.stream_tag;
   int32_t* counts = d_counts ? d_counts : p->d_counts;
-  if (d_mask) {
-    int st = sloam_fill_u32(ctx, d_mask, (size_t)((p->n_points + 31) / 32), 0u);
-    if (st) return st;
-  }
+  const int H = p->cfg.n_hyp;
+  const float thr = p->cfg.thr;
+  const dim3 block(kPlB), chunks(p->n_refit);
   {
     SloamKernelScope ks(ctx, "plane_seed");
-    hipLaunchKernelGGL(plane_seed_kernel, dim3(p->n_sets), dim3(kPlB), 0, ctx->stream, d_xyz,
-                       d_offsets, p->n_sets, p->d_frames);
+    hipLaunchKernelGGL(plane_box_kernel, chunks, block, 0, ctx->stream, d_xyz, d_offsets,
+                       p->d_refit, H, p->d_box, counts, p->d_arrived, d_mask,
+                       (long long)((p->n_points + 31) / 32));
   }
   SLOAM_HIP(ctx, hipGetLastError());
-  if (p->n_work > 0) {
-    const size_t lds = (size_t)p->hcap * (sizeof(float4) + sizeof(int)) + 3 * sizeof(float) * kPlTile;
+  {
     SloamKernelScope ks(ctx, "plane_score");
-    hipLaunchKernelGGL(plane_score_kernel, dim3(p->n_work), dim3(kPlB), lds, ctx->stream, d_xyz,
-                       d_offsets, p->d_frames, p->d_work, p->cfg.n_hyp, p->hcap, p->cfg.thr, k0,
-                       k1, tag, counts, d_samples);
+    hipLaunchKernelGGL(plane_score_kernel, dim3(p->n_score, (H + kPlHyps - 1) / kPlHyps), block, 0,
+                       ctx->stream, d_xyz, d_offsets, p->d_box, p->d_sets, p->d_score, H, thr, k0,
+                       k1, tag, p->d_frames, counts, d_samples);
   }
   SLOAM_HIP(ctx, hipGetLastError());
   {
     SloamKernelScope ks(ctx, "plane_refit");
-    hipLaunchKernelGGL(plane_refit_kernel, dim3(p->n_sets), dim3(kPlB), 0, ctx->stream, d_xyz,
-                       d_offsets, p->d_frames, counts, p->cfg.n_hyp, p->cfg.thr, k0, k1, tag,
-                       d_mask, d_best, d_model);
+    hipLaunchKernelGGL(plane_refit_kernel, chunks, block, 0, ctx->stream, d_xyz, d_offsets,
+                       p->d_frames, p->d_refit, counts, H, thr, k0, k1, tag, p->d_part,
+                       p->d_state, d_mask, d_best, d_model);
+    if (p->multi)
+      hipLaunchKernelGGL(plane_finish_kernel, chunks, block, 0, ctx->stream, d_xyz, d_offsets,
+                         p->d_frames, p->d_sets, p->d_refit, thr, p->d_state, p->d_part,
+                         p->d_arrived, d_model);
   }
   SLOAM_HIP(ctx, hipGetLastError());
   return SLOAM_OK;

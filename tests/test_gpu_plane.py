@@ -80,6 +80,36 @@ def test_plane_ransac_bit_exact(ctx):
     assert np.all(np.abs(g["model"][:, 7] - o["model"][:, 7]) <= 1)
 
 
+@pytest.mark.parametrize("n_hyp", [1, 65, 333])
+@pytest.mark.parametrize("sizes", [(2048, 1024, 1025, 0, 3, 2, 63), (2049, 12289, 1, 5000),
+                                   (27001,)], ids=["one-refit-chunk", "several", "one-set"])
+def test_plane_ransac_chunks(ctx, sizes, n_hyp):
+    """Sets cut into score chunks (1,024 points x 64 hypotheses) and refit
+    chunks (2,048 points): sizes at and next to both, alone and beside smaller
+    sets.  Counts, masks and samples are integers (exact); the models' FP64
+    sums differ in order only (relative 2^-53 per addition: 1e-9 holds far
+    beyond 30,000 points)."""
+    rng = np.random.default_rng(n_hyp)
+    sets = []
+    for m in sizes:
+        xy = rng.uniform(-15, 15, (m, 2))
+        z = 0.05 * xy[:, 0] - 0.02 * xy[:, 1] - 1.5 + rng.normal(0, 0.02, m)
+        P = np.c_[xy, z]
+        P[:m // 4, 2] += rng.uniform(-2, 2, m // 4)
+        sets.append(P)
+    xyz = np.concatenate(sets).astype(np.float32)
+    off = np.cumsum([0] + list(sizes)).astype(np.int32)
+    print(f"[plane] chunks {sizes} x {n_hyp}", flush=True)
+    for rep in range(2):
+        g = fit_planes(ctx, xyz, off, n_hyp=n_hyp, thr=0.05, counts=True, samples=True, mask=True,
+                       best=True)
+        o = oracle.plane_fit_batch(xyz, off, n_hyp, thr=0.05, samples=True, threads=8)
+        for k in ("samples", "counts", "best", "mask"):
+            assert np.array_equal(g[k], o[k]), k
+        assert np.allclose(g["model"][:, :7], o["model"][:, :7], atol=1e-9, rtol=0)
+        assert np.all(np.abs(g["model"][:, 7] - o["model"][:, 7]) <= 1)
+
+
 @pytest.mark.parametrize("n,bins", [(3000, (1, 1)), (30000, (1, 4)), (40000, (1, 1))],
                          ids=["3000-one-cell", "30000-four-cells", "40000-one-cell"])
 def test_ground_planes_bottom_k_order(ctx, n, bins):
