@@ -136,3 +136,43 @@ def test_ground_planes_bottom_k_order(ctx, n, bins):
     assert np.array_equal(g["model"][valid, 4:7], o["model"][valid, 4:7])
     assert np.allclose(g["model"][valid, :4], o["model"][valid, :4], atol=1e-9, rtol=0)
     assert np.array_equal(g["features"][valid, :60], o["features"][valid, :60])
+
+
+@pytest.mark.parametrize("retain", [0.05, 0.4, 1.0])
+@pytest.mark.parametrize("n", [1, 1023, 1025, 9000, 30000])
+@pytest.mark.parametrize("ties", ["none", "some", "most"])
+def test_ground_planes_selection_rounds(ctx, n, retain, ties):
+    """The per-cell selection (few cells) where one cell holds most of the
+    points: cells larger than the keys held in LDS (4,096), more kept points
+    than one round sorts (2,048), more ties of one z than that, and scans of a
+    few points.  At retain 1.0 the larger clouds take the radix sorts.  The
+    float centroid is a sequential sum, so it is equal only if every kept
+    point comes in the oracle's order."""
+    rng = np.random.default_rng(n)
+    r = rng.uniform(6.0, 24.0, n)
+    th = np.where(rng.uniform(0, 1, n) < 0.85, rng.uniform(0.05, 0.3, n),
+                  rng.uniform(-np.pi, np.pi, n))
+    pts = np.zeros((n, 4), np.float32)
+    pts[:, 0], pts[:, 1] = r * np.cos(th), r * np.sin(th)
+    z = rng.normal(-1.5, 0.3, n)
+    if ties != "none":
+        z = np.round(z, 2)
+    if ties == "most":
+        z[rng.uniform(0, 1, n) < 0.6] = -1.5
+    pts[:, 2] = z
+    prm = dict(radii_bins=2, theta_bins=18, min_dist=5.0, max_dist=25.0, retain_thresh=retain,
+               num_features=5)
+    g = ground_planes(ctx, pts, **prm)
+    o = oracle.ground_planes(pts, **prm)
+    assert np.array_equal(g["info"], o["info"])
+    valid = o["info"][:, 0] == 1
+    assert np.array_equal(g["model"][valid, 4:7], o["model"][valid, 4:7])
+    # planes of three or more points (the normal of fewer is not determined)
+    assert np.allclose(g["model"][valid, :4], o["model"][valid, :4], atol=1e-9, rtol=0)
+    assert np.array_equal(g["features"][valid], o["features"][valid])
+    assert np.array_equal(g["kept_offsets"], np.r_[0, np.cumsum(o["info"][:, 2])])
+    idx = g["kept_index"]
+    for c in np.flatnonzero(valid):
+        b, k = g["kept_offsets"][c], o["info"][c, 1]
+        assert len(np.unique(idx[b:b + k])) == k and np.all(idx[b:b + k] >= 0)
+        assert np.all(idx[b + k:g["kept_offsets"][c + 1]] == -1)
