@@ -123,6 +123,14 @@ int sloam_radix_sort(sloam_ctx* ctx, unsigned long long* keys, int32_t* vals,
                      unsigned long long** keys_out = nullptr, int32_t** vals_out = nullptr);
 size_t sloam_radix_hist_ints(int n);
 
+// sloam_trellis that also writes the vertex medians as float (x, y, z per
+// vertex; d_medians nullable), the points the line fits take.
+int sloam_trellis_medians(sloam_ctx* ctx, const float* d_cloud, int32_t height, int32_t width,
+                          const sloam_trellis_cfg* cfg, int32_t* d_labels, int32_t cap_trees,
+                          int32_t cap_vertices, int32_t cap_points, int32_t* d_tree_offsets,
+                          int32_t* d_vertex_int, double* d_vertex_f64, int32_t* d_point_offsets,
+                          float* d_points, int32_t* d_counts, float* d_medians);
+
 // sloam_fit_lines over n_sets sets of which the first *d_n_sets (device,
 // nullable: all) are fitted; the others are left untouched.
 int sloam_fit_lines_dev(sloam_ctx* ctx, const float* d_xyz, const int32_t* d_offsets,

@@ -66,34 +66,18 @@ __global__ __launch_bounds__(256) void fe_pack_kernel(PackArgs a) {
     for (size_t i = t0; i < len[r]; i += stride) a.dst[r][i] = a.src[r][i];
 }
 
-// Vertex medians (vertex_f64 x, y, z) as float, the points the line fit of a
-// tree takes.
-__global__ __launch_bounds__(256) void fe_medians_kernel(const double* __restrict__ vf,
-                                                         const int32_t* __restrict__ counts,
-                                                         int cap_vertices,
-                                                         float* __restrict__ med) {
-  const int nv = min(max(counts[1], 0), cap_vertices);
-  for (int v = blockIdx.x * 256 + threadIdx.x; v < nv; v += gridDim.x * 256) {
-    med[3 * (size_t)v] = (float)vf[4 * (size_t)v + 1];
-    med[3 * (size_t)v + 1] = (float)vf[4 * (size_t)v + 2];
-    med[3 * (size_t)v + 2] = (float)vf[4 * (size_t)v + 3];
-  }
-}
-
 int enqueue(sloam_frontend* f) {
   sloam_ctx* ctx = f->ctx;
   const sloam_frontend_out& o = f->out;
   int st = sloam_project_partition(ctx, o.xyzi, o.label, f->N, &f->cfg.proj, nullptr, nullptr,
                                    nullptr, o.mask, o.ground, o.n_ground, o.tree);
   if (st) return st;
-  st = sloam_trellis(ctx, o.tree, f->cfg.proj.height, f->cfg.proj.width, &f->cfg.trellis,
-                     nullptr, o.cap_trees, o.cap_vertices, o.cap_points, o.tree_offsets,
-                     o.vertex_int, o.vertex_f64, o.point_offsets, o.points, o.trellis_counts);
+  st = sloam_trellis_medians(ctx, o.tree, f->cfg.proj.height, f->cfg.proj.width,
+                             &f->cfg.trellis, nullptr, o.cap_trees, o.cap_vertices, o.cap_points,
+                             o.tree_offsets, o.vertex_int, o.vertex_f64, o.point_offsets, o.points,
+                             o.trellis_counts, f->medians);
   if (st) return st;
   if (f->cfg.fit_lines) {
-    hipLaunchKernelGGL(fe_medians_kernel, dim3(64), dim3(256), 0, ctx->stream, o.vertex_f64,
-                       o.trellis_counts, o.cap_vertices, f->medians);
-    SLOAM_HIP(ctx, hipGetLastError());
     // one set per tree (up to the device-side tree count)
     st = sloam_fit_lines_dev(ctx, f->medians, o.tree_offsets, o.cap_trees, o.trellis_counts,
                              &f->cfg.line, o.line_coeff, o.line_stats, nullptr);

@@ -12,15 +12,16 @@
 //                 nearest point wins, the lowest index on equal ranges (for
 //                 non-negative floats the IEEE bit pattern is monotonic)
 //   proj_pixels   one thread per pixel: range image, winner, mask
-//                 ((int)range == 0 -> invalid -> 0; tree 255, ground 1)
-//   part_count    ground flags per block of kPartItems points
-//   part_scan     exclusive scan of the block counts (one workgroup)
+//                 ((int)range == 0 -> invalid -> 0; tree 255, ground 1); and
+//                 the ground points per block of kPartItems points
+//   part_scan     (over a million points) exclusive scan of the block counts
 //   part_scatter  order-preserving ground compaction + dense tree cloud
 //                 (NaN where the pixel is not tree; optional destagger)
 // Points with a non-finite coordinate take no part (the reference sorts their
 // NaN ranges, which is undefined behaviour).
 #include "common.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -28,6 +29,9 @@ namespace {
 
 constexpr int kPB = 256;
 constexpr int kPartItems = 1024;  // points per partition block (4 per thread)
+// blocks up to which every scatter block sums the counts before its own (four
+// loads a thread) instead of waiting for a scan launch
+constexpr int kPartSum = 1024;
 
 struct ProjCfgDev {
   int H, W;
@@ -77,44 +81,40 @@ __global__ __launch_bounds__(kPB) void proj_zbuf_kernel(const float4* __restrict
   atomicMin(keys + (size_t)row * cfg.W + col, key);
 }
 
+// class of a pixel from its z-buffer key: the label of its nearest point,
+// 0 where the range is below one metre
+__device__ inline uint8_t pixel_mask(unsigned long long k, const uint8_t* __restrict__ label) {
+  if (k == ~0ull) return 0;
+  if ((int)__uint_as_float((uint32_t)(k >> 32)) == 0) return 0;
+  const uint8_t c = label[(uint32_t)k];
+  return c == 2 ? 255 : (c == 1 ? 1 : 0);
+}
+
+// Workgroup b: the images' pixels, and the ground points among the partition
+// block b's points (their class from the z-buffer keys, so that the count does
+// not wait for the mask of every pixel).
 __global__ __launch_bounds__(kPB) void proj_pixels_kernel(
     const unsigned long long* __restrict__ keys, const uint8_t* __restrict__ label, int n_pix,
-    float* __restrict__ range_img, int32_t* __restrict__ winner, uint8_t* __restrict__ mask) {
-  const int p = blockIdx.x * kPB + threadIdx.x;
-  if (p >= n_pix) return;
-  const unsigned long long k = keys[p];
-  float r = 0.f;
-  int w = -1;
-  if (k != ~0ull) {
-    r = __uint_as_float((uint32_t)(k >> 32));
-    w = (int)(uint32_t)k;
-  }
-  uint8_t m = 0;
-  if (w >= 0 && (int)r != 0) {
-    const uint8_t c = label[w];
-    m = c == 2 ? 255 : (c == 1 ? 1 : 0);
-  }
-  if (range_img) range_img[p] = r;
-  if (winner) winner[p] = w;
-  mask[p] = m;
-}
-
-__device__ inline uint8_t point_mask(const int2* __restrict__ proj, const uint8_t* __restrict__ mask,
-                                     int W, int i) {
-  const int2 q = proj[i];
-  if (q.x < 0) return 0;
-  return mask[(size_t)q.y * W + q.x];
-}
-
-__global__ __launch_bounds__(kPB) void part_count_kernel(const int2* __restrict__ proj,
-                                                         const uint8_t* __restrict__ mask, int n,
-                                                         int W, int32_t* __restrict__ block_counts) {
+    float* __restrict__ range_img, int32_t* __restrict__ winner, uint8_t* __restrict__ mask,
+    const int2* __restrict__ proj, int n, int W, int32_t* __restrict__ block_counts) {
   __shared__ int wsum[kPB / 64];
-  const int base = blockIdx.x * kPartItems;
+#pragma unroll
+  for (int j = 0; j < kPartItems / kPB; ++j) {
+    const int p = blockIdx.x * kPartItems + j * kPB + (int)threadIdx.x;
+    if (p >= n_pix) continue;
+    const unsigned long long k = keys[p];
+    if (range_img) range_img[p] = k != ~0ull ? __uint_as_float((uint32_t)(k >> 32)) : 0.f;
+    if (winner) winner[p] = k != ~0ull ? (int)(uint32_t)k : -1;
+    mask[p] = pixel_mask(k, label);
+  }
+  if ((int)blockIdx.x * kPartItems >= n) return;  // more pixels than points
   int c = 0;
-  for (int j = threadIdx.x; j < kPartItems; j += kPB) {
-    const int i = base + j;
-    if (i < n && point_mask(proj, mask, W, i) == 1) ++c;
+#pragma unroll
+  for (int j = 0; j < kPartItems / kPB; ++j) {
+    const int i = blockIdx.x * kPartItems + j * kPB + (int)threadIdx.x;
+    if (i >= n) continue;
+    const int2 q = proj[i];
+    if (q.x >= 0 && pixel_mask(keys[(size_t)q.y * W + q.x], label) == 1) ++c;
   }
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
   if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = c;
@@ -124,6 +124,13 @@ __global__ __launch_bounds__(kPB) void part_count_kernel(const int2* __restrict_
     for (int w = 0; w < kPB / 64; ++w) t += wsum[w];
     block_counts[blockIdx.x] = t;
   }
+}
+
+__device__ inline uint8_t point_mask(const int2* __restrict__ proj, const uint8_t* __restrict__ mask,
+                                     int W, int i) {
+  const int2 q = proj[i];
+  if (q.x < 0) return 0;
+  return mask[(size_t)q.y * W + q.x];
 }
 
 // exclusive scan of up to any number of block counts by one workgroup
@@ -159,13 +166,29 @@ __global__ __launch_bounds__(kPB) void part_scan_kernel(int32_t* __restrict__ bl
 __global__ __launch_bounds__(kPB) void part_scatter_kernel(
     const float4* __restrict__ xyzi, const int2* __restrict__ proj,
     const uint8_t* __restrict__ mask, int n, int W, int destagger,
-    const int32_t* __restrict__ block_offsets, float4* __restrict__ ground,
-    float4* __restrict__ tree) {
+    const int32_t* __restrict__ block_offsets, int32_t* __restrict__ total,
+    float4* __restrict__ ground, float4* __restrict__ tree) {
   __shared__ int wcount[kPB / 64];
   __shared__ int run;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int base = blockIdx.x * kPartItems;
-  if (threadIdx.x == 0) run = block_offsets[blockIdx.x];
+  if (total) {
+    // block_offsets holds the blocks' counts: this block's offset is the sum
+    // of those before it
+    int v = 0;
+    for (int b = threadIdx.x; b < (int)blockIdx.x; b += kPB) v += block_offsets[b];
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (lane == 0) wcount[wave] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int t = 0;
+      for (int w = 0; w < kPB / 64; ++w) t += wcount[w];
+      run = t;
+      if (blockIdx.x == gridDim.x - 1) *total = t + block_offsets[blockIdx.x];
+    }
+  } else if (threadIdx.x == 0) {
+    run = block_offsets[blockIdx.x];
+  }
   __syncthreads();
   for (int j0 = 0; j0 < kPartItems; j0 += kPB) {
     const int i = base + j0 + (int)threadIdx.x;
@@ -290,21 +313,24 @@ int proj_run(sloam_ctx* ctx, const float* d_xyzi, const uint8_t* d_label, int64_
   SLOAM_HIP(ctx, hipGetLastError());
   {
     SloamKernelScope ks(tctx, "proj_pixels");
-    hipLaunchKernelGGL(proj_pixels_kernel, dim3((n_pix + kPB - 1) / kPB), dim3(kPB), 0,
-                       ctx->stream, keys, d_label, n_pix, d_range, d_winner, d_mask);
+    hipLaunchKernelGGL(proj_pixels_kernel,
+                       dim3((std::max(n_pix, N) + kPartItems - 1) / kPartItems), dim3(kPB), 0,
+                       ctx->stream, keys, d_label, n_pix, d_range, d_winner, d_mask, proj, N, W,
+                       counts);
   }
   SLOAM_HIP(ctx, hipGetLastError());
   {
     SloamKernelScope ks(tctx, "partition");
     if (N > 0) {
-      hipLaunchKernelGGL(part_count_kernel, dim3(n_blocks), dim3(kPB), 0, ctx->stream, proj,
-                         d_mask, N, W, counts);
-      hipLaunchKernelGGL(part_scan_kernel, dim3(1), dim3(kPB), 0, ctx->stream, counts, n_blocks,
-                         d_n_ground);
+      // up to kPartSum blocks each scatter block adds the counts before its own
+      const bool scan = n_blocks > kPartSum;
+      if (scan)
+        hipLaunchKernelGGL(part_scan_kernel, dim3(1), dim3(kPB), 0, ctx->stream, counts, n_blocks,
+                           d_n_ground);
       hipLaunchKernelGGL(part_scatter_kernel, dim3(n_blocks), dim3(kPB), 0, ctx->stream,
                          reinterpret_cast<const float4*>(d_xyzi), proj, d_mask, N, W,
-                         cfg->destagger, counts, reinterpret_cast<float4*>(d_ground),
-                         reinterpret_cast<float4*>(d_tree));
+                         cfg->destagger, counts, scan ? nullptr : d_n_ground,
+                         reinterpret_cast<float4*>(d_ground), reinterpret_cast<float4*>(d_tree));
     } else {
       int st2 = sloam_fill_u32(ctx, (uint32_t*)d_n_ground, 1, 0u);
       if (st2) return st2;

@@ -2,7 +2,7 @@
 // tree cloud and per-beam tree vertices (sloam/src/segmentation/trellis.cpp:
 // 15-132, Instance::findClusters / findTrees / computeVertexProperties).
 //
-//   tr_tile             connected components inside tiles of 64 x 16 pixels: a
+//   tr_tile             connected components inside tiles of 64 x 32 pixels: a
 //                       pixel (finite x) joins its left and upper neighbours
 //                       when their float distance is < the cluster threshold;
 //                       the runs of a row come from one ballot, the rows are
@@ -14,13 +14,13 @@
 //                       pixel in row-major order
 //   tr_flatten          every pixel's root; the tile components add size and
 //                       box to their root's; roots per block
-//   tr_number           roots ranked in pixel order give the component
-//                       numbers; the last workgroup lists the components with
-//                       more than 80 points and their rows.  A component is
-//                       4-connected, so each row of its box is one beam of
-//                       the tree: no sort is needed to find them
+//   tr_number           roots ranked in pixel order give the component numbers
+//   tr_layout           one workgroup: the components with more than 80
+//                       points and their rows.  A component is 4-connected,
+//                       so each row of its box is one beam of the tree: no
+//                       sort is needed to find them
 //   tr_label            (labels asked for) the component number per pixel
-//   tr_vertex           one workgroup per beam: its points in column order,
+//   tr_vertex           a wave per beam: its points in column order,
 //                       medians of x, y, z, the points within 0.2 m of the
 //                       median in (z, y, x, column) order, radius of the
 //                       first / last
@@ -28,7 +28,7 @@
 //                       56), tree / vertex / point offsets
 //   tr_copy             the vertex records and their kept points to the output
 //
-// Seven launches and about 100 us at 128 x 2048 with 36,000 tree pixels; a
+// Eight launches and about 77 us at 128 x 2048 with 36,000 tree pixels; a
 // union-find over single pixels, ranks by three block scans and a radix sort of
 // all pixels by component took nineteen and 220 us.
 #include "common.hpp"
@@ -38,8 +38,9 @@
 namespace {
 
 constexpr int kTB = 256;        // pixel kernels
+constexpr int kTileB = 512;     // tile kernel
 constexpr int kTileW = 64;      // a wave holds a row of a tile
-constexpr int kTileH = 16;
+constexpr int kTileH = 32;
 constexpr int kItems = 1024;    // pixels per block of the root numbering
 constexpr int kAsm = 1024;      // assemble workgroup
 constexpr int kSegLds = 1024;   // beam points staged in LDS (larger beams read HBM)
@@ -53,14 +54,15 @@ struct TrCfgDev {
   int cap_trees, cap_vertices, cap_points;
 };
 
-// scratch counters: components, beams of the kept components, kept
-// components, points handed out to beams, workgroups done
-enum { kCntComps = 0, kCntSegs, kCntKept, kCntAlloc, kCntDone, kCntN = 8 };
+// scratch counters: components, beams of the kept components, kept components
+enum { kCntComps = 0, kCntSegs, kCntKept, kCntN = 8 };
 
-// A kept component: its first pixel, number, last row, rows; first beam, columns.
+// A kept component: its first pixel, number, last row, rows; first beam,
+// columns; points before it and its beams so far (one counter per component:
+// one for all beams serialised them)
 struct TrComp {
   int root, id, row1, rows;
-  int seg0, col0, col1, pad;
+  int seg0, col0, col1, alloc;
 };
 
 __device__ inline int ld_relaxed(const int* p) {
@@ -148,10 +150,10 @@ __device__ inline int run_start(uint64_t left, int lane) {
   return 63 - __builtin_clzll(~left & (~0ull >> (63 - lane)));
 }
 
-__global__ __launch_bounds__(kTB) void tr_tile_kernel(const float4* __restrict__ cloud,
+__global__ __launch_bounds__(kTileB) void tr_tile_kernel(const float4* __restrict__ cloud,
                                                       TrCfgDev cfg, int* __restrict__ L, TrBox box,
                                                       int* __restrict__ counters) {
-  constexpr int kRows = kTileH / (kTB / 64);  // rows per wave
+  constexpr int kRows = kTileH / (kTileB / 64);  // rows per wave
   __shared__ int lab[kTileW * kTileH], size[kTileW * kTileH], row1[kTileW * kTileH],
       col0[kTileW * kTileH], col1[kTileW * kTileH];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -301,6 +303,35 @@ __device__ inline int block_excl(int v, int* wtot, int* total) {
   return off + s - v;
 }
 
+// The same for up to three counts below 2^21 each, packed.
+__device__ inline uint64_t pack3(int a, int b, int c) {
+  return (uint64_t)a | ((uint64_t)b << 21) | ((uint64_t)c << 42);
+}
+__device__ inline int unpack3(uint64_t v, int i) { return (int)((v >> (21 * i)) & 0x1fffff); }
+
+template <int NT>
+__device__ inline uint64_t block_excl3(uint64_t v, unsigned long long* wtot, uint64_t* total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint64_t s = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint64_t t = __shfl_up((unsigned long long)s, o, 64);
+    if (lane >= o) s += t;
+  }
+  if (lane == 63) wtot[wave] = s;
+  __syncthreads();
+  uint64_t off = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) {
+    const uint64_t t = wtot[w];
+    off += w < wave ? t : 0;
+    all += t;
+  }
+  __syncthreads();
+  *total = all;
+  return off + s - v;
+}
+
 // Roots of kItems pixels per block, and their number.
 __global__ __launch_bounds__(kTB) void tr_flatten_kernel(int N, const int* __restrict__ L,
                                                          int* __restrict__ root, TrBox box,
@@ -337,82 +368,106 @@ __global__ __launch_bounds__(kTB) void tr_flatten_kernel(int N, const int* __res
 }
 
 // Numbers the roots in pixel order (id, only at the roots); each block lists
-// its kept components' roots, kept[block * kItems ..], and their number and
-// rows; the last block to finish lays out the components and beams in order.
+// its kept components' roots, kept[block * kItems ..], and their number.
 __global__ __launch_bounds__(kTB) void tr_number_kernel(
     const int* __restrict__ root, TrBox box, TrCfgDev cfg, const int* __restrict__ block_roots,
-    int* __restrict__ id, int* __restrict__ kept, int2* __restrict__ block_kept,
-    TrComp* __restrict__ comps, int* __restrict__ seg_comp, int* __restrict__ counters) {
+    int* __restrict__ id, int* __restrict__ kept, int* __restrict__ block_kept,
+    int* __restrict__ counters) {
+  constexpr int kPer = kItems / kTB;  // consecutive pixels per thread
   __shared__ int wtot[kTB / 64];
-  __shared__ int s_rows, s_last;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int base = blockIdx.x * kItems;
-  if (threadIdx.x == 0) s_rows = 0;
   // roots before this block
   int mine = 0;
   for (int b = threadIdx.x; b < (int)blockIdx.x; b += kTB) mine += block_roots[b];
-  int run;
+  int run, nk = 0;
   block_excl<kTB>(mine, wtot, &run);
-  int nk = 0;
-  for (int j0 = 0; j0 < kItems; j0 += kTB) {
-    const int p = base + j0 + (int)threadIdx.x;
-    const bool is_root = p < cfg.N && root[p] == p;
-    int all, all_k;
-    const int e = block_excl<kTB>(is_root ? 1 : 0, wtot, &all);
-    if (is_root) id[p] = run + e;
-    const bool keep = is_root && box.size[p] > cfg.min_label_points;
-    const int k = block_excl<kTB>(keep ? 1 : 0, wtot, &all_k);
-    if (keep) {
-      kept[base + nk + k] = p;
-      atomicAdd(&s_rows, box.row1[p] - p / cfg.W + 1);
+  if (block_roots[blockIdx.x] > 0) {
+    const int p0 = base + kPer * (int)threadIdx.x;
+    int n = 0;  // roots + 65536 x kept ones
+    int size[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      size[j] = p0 + j < cfg.N && root[p0 + j] == p0 + j ? box.size[p0 + j] : -1;
+      n += size[j] < 0 ? 0 : (size[j] > cfg.min_label_points ? 65537 : 1);
     }
-    run += all;
-    nk += all_k;
+    int all;
+    const int e = block_excl<kTB>(n, wtot, &all);
+    int i = run + (e & 65535), k = e >> 16;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (size[j] < 0) continue;
+      const int p = p0 + j;
+      id[p] = i++;
+      if (size[j] > cfg.min_label_points) kept[base + k++] = p;
+    }
+    run += all & 65535;
+    nk = all >> 16;
   }
-  __syncthreads();
   if (threadIdx.x == 0) {
-    block_kept[blockIdx.x] = make_int2(nk, s_rows);
+    block_kept[blockIdx.x] = nk;
     if (blockIdx.x == gridDim.x - 1) counters[kCntComps] = run;
-    __threadfence();
-    s_last = atomicAdd(counters + kCntDone, 1) == (int)gridDim.x - 1 ? 1 : 0;
-    __threadfence();
   }
+}
+
+// The kept components and their beams in order, one workgroup, a thread per
+// component (found by bisection of the blocks' prefix in LDS).  As the last
+// workgroup of tr_number, behind a fence in each of its workgroups, this took
+// longer than a launch of its own.
+__global__ __launch_bounds__(kAsm) void tr_layout_kernel(
+    TrBox box, TrCfgDev cfg, int n_blocks, const int* __restrict__ id,
+    const int* __restrict__ kept, const int* __restrict__ block_kept, TrComp* __restrict__ comps,
+    int* __restrict__ seg_comp, int* __restrict__ counters) {
+  __shared__ int wtot[kAsm / 64];
+  __shared__ unsigned long long wtot3[kAsm / 64];
+  __shared__ int first[kAsm + 1];  // kept components before each block
+  const int t = threadIdx.x;
+  int K;
+  const int e = block_excl<kAsm>(t < n_blocks ? block_kept[t] : 0, wtot, &K);
+  first[t] = e;
+  if (t == 0) first[kAsm] = K;
   __syncthreads();
-  if (!s_last) return;
-  int K = 0, S = 0;
-  for (int b0 = 0; b0 < (int)gridDim.x; b0 += kTB) {
-    const int b = b0 + (int)threadIdx.x;
-    const int2 v = b < (int)gridDim.x ? block_kept[b] : make_int2(0, 0);
-    int ak, as;
-    int k = K + block_excl<kTB>(v.x, wtot, &ak);
-    int s = S + block_excl<kTB>(v.y, wtot, &as);
-    for (int j = 0; j < v.x; ++j, ++k) {
-      const int p = kept[b * kItems + j];
-      TrComp o;
+  int S = 0, P = 0;
+  for (int k0 = 0; k0 < K; k0 += kAsm) {
+    const int k = k0 + t;
+    TrComp o;
+    int size = 0;
+    o.rows = 0;
+    if (k < K) {
+      int lo = 0, hi = kAsm;  // first[lo] <= k < first[hi]
+#pragma unroll
+      for (int it = 0; it < 10; ++it) {
+        const int mid = (lo + hi) >> 1;
+        if (first[mid] <= k)
+          lo = mid;
+        else
+          hi = mid;
+      }
+      const int p = kept[lo * kItems + (k - first[lo])];
       o.root = p;
       o.id = id[p];
       o.row1 = box.row1[p];
       o.rows = o.row1 - p / cfg.W + 1;
-      o.seg0 = s;
       o.col0 = box.col0[p];
       o.col1 = box.col1[p];
-      o.pad = 0;
-      comps[k] = o;
-      s += o.rows;
+      size = box.size[p];
     }
-    K += ak;
-    S += as;
+    uint64_t all;
+    const uint64_t at = block_excl3<kAsm>(pack3(o.rows, size, 0), wtot3, &all);
+    if (k < K) {
+      o.seg0 = S + unpack3(at, 0);
+      o.alloc = P + unpack3(at, 1);
+      comps[k] = o;
+      for (int r = 0; r < o.rows; ++r) seg_comp[o.seg0 + r] = k;
+    }
+    S += unpack3(all, 0);
+    P += unpack3(all, 1);
   }
-  if (threadIdx.x == 0) {
+  if (t == 0) {
     counters[kCntKept] = K;
     counters[kCntSegs] = S;
   }
-  __syncthreads();
-  for (int k = wave; k < K; k += kTB / 64) {
-    const int s0 = comps[k].seg0, rows = comps[k].rows;
-    for (int j = lane; j < rows; j += 64) seg_comp[s0 + j] = k;
-  }
 }
+static_assert(kAsm == 1024 && (1 << 20) / kItems <= kAsm, "a thread per block, ten bisections");
 
 // label[p] = component id of pixel p (-1: no component)
 __global__ __launch_bounds__(kTB) void tr_label_kernel(const int* __restrict__ root,
@@ -475,185 +530,328 @@ __device__ inline int pow2_from(int n, int least) {
   return P;
 }
 
-// One workgroup per beam (component k, one row).  Beams of up to 256 points (a
-// trunk 1.5 m away covers 180 columns of 2048) rank every point against all
-// the others from LDS, one point per thread; up to kSegLds points are sorted
-// in LDS; longer ones rank from memory.  With one wave per beam and a rank
-// loop per axis the few longest beams set the kernel's time: 59 us for the
-// 1,400 beams of a 128 x 2048 scan.
-__global__ __launch_bounds__(kTB) void tr_vertex_kernel(
-    const float4* __restrict__ cloud, const int* __restrict__ root,
-    const int* __restrict__ seg_comp, const TrComp* __restrict__ comps,
-    int* __restrict__ counters, TrCfgDev cfg, SegOut* __restrict__ seg_out,
-    int* __restrict__ cols, float4* __restrict__ tmp) {
+struct BeamLds {
+  float4 sp[kSegLds];
+  int sc[kSegLds];
+  unsigned long long srt[kSegLds];
+  unsigned long long keepw[kSegLds / 64];
+  int wcount[kTB / 64];
+  int base, m;
+  float med[3];
+  float4 first, last;
+};
+
+// A beam by the whole workgroup.  Up to kSegLds points are sorted in LDS;
+// longer beams rank every point against all the others from memory.
+__device__ inline void beam_block(const float4* __restrict__ cloud, const int* __restrict__ root,
+                                  const TrComp& comp, int row, int* alloc, const TrCfgDev& cfg,
+                                  SegOut* __restrict__ out, int* __restrict__ cols,
+                                  float4* __restrict__ tmp, BeamLds& B) {
   constexpr int kWaves = kTB / 64;
-  __shared__ float4 sp[kSegLds];
-  __shared__ int sc[kSegLds];
-  __shared__ unsigned long long srt[kSegLds];
-  __shared__ unsigned long long keepw[kSegLds / 64];
-  __shared__ int wcount[kWaves];
-  __shared__ int s_base, s_m;
-  __shared__ float s_med[3];
-  __shared__ float4 s_first, s_last;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int S = counters[kCntSegs];
-  for (int s = blockIdx.x; s < S; s += gridDim.x) {
-    const TrComp comp = comps[seg_comp[s]];
-    const int row = comp.row1 - (s - comp.seg0);
-    const float4* line = cloud + (size_t)row * cfg.W;
-    const int* rline = root + (size_t)row * cfg.W;
-    // the beam's points in column order
-    auto gather = [&](auto put) {
-      int run = 0;
-      for (int c0 = comp.col0; c0 <= comp.col1; c0 += kTB) {
-        const int c = c0 + t;
-        const bool in = c <= comp.col1 && rline[c] == comp.root;
-        const uint64_t b = __builtin_amdgcn_ballot_w64(in);
-        if (lane == 0) wcount[wave] = __builtin_popcountll(b);
-        __syncthreads();
-        int off = run + __builtin_popcountll(b & ((1ull << lane) - 1ull));
-        for (int w = 0; w < kWaves; ++w) {
-          off += w < wave ? wcount[w] : 0;
-          run += wcount[w];
-        }
-        if (in) put(off, c);
-        __syncthreads();
+  const float4* line = cloud + (size_t)row * cfg.W;
+  const int* rline = root + (size_t)row * cfg.W;
+  // the beam's points in column order
+  auto gather = [&](auto put) {
+    int run = 0;
+    for (int c0 = comp.col0; c0 <= comp.col1; c0 += kTB) {
+      const int c = c0 + t;
+      const bool in = c <= comp.col1 && rline[c] == comp.root;
+      const uint64_t b = __builtin_amdgcn_ballot_w64(in);
+      if (lane == 0) B.wcount[wave] = __builtin_popcountll(b);
+      __syncthreads();
+      int off = run + __builtin_popcountll(b & ((1ull << lane) - 1ull));
+      for (int w = 0; w < kWaves; ++w) {
+        off += w < wave ? B.wcount[w] : 0;
+        run += B.wcount[w];
       }
-      return run;
+      if (in) put(off, c);
+      __syncthreads();
+    }
+    return run;
+  };
+  const int n = gather([&](int j, int c) {
+    if (j < kSegLds) {
+      B.sc[j] = c;
+      B.sp[j] = line[c];
+    }
+  });
+  const bool in_lds = n <= kSegLds;
+  if (t == 0) {
+    B.base = atomicAdd(alloc, n);
+    B.m = 0;
+    B.med[0] = B.med[1] = B.med[2] = 0.f;
+  }
+  __syncthreads();
+  const int base = B.base;
+  if (!in_lds) {
+    gather([&](int j, int c) { cols[base + j] = c; });
+    __syncthreads();
+  }
+  auto C = [&](int j) -> int { return in_lds ? B.sc[j] : cols[base + j]; };
+  auto P = [&](int j) -> float4 { return in_lds ? B.sp[j] : line[cols[base + j]]; };
+  // medians: the element of rank floor(n / 2) by (value, index)
+  const int mid = n / 2;
+  if (!in_lds) {
+    for (int i = t; i < n; i += kTB) {
+      const float4 v = P(i);
+      int rx = 0, ry = 0, rz = 0;
+      for (int j = 0; j < n; ++j) {
+        const float4 q = P(j);
+        rx += (q.x < v.x || (q.x == v.x && j < i)) ? 1 : 0;
+        ry += (q.y < v.y || (q.y == v.y && j < i)) ? 1 : 0;
+        rz += (q.z < v.z || (q.z == v.z && j < i)) ? 1 : 0;
+      }
+      if (rx == mid) B.med[0] = v.x;
+      if (ry == mid) B.med[1] = v.y;
+      if (rz == mid) B.med[2] = v.z;
+    }
+  } else {
+    const int Q = pow2_from(n, 2);
+    for (int a = 0; a < 3; ++a) {
+      for (int j = t; j < Q; j += kTB)
+        B.srt[j] =
+            j < n ? ((unsigned long long)order_key(axis_of(B.sp[j], a)) << 32) | (unsigned)j
+                  : ~0ull;
+      bitonic(B.srt, Q, [](unsigned long long x, unsigned long long y) { return x < y; });
+      if (t == 0) B.med[a] = axis_of(B.sp[(uint32_t)B.srt[mid]], a);
+      __syncthreads();
+    }
+  }
+  __syncthreads();
+  const float med[3] = {B.med[0], B.med[1], B.med[2]};
+  auto near = [&](const float4& p) {
+    return dist3(p.x, p.y, p.z, med[0], med[1], med[2]) < cfg.max_dist;
+  };
+  int mw = 0;
+  for (int i0 = 0; i0 < n; i0 += kTB) {
+    const int i = i0 + t;
+    const uint64_t b = __builtin_amdgcn_ballot_w64(i < n && near(P(i)));
+    if (in_lds && lane == 0) B.keepw[(i0 >> 6) + wave] = b;
+    mw += __builtin_popcountll(b);
+  }
+  if (lane == 0 && mw) atomicAdd(&B.m, mw);
+  __syncthreads();
+  const int m = B.m;
+  if (m > 1) {
+    auto place = [&](int rank, const float4& p) {
+      tmp[base + rank] = p;
+      if (rank == 0) B.first = p;
+      if (rank == m - 1) B.last = p;
     };
-    const int n = gather([&](int j, int c) {
-      if (j < kSegLds) {
-        sc[j] = c;
-        sp[j] = line[c];
-      }
-    });
-    SegOut o;
-    o.med = make_float4(0.f, 0.f, 0.f, 0.f);
-    o.radius = 0.0;
-    o.valid = 0;
-    o.m = 0;
-    o.start = 0;
-    o.pad = 0;
-    if (n > cfg.min_row_points) {
-      const bool in_lds = n <= kSegLds;
-      if (t == 0) {
-        s_base = atomicAdd(counters + kCntAlloc, n);
-        s_m = 0;
-        s_med[0] = s_med[1] = s_med[2] = 0.f;
-      }
-      __syncthreads();
-      const int base = s_base;
-      if (!in_lds) {
-        gather([&](int j, int c) { cols[base + j] = c; });
-        __syncthreads();
-      }
-      auto C = [&](int j) -> int { return in_lds ? sc[j] : cols[base + j]; };
-      auto P = [&](int j) -> float4 { return in_lds ? sp[j] : line[cols[base + j]]; };
-      // medians: the element of rank floor(n / 2) by (value, index)
-      const int mid = n / 2;
-      if (n <= kTB || !in_lds) {
-        for (int i = t; i < n; i += kTB) {
-          const float4 v = P(i);
-          int rx = 0, ry = 0, rz = 0;
-          for (int j = 0; j < n; ++j) {
-            const float4 q = P(j);
-            rx += (q.x < v.x || (q.x == v.x && j < i)) ? 1 : 0;
-            ry += (q.y < v.y || (q.y == v.y && j < i)) ? 1 : 0;
-            rz += (q.z < v.z || (q.z == v.z && j < i)) ? 1 : 0;
-          }
-          if (rx == mid) s_med[0] = v.x;
-          if (ry == mid) s_med[1] = v.y;
-          if (rz == mid) s_med[2] = v.z;
-        }
-      } else {
-        const int Q = pow2_from(n, 2 * kTB);
-        for (int a = 0; a < 3; ++a) {
-          for (int j = t; j < Q; j += kTB)
-            srt[j] = j < n ? ((unsigned long long)order_key(axis_of(sp[j], a)) << 32) | (unsigned)j
-                           : ~0ull;
-          bitonic(srt, Q, [](unsigned long long x, unsigned long long y) { return x < y; });
-          if (t == 0) s_med[a] = axis_of(sp[(uint32_t)srt[mid]], a);
-          __syncthreads();
-        }
-      }
-      __syncthreads();
-      const float med[3] = {s_med[0], s_med[1], s_med[2]};
-      // kept points
-      auto near = [&](const float4& p) {
-        return dist3(p.x, p.y, p.z, med[0], med[1], med[2]) < cfg.max_dist;
-      };
-      int mw = 0;
+    if (in_lds) {
+      // kept indices, then sorted (all ones: past the end)
+      const int Q = pow2_from(m, 2);
+      int before = 0;
+      for (int w = 0; w < wave; ++w) before += 64 * w < n ? __builtin_popcountll(B.keepw[w]) : 0;
       for (int i0 = 0; i0 < n; i0 += kTB) {
         const int i = i0 + t;
-        const uint64_t b = __builtin_amdgcn_ballot_w64(i < n && near(P(i)));
-        if (in_lds && lane == 0) keepw[(i0 >> 6) + wave] = b;
-        mw += __builtin_popcountll(b);
+        const uint64_t b = i0 + 64 * wave < n ? B.keepw[(i0 >> 6) + wave] : 0ull;
+        if (i < n && ((b >> lane) & 1ull))
+          B.srt[before + __builtin_popcountll(b & ((1ull << lane) - 1ull))] = (unsigned)i;
+        for (int w = wave; w < wave + kWaves; ++w)
+          before += i0 + 64 * w < n ? __builtin_popcountll(B.keepw[(i0 >> 6) + w]) : 0;
       }
-      if (lane == 0 && mw) atomicAdd(&s_m, mw);
-      __syncthreads();
-      const int m = s_m;
-      o.med = make_float4(med[0], med[1], med[2], 0.f);
-      o.m = m;
-      o.start = base;
-      if (m > 1) {
-        auto place = [&](int rank, const float4& p) {
-          tmp[base + rank] = p;
-          if (rank == 0) s_first = p;
-          if (rank == m - 1) s_last = p;
-        };
-        if (n <= kTB) {
-          if (t < n && ((keepw[wave] >> lane) & 1ull)) {
-            const float4 p = sp[t];
-            const int ci = sc[t];
-            int rank = 0;
-            for (int w = 0; w <= (n - 1) >> 6; ++w)
-              for (uint64_t b = keepw[w]; b != 0; b &= b - 1) {
-                const int j = 64 * w + (int)__builtin_ctzll(b);
-                rank += zless(sp[j], sc[j], p, ci) ? 1 : 0;
-              }
-            place(rank, p);
-          }
-        } else if (in_lds) {
-          // kept indices, then sorted (index -1: past the end)
-          const int Q = pow2_from(m, 2);
-          int before = 0;
-          for (int w = 0; w < wave; ++w) before += __builtin_popcountll(keepw[w]);
-          for (int i0 = 0; i0 < n; i0 += kTB) {
-            const int i = i0 + t;
-            const uint64_t b = i0 + 64 * wave < n ? keepw[(i0 >> 6) + wave] : 0ull;
-            if (i < n && ((b >> lane) & 1ull))
-              srt[before + __builtin_popcountll(b & ((1ull << lane) - 1ull))] = (unsigned)i;
-            for (int w = wave; w < wave + kWaves; ++w)
-              before += i0 + 64 * w < n ? __builtin_popcountll(keepw[(i0 >> 6) + w]) : 0;
-          }
-          for (int j = m + t; j < Q; j += kTB) srt[j] = ~0ull;
-          bitonic(srt, Q, [&](unsigned long long x, unsigned long long y) {
-            if (x == ~0ull) return false;
-            if (y == ~0ull) return true;
-            return zless(sp[x], sc[x], sp[y], sc[y]);
-          });
-          for (int j = t; j < m; j += kTB) place(j, sp[srt[j]]);
-        } else {
-          for (int i = t; i < n; i += kTB) {
-            const float4 p = P(i);
-            if (!near(p)) continue;
-            const int ci = C(i);
-            int rank = 0;
-            for (int j = 0; j < n; ++j) {
-              const float4 q = P(j);
-              if (near(q) && zless(q, C(j), p, ci)) ++rank;
-            }
-            place(rank, p);
-          }
+      for (int j = m + t; j < Q; j += kTB) B.srt[j] = ~0ull;
+      bitonic(B.srt, Q, [&](unsigned long long x, unsigned long long y) {
+        if (x == ~0ull) return false;
+        if (y == ~0ull) return true;
+        return zless(B.sp[x], B.sc[x], B.sp[y], B.sc[y]);
+      });
+      for (int j = t; j < m; j += kTB) place(j, B.sp[B.srt[j]]);
+    } else {
+      for (int i = t; i < n; i += kTB) {
+        const float4 p = P(i);
+        if (!near(p)) continue;
+        const int ci = C(i);
+        int rank = 0;
+        for (int j = 0; j < n; ++j) {
+          const float4 q = P(j);
+          if (near(q) && zless(q, C(j), p, ci)) ++rank;
         }
-        __syncthreads();
-        o.radius = cfg.radius_scale * (double)dist3(s_first.x, s_first.y, s_first.z, s_last.x,
-                                                    s_last.y, s_last.z);
-        o.valid = 1;
+        place(rank, p);
       }
-      __syncthreads();  // LDS reused by the next beam
     }
-    if (t == 0) seg_out[s] = o;
+    __syncthreads();
+  }
+  if (t == 0) {
+    SegOut o;
+    o.med = make_float4(med[0], med[1], med[2], 0.f);
+    o.radius = m > 1 ? cfg.radius_scale * (double)dist3(B.first.x, B.first.y, B.first.z,
+                                                        B.last.x, B.last.y, B.last.z)
+                     : 0.0;
+    o.valid = m > 1 ? 1 : 0;
+    o.m = m;
+    o.start = base;
+    o.pad = 0;
+    *out = o;
+  }
+  __syncthreads();  // LDS is reused
+}
+
+// A beam of n <= kWaveBeam points (LDS, column order, padded with infinities
+// to a multiple of kRankStep) by one wave, kWaveBeam / 64 points per lane.
+// Every point is ranked against all the others, kRankStep LDS reads in flight
+// (the columns increase with the index, so ties go by index).
+constexpr int kWaveBeam = 128;
+constexpr int kRankStep = 8;
+__device__ inline void beam_wave(const float4* sp, int n, int* alloc, const TrCfgDev& cfg,
+                                 SegOut* __restrict__ out, float4* __restrict__ tmp) {
+  constexpr int kPer = kWaveBeam / 64;
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  if (lane == 0) base = atomicAdd(alloc, n);
+  float4 v[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u)
+    v[u] = 64 * u + lane < n ? sp[64 * u + lane] : make_float4(NAN, NAN, NAN, 0.f);
+  const int mid = n / 2;
+  float med[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    if (64 * u >= n) break;
+    const int i = 64 * u + lane;
+    int rx = 0, ry = 0, rz = 0;
+    for (int j0 = 0; j0 < n; j0 += kRankStep) {
+      float4 q[kRankStep];
+#pragma unroll
+      for (int e = 0; e < kRankStep; ++e) q[e] = sp[j0 + e];
+#pragma unroll
+      for (int e = 0; e < kRankStep; ++e) {
+        const bool before = j0 + e < i;
+        rx += (q[e].x < v[u].x || (q[e].x == v[u].x && before)) ? 1 : 0;
+        ry += (q[e].y < v[u].y || (q[e].y == v[u].y && before)) ? 1 : 0;
+        rz += (q[e].z < v[u].z || (q[e].z == v[u].z && before)) ? 1 : 0;
+      }
+    }
+    const uint64_t bx = __builtin_amdgcn_ballot_w64(i < n && rx == mid);
+    const uint64_t by = __builtin_amdgcn_ballot_w64(i < n && ry == mid);
+    const uint64_t bz = __builtin_amdgcn_ballot_w64(i < n && rz == mid);
+    if (bx) med[0] = __shfl(v[u].x, (int)__builtin_ctzll(bx), 64);
+    if (by) med[1] = __shfl(v[u].y, (int)__builtin_ctzll(by), 64);
+    if (bz) med[2] = __shfl(v[u].z, (int)__builtin_ctzll(bz), 64);
+  }
+  uint64_t keep[kPer];
+  int m = 0;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    keep[u] = __builtin_amdgcn_ballot_w64(
+        64 * u + lane < n &&
+        dist3(v[u].x, v[u].y, v[u].z, med[0], med[1], med[2]) < cfg.max_dist);
+    m += __builtin_popcountll(keep[u]);
+  }
+  base = __shfl(base, 0, 64);
+  SegOut o;
+  o.med = make_float4(med[0], med[1], med[2], 0.f);
+  o.radius = 0.0;
+  o.valid = 0;
+  o.m = m;
+  o.start = base;
+  o.pad = 0;
+  if (m > 1) {
+    float4 first = make_float4(0.f, 0.f, 0.f, 0.f), last = first;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      if (keep[u] == 0) continue;
+      const int i = 64 * u + lane;
+      int rank = 0;
+      for (int j0 = 0; j0 < n; j0 += kRankStep) {
+        float4 q[kRankStep];
+#pragma unroll
+        for (int e = 0; e < kRankStep; ++e) q[e] = sp[j0 + e];
+#pragma unroll
+        for (int e = 0; e < kRankStep; ++e) {
+          const int j = j0 + e;
+          uint64_t kw = keep[0];
+#pragma unroll
+          for (int x = 1; x < kPer; ++x) kw = j >= 64 * x ? keep[x] : kw;
+          const bool kj = ((kw >> (j & 63)) & 1ull) != 0;  // uniform
+          rank += kj && zless(q[e], j, v[u], i) ? 1 : 0;
+        }
+      }
+      const bool mine = ((keep[u] >> lane) & 1ull) != 0;
+      if (mine) tmp[base + rank] = v[u];
+      const uint64_t bf = __builtin_amdgcn_ballot_w64(mine && rank == 0);
+      const uint64_t bl = __builtin_amdgcn_ballot_w64(mine && rank == m - 1);
+      if (bf) {
+        const int l = (int)__builtin_ctzll(bf);
+        first = make_float4(__shfl(v[u].x, l, 64), __shfl(v[u].y, l, 64), __shfl(v[u].z, l, 64),
+                            0.f);
+      }
+      if (bl) {
+        const int l = (int)__builtin_ctzll(bl);
+        last = make_float4(__shfl(v[u].x, l, 64), __shfl(v[u].y, l, 64), __shfl(v[u].z, l, 64),
+                           0.f);
+      }
+    }
+    o.radius = cfg.radius_scale * (double)dist3(first.x, first.y, first.z, last.x, last.y, last.z);
+    o.valid = 1;
+  }
+  if (lane == 0) *out = o;
+}
+
+// A wave per beam (component k, one row); beams of more than kWaveBeam points
+// (a trunk 1.5 m away covers 180 columns of 2048) then take the workgroup.
+// 1,955 beams of a 128 x 2048 scan (half of them under 10 points, the longest
+// 68): 23 us, by the longest beams' rank loops; 41 us with a workgroup per beam
+// and one counter for the points of all beams, 59 us with a wave per beam and a
+// rank loop per axis.
+__global__ __launch_bounds__(kTB) void tr_vertex_kernel(
+    const float4* __restrict__ cloud, const int* __restrict__ root,
+    const int* __restrict__ seg_comp, TrComp* __restrict__ comps,
+    const int* __restrict__ counters, TrCfgDev cfg, SegOut* __restrict__ seg_out,
+    int* __restrict__ cols, float4* __restrict__ tmp) {
+  constexpr int kWaves = kTB / 64;
+  __shared__ BeamLds B;
+  __shared__ int s_long[kWaves];
+  static_assert(kWaves * (kWaveBeam + kRankStep) <= kSegLds, "the waves' parts of the LDS stage");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int S = counters[kCntSegs];
+  for (int s0 = blockIdx.x * kWaves; s0 < S; s0 += gridDim.x * kWaves) {
+    const int s = s0 + wave;
+    int is_long = 0;
+    if (s < S) {
+      const int k = seg_comp[s];
+      const TrComp comp = comps[k];
+      const int row = comp.row1 - (s - comp.seg0);
+      const float4* line = cloud + (size_t)row * cfg.W;
+      const int* rline = root + (size_t)row * cfg.W;
+      float4* sp = B.sp + wave * (kWaveBeam + kRankStep);
+      int n = 0;
+      for (int c0 = comp.col0; c0 <= comp.col1; c0 += 64) {
+        const int c = c0 + lane;
+        const bool in = c <= comp.col1 && rline[c] == comp.root;
+        const uint64_t b = __builtin_amdgcn_ballot_w64(in);
+        const int off = n + __builtin_popcountll(b & ((1ull << lane) - 1ull));
+        if (in && off < kWaveBeam) sp[off] = line[c];
+        n += __builtin_popcountll(b);
+      }
+      if (n <= cfg.min_row_points) {
+        if (lane == 0) {
+          SegOut o;
+          o.med = make_float4(0.f, 0.f, 0.f, 0.f);
+          o.radius = 0.0;
+          o.valid = o.m = o.start = o.pad = 0;
+          seg_out[s] = o;
+        }
+      } else if (n <= kWaveBeam) {
+        if (lane < kRankStep) sp[n + lane] = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+        __builtin_amdgcn_wave_barrier();
+        beam_wave(sp, n, &comps[k].alloc, cfg, seg_out + s, tmp);
+      } else {
+        is_long = 1;
+      }
+    }
+    if (lane == 0) s_long[wave] = is_long;
+    __syncthreads();
+    for (int w = 0; w < kWaves; ++w) {
+      if (!s_long[w]) continue;
+      const int k = seg_comp[s0 + w];
+      const TrComp comp = comps[k];
+      beam_block(cloud, root, comp, comp.row1 - (s0 + w - comp.seg0), &comps[k].alloc, cfg,
+                 seg_out + s0 + w, cols, tmp, B);
+    }
+    __syncthreads();
   }
 }
 
@@ -669,44 +867,67 @@ __global__ __launch_bounds__(kAsm) void tr_assemble_kernel(
     const int* __restrict__ counters, TrCfgDev cfg, int2* __restrict__ seg_at,
     int2* __restrict__ comp_at, int32_t* __restrict__ tree_offsets,
     int32_t* __restrict__ point_offsets, int32_t* __restrict__ out_counts) {
-  __shared__ int wtot[kAsm / 64];
+  __shared__ unsigned long long wtot[kAsm / 64];
+  __shared__ int2 s_comp[kAsm];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int K = counters[kCntKept];
-  for (int k = wave; k < K; k += kAsm / 64) {
-    const int s0 = comps[k].seg0, rows = comps[k].rows;
-    int nv = 0, np = 0;
-    for (int j0 = 0; j0 < rows; j0 += 64) {
-      const int j = j0 + lane;
-      int valid = 0, m = 0;
-      if (j < rows) {
-        valid = seg_out[s0 + j].valid;
-        m = seg_out[s0 + j].m;
-      }
-      const uint64_t b = __builtin_amdgcn_ballot_w64(valid != 0);
-      const int rank = nv + __builtin_popcountll(b & ((1ull << lane) - 1ull));
-      const bool use = valid && rank < cfg.max_vertices;
-      const int incl = wave_incl(use ? m : 0, lane);
-      if (j < rows) seg_at[s0 + j] = make_int2(use ? rank : -1, np + incl - (use ? m : 0));
-      nv += __builtin_popcountll(b);
-      np += __shfl(incl, 63, 64);
+  constexpr int kWaves = kAsm / 64;
+  constexpr int kAhead = 4;  // components per wave whose loads are in flight
+  for (int k0 = wave; k0 < K; k0 += kWaves * kAhead) {
+    int s0[kAhead], rows[kAhead], nv[kAhead], np[kAhead], most = 0;
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int k = k0 + u * kWaves;
+      s0[u] = k < K ? comps[k].seg0 : 0;
+      rows[u] = k < K ? comps[k].rows : 0;
+      nv[u] = np[u] = 0;
     }
-    if (lane == 0) comp_at[k] = make_int2(nv, np);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) most = max(most, rows[u]);
+    for (int j0 = 0; j0 < most; j0 += 64) {
+      const int j = j0 + lane;
+      int valid[kAhead], m[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        valid[u] = j < rows[u] ? seg_out[s0[u] + j].valid : 0;
+        m[u] = j < rows[u] ? seg_out[s0[u] + j].m : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const uint64_t b = __builtin_amdgcn_ballot_w64(valid[u] != 0);
+        const int rank = nv[u] + __builtin_popcountll(b & ((1ull << lane) - 1ull));
+        const bool use = valid[u] && rank < cfg.max_vertices;
+        const int incl = wave_incl(use ? m[u] : 0, lane);
+        if (j < rows[u])
+          seg_at[s0[u] + j] = make_int2(use ? rank : -1, np[u] + incl - (use ? m[u] : 0));
+        nv[u] += __builtin_popcountll(b);
+        np[u] += __shfl(incl, 63, 64);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (lane == 0 && k0 + u * kWaves < K) {
+        if (k0 + u * kWaves < kAsm)
+          s_comp[k0 + u * kWaves] = make_int2(nv[u], np[u]);
+        else
+          comp_at[k0 + u * kWaves] = make_int2(nv[u], np[u]);
+      }
   }
   __syncthreads();
   int ct = 0, cv = 0, cp = 0;
   for (int k0 = 0; k0 < K; k0 += kAsm) {
     const int k = k0 + (int)threadIdx.x;
-    const int2 v = k < K ? comp_at[k] : make_int2(0, 0);
+    const int2 v = k >= K ? make_int2(0, 0) : (k < kAsm ? s_comp[k] : comp_at[k]);
     const bool tree = k < K && v.x > cfg.min_vertices;
-    int at, av, ap;
-    const int et = block_excl<kAsm>(tree ? 1 : 0, wtot, &at);
-    const int ev = block_excl<kAsm>(tree ? min(v.x, cfg.max_vertices) : 0, wtot, &av);
-    const int ep = block_excl<kAsm>(tree ? v.y : 0, wtot, &ap);
-    if (k < K) comp_at[k] = make_int2(tree ? cv + ev : -1, cp + ep);
-    if (tree && ct + et < cfg.cap_trees) tree_offsets[ct + et] = cv + ev;
-    ct += at;
-    cv += av;
-    cp += ap;
+    uint64_t all;
+    const uint64_t e = block_excl3<kAsm>(
+        tree ? pack3(1, min(v.x, cfg.max_vertices), v.y) : 0ull, wtot, &all);
+    const int vi = cv + unpack3(e, 1), ti = ct + unpack3(e, 0);
+    if (k < K) comp_at[k] = make_int2(tree ? vi : -1, cp + unpack3(e, 2));
+    if (tree && ti < cfg.cap_trees) tree_offsets[ti] = vi;
+    ct += unpack3(all, 0);
+    cv += unpack3(all, 1);
+    cp += unpack3(all, 2);
   }
   if (threadIdx.x == 0) {
     const bool over = ct > cfg.cap_trees || cv > cfg.cap_vertices || cp > cfg.cap_points;
@@ -723,14 +944,15 @@ __global__ __launch_bounds__(kAsm) void tr_assemble_kernel(
   }
 }
 
-// The used beams' vertex records and points, one wave per beam.
+// The used beams' vertex records and points, one wave per beam; medians
+// (nullable): 3 floats per vertex for the line fits.
 __global__ __launch_bounds__(64) void tr_copy_kernel(
     const int* __restrict__ seg_comp, const TrComp* __restrict__ comps,
     const int* __restrict__ counters, const SegOut* __restrict__ seg_out,
     const int2* __restrict__ seg_at, const int2* __restrict__ comp_at, TrCfgDev cfg,
     const float4* __restrict__ tmp, int32_t* __restrict__ vertex_int,
     double* __restrict__ vertex_f64, int32_t* __restrict__ point_offsets,
-    float4* __restrict__ points) {
+    float4* __restrict__ points, float* __restrict__ medians) {
   const int S = counters[kCntSegs];
   for (int s = blockIdx.x; s < S; s += gridDim.x) {
     const int k = seg_comp[s];
@@ -749,6 +971,11 @@ __global__ __launch_bounds__(64) void tr_copy_kernel(
       vertex_f64[4 * (size_t)vi + 2] = (double)o.med.y;
       vertex_f64[4 * (size_t)vi + 3] = (double)o.med.z;
       point_offsets[vi] = po;
+      if (medians) {
+        medians[3 * (size_t)vi + 0] = o.med.x;
+        medians[3 * (size_t)vi + 1] = o.med.y;
+        medians[3 * (size_t)vi + 2] = o.med.z;
+      }
     }
     if (po + o.m > cfg.cap_points) continue;
     for (int j = threadIdx.x; j < o.m; j += 64) points[po + j] = tmp[o.start + j];
@@ -757,13 +984,11 @@ __global__ __launch_bounds__(64) void tr_copy_kernel(
 
 }  // namespace
 
-extern "C" {
-
-int sloam_trellis(sloam_ctx* ctx, const float* d_cloud, int32_t height, int32_t width,
-                  const sloam_trellis_cfg* cfg, int32_t* d_labels, int32_t cap_trees,
-                  int32_t cap_vertices, int32_t cap_points, int32_t* d_tree_offsets,
-                  int32_t* d_vertex_int, double* d_vertex_f64, int32_t* d_point_offsets,
-                  float* d_points, int32_t* d_counts) {
+int sloam_trellis_medians(sloam_ctx* ctx, const float* d_cloud, int32_t height, int32_t width,
+                          const sloam_trellis_cfg* cfg, int32_t* d_labels, int32_t cap_trees,
+                          int32_t cap_vertices, int32_t cap_points, int32_t* d_tree_offsets,
+                          int32_t* d_vertex_int, double* d_vertex_f64, int32_t* d_point_offsets,
+                          float* d_points, int32_t* d_counts, float* d_medians) {
   if (!ctx || !cfg || !d_counts || height < 0 || width < 0) return SLOAM_ERR_INVALID_ARG;
   if (cap_trees < 0 || cap_vertices < 0 || cap_points < 0) return SLOAM_ERR_INVALID_ARG;
   if (!d_tree_offsets || !d_vertex_int || !d_vertex_f64 || !d_point_offsets ||
@@ -800,7 +1025,7 @@ int sloam_trellis(sloam_ctx* ctx, const float* d_cloud, int32_t height, int32_t 
   const size_t need = 10 * al(ib) + al(sizeof(int2) * (size_t)n1) +
                       al(sizeof(TrComp) * n_comps) + al(sizeof(int2) * n_comps) +
                       al(sizeof(SegOut) * (size_t)n1) + al(sizeof(float4) * (size_t)n1) +
-                      al(sizeof(int) * (size_t)n_blocks) + al(sizeof(int2) * (size_t)n_blocks) +
+                      2 * al(sizeof(int) * (size_t)n_blocks) +
                       al(sizeof(int) * kCntN);
   void* base = nullptr;
   int st = sloam_ctx_scratch(ctx, 2, need, &base);
@@ -828,7 +1053,7 @@ int sloam_trellis(sloam_ctx* ctx, const float* d_cloud, int32_t height, int32_t 
   SegOut* seg_out = (SegOut*)take(sizeof(SegOut) * (size_t)n1);
   float4* tmp = (float4*)take(sizeof(float4) * (size_t)n1);
   int* block_roots = (int*)take(sizeof(int) * (size_t)n_blocks);
-  int2* block_kept = (int2*)take(sizeof(int2) * (size_t)n_blocks);
+  int* block_kept = (int*)take(sizeof(int) * (size_t)n_blocks);
   int* counters = (int*)take(sizeof(int) * kCntN);
   const float4* cloud = reinterpret_cast<const float4*>(d_cloud);
   if (N == 0) {
@@ -842,14 +1067,16 @@ int sloam_trellis(sloam_ctx* ctx, const float* d_cloud, int32_t height, int32_t 
           (height - 1) / kTileH * width + (width - 1) / kTileW * height;
       hipLaunchKernelGGL(tr_tile_kernel,
                          dim3((width + kTileW - 1) / kTileW, (height + kTileH - 1) / kTileH),
-                         dim3(kTB), 0, ctx->stream, cloud, dc, L, box, counters);
+                         dim3(kTileB), 0, ctx->stream, cloud, dc, L, box, counters);
       if (n_border > 0)
         hipLaunchKernelGGL(tr_border_kernel, dim3((n_border + kTB - 1) / kTB), dim3(kTB), 0,
                            ctx->stream, cloud, dc, L);
       hipLaunchKernelGGL(tr_flatten_kernel, dim3(n_blocks), dim3(kTB), 0, ctx->stream, N, L, root,
                          box, block_roots);
       hipLaunchKernelGGL(tr_number_kernel, dim3(n_blocks), dim3(kTB), 0, ctx->stream, root, box,
-                         dc, block_roots, id, kept, block_kept, comps, seg_comp, counters);
+                         dc, block_roots, id, kept, block_kept, counters);
+      hipLaunchKernelGGL(tr_layout_kernel, dim3(1), dim3(kAsm), 0, ctx->stream, box, dc, n_blocks,
+                         id, kept, block_kept, comps, seg_comp, counters);
       if (d_labels)
         hipLaunchKernelGGL(tr_label_kernel, dim3((N + kTB - 1) / kTB), dim3(kTB), 0, ctx->stream,
                            root, id, N, d_labels);
@@ -871,10 +1098,22 @@ int sloam_trellis(sloam_ctx* ctx, const float* d_cloud, int32_t height, int32_t 
       hipLaunchKernelGGL(tr_copy_kernel, dim3(std::min(kVtxBlocks, N)), dim3(64), 0, ctx->stream,
                          seg_comp, comps, counters, seg_out, seg_at, comp_at, dc, tmp,
                          d_vertex_int, d_vertex_f64, d_point_offsets,
-                         reinterpret_cast<float4*>(d_points));
+                         reinterpret_cast<float4*>(d_points), d_medians);
   }
   SLOAM_HIP(ctx, hipGetLastError());
   return SLOAM_OK;
+}
+
+extern "C" {
+
+int sloam_trellis(sloam_ctx* ctx, const float* d_cloud, int32_t height, int32_t width,
+                  const sloam_trellis_cfg* cfg, int32_t* d_labels, int32_t cap_trees,
+                  int32_t cap_vertices, int32_t cap_points, int32_t* d_tree_offsets,
+                  int32_t* d_vertex_int, double* d_vertex_f64, int32_t* d_point_offsets,
+                  float* d_points, int32_t* d_counts) {
+  return sloam_trellis_medians(ctx, d_cloud, height, width, cfg, d_labels, cap_trees, cap_vertices,
+                               cap_points, d_tree_offsets, d_vertex_int, d_vertex_f64,
+                               d_point_offsets, d_points, d_counts, nullptr);
 }
 
 }  // extern "C"

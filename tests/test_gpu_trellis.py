@@ -96,6 +96,29 @@ def test_medians_of_long_beams_with_ties(ctx, length):
     assert len(g["tree_offsets"]) > 1
 
 
+@pytest.mark.parametrize("H,W", [(1, 1), (1, 200), (31, 63), (32, 64), (33, 65), (70, 130),
+                                 (17, 1100)])
+@pytest.mark.parametrize("fill", [0.2, 0.55, 0.8])
+def test_components_across_tiles(ctx, H, W, fill):
+    """Random masks of one depth (every neighbour links: snakes and combs at
+    0.55, one large component with holes at 0.8) at image sizes next to the 64
+    x 32 tiles, every component and beam kept; beams of up to 128 points go to
+    a wave, longer ones to a workgroup, over 1,024 to memory."""
+    rng = np.random.default_rng(H * 1000 + W)
+    cloud = np.full((H * W, 4), np.nan, np.float32)
+    on = rng.uniform(0, 1, H * W) < fill
+    r, c = np.divmod(np.flatnonzero(on), W)
+    cloud[on, 0] = 5.0 + 0.01 * c
+    cloud[on, 1] = np.round(0.3 * np.sin(c / 7.0), 2)
+    cloud[on, 2] = np.round(rng.normal(0.0, 0.1, len(c)) - 0.05 * r, 2)
+    cloud[on, 3] = r
+    kw = dict(min_label_points=1, min_row_points=1, min_vertices=1, max_vertices=40)
+    print(f"[trellis] random {H}x{W} fill {fill}", flush=True)
+    g = trellis(ctx, cloud, H, W, max_dist_to_centroid=2.0, **kw)
+    o = oracle.trellis(cloud, H, W, max_dist=2.0, **kw)
+    _same(g, o)
+
+
 def test_empty_and_overflow(ctx):
     H, W = 8, 64
     cloud = np.full((H * W, 4), np.nan, np.float32)
