@@ -21,7 +21,7 @@
 // ||(p - c) x a||^2 = (u - cu)^2 + (v - cv)^2 = s + A u + B v + K with
 // A = -2 cu, B = -2 cv, K = cu^2 + cv^2, so the test becomes
 // L < fma(u, A, fma(v, B, s)) < U with L = (r - thr)^2 - K (or -inf when
-// r <= thr) and U = (r + thr)^2 - K: two FMAs and two compares per pair.
+// r <= thr) and U = (r + thr)^2 - K: two FMAs, a clamp and a compare per pair.
 #include "common.hpp"
 
 #include <algorithm>
@@ -38,6 +38,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kHB = 8;  // hypotheses held in registers per pass over a tile
+constexpr int kScoreFill = 2048;  // score workgroups that fill the chip (8 a CU)
 constexpr int kMaxLds = 65536;  // LDS bytes per workgroup this kernel asks for
 
 struct CylFrame {
@@ -279,9 +280,34 @@ __global__ __launch_bounds__(kBlock) void cyl_seed_kernel(const float* __restric
 
 // ---------------------------------------------------------------------------
 // score: hypotheses x points, ballot/popcount inlier counts
+//
+// L < t < U is tested as med3(t, L', U') == t with L' the next float above L
+// and U' the next below U: one VALU instruction and one compare, as two
+// compares are, but one lane mask instead of two, so the scalar unit, shared
+// by the CU's four SIMDs, has two operations per 64 pairs (count, add) instead
+// of three (and).  The loop was bound by those: 19.5 cycles per 64 pairs and
+// SIMD against 15.5 now, 16 being the issue of its four VALU instructions.
+// 2000 clusters x 1024 hypotheses, 2.20e9 pairs: PLACEHOLDER.  (The product
+// on v_mfma_f32_4x4x1_16b, which rounds like fmaf, takes 18.5: it does not
+// overlap the VALU.)
 // work item = {cluster, first hypothesis, hypothesis count, unused}
 // LDS: hyp params [hcap] float4 | counts [hcap] int | u,v,s [tile] float
 // ---------------------------------------------------------------------------
+// The next float above x (NaN and +inf stay).
+__device__ inline float next_up(float x) {
+  if (!(x < INFINITY)) return x;
+  const int b = __float_as_int(x);
+  return x == 0.0f ? __int_as_float(1) : __int_as_float(x > 0.0f ? b + 1 : b - 1);
+}
+
+// Score parameters {A, B, L', U'} of a hypothesis; one whose band holds no
+// float (or that is invalid) gets A = B = 0 and L' = U' = -1: t is then
+// s >= 0, never -1.
+__device__ inline float4 score_params(const HypOut& h) {
+  const float lo = next_up(h.L), hi = -next_up(-h.U);
+  return lo <= hi ? make_float4(h.A, h.B, lo, hi) : make_float4(0.f, 0.f, -1.f, -1.f);
+}
+
 __global__ __launch_bounds__(kBlock) void cyl_score_kernel(
     const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
     const CylFrame* __restrict__ frames, const int4* __restrict__ work, int n_hyp, int hcap,
@@ -308,11 +334,11 @@ __global__ __launch_bounds__(kBlock) void cyl_score_kernel(
   const CylFrame f = frames[c];
 
   for (int t = threadIdx.x; t < hcap; t += kBlock) {
-    float4 prm = make_float4(0.f, 0.f, INFINITY, -INFINITY);
+    float4 prm = make_float4(0.f, 0.f, -1.f, -1.f);
     if (t < hc && n >= 3) {
       int32_t idx[3];
       const HypOut h = hyp_for(P, n, c, h0 + t, f, thr, max_radius, k0, k1, tag, idx, pc);
-      prm = make_float4(h.A, h.B, h.L, h.U);
+      prm = score_params(h);
       if (samples) {
         int32_t* o = samples + 3 * ((size_t)c * n_hyp + h0 + t);
         o[0] = idx[0];
@@ -362,20 +388,27 @@ __global__ __launch_bounds__(kBlock) void cyl_score_kernel(
         U[j] = q.w;
         cc[j] = 0;
       }
-      // uniform trip count: i0 lives in a scalar register, the two compares
-      // write scalar lane masks that are and-ed and popcounted on the SALU
+      // uniform trip count: i0 lives in a scalar register, the compares write
+      // scalar lane masks that are popcounted on the SALU.  All eight masks
+      // before the first count (scheduled mask by mask through one register,
+      // each compare waits for the count before it: 48 cycles per 64 pairs).
       for (int i0 = 0; i0 < tn64; i0 += 64) {
         const int i = i0 + lane;
         const float u = su[i];
         const float v = sv[i];
         const float s = ss[i];
+        uint64_t in[kHB];
+        float t[kHB], m[kHB];
 #pragma unroll
         for (int j = 0; j < kHB; ++j) {
-          const float t = __builtin_fmaf(u, A[j], __builtin_fmaf(v, B[j], s));
-          const uint64_t gt = __builtin_amdgcn_ballot_w64(t > L[j]);
-          const uint64_t lt = __builtin_amdgcn_ballot_w64(t < U[j]);
-          cc[j] += __builtin_popcountll(gt & lt);
+          t[j] = __builtin_fmaf(u, A[j], __builtin_fmaf(v, B[j], s));
+          m[j] = __builtin_amdgcn_fmed3f(t[j], L[j], U[j]);
         }
+#pragma unroll
+        for (int j = 0; j < kHB; ++j) in[j] = __builtin_amdgcn_ballot_w64(m[j] == t[j]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < kHB; ++j) cc[j] += __builtin_popcountll(in[j]);
       }
       if (lane == 0) {
 #pragma unroll
@@ -1406,6 +1439,17 @@ static int plan_layout(sloam_cyl_plan* p, const int32_t* h_offsets, int32_t n_cl
   }
   p->n_clusters = n_clusters;
   p->n_points = h_offsets[n_clusters];
+  if (cfg.hyp_chunk == 0) {
+    // no chunk asked for: 256 hypotheses a workgroup (each workgroup takes the
+    // cluster's points into the local frame, for all its hypotheses), fewer
+    // where that would leave CUs idle, down to one pass of each wave.  12
+    // trees x 1024 hypotheses: 48 workgroups took 34 us, 384 take PLACEHOLDER2.
+    const int least = kWaves * kHB;
+    p->hcap = std::min(256, round_up(cfg.n_hyp, least));
+    while (p->hcap > least &&
+           (int64_t)n_clusters * ((cfg.n_hyp + p->hcap - 1) / p->hcap) < kScoreFill)
+      p->hcap = round_up(p->hcap / 2, least);
+  }
 
   // work list: clusters by decreasing size (ties: lower index), each cluster
   // split into hypothesis chunks.  Workgroups go to the XCDs round robin
