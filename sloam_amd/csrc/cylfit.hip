@@ -9,10 +9,11 @@
 //               cluster's points through LDS tiles as (u, v, s = u^2 + v^2) and
 //               counts inliers with a wavefront ballot + popcount, 64 points per
 //               compare, eight hypotheses per pass over a tile.
-//   cyl_refit   one workgroup per cluster (one wave for small clusters): best
-//               hypothesis (max count, lowest index), inlier bit mask, FP64
-//               LO-RANSAC refit (Gauss-Newton on the 5-parameter geometric
-//               cylinder residual with inlier re-selection).
+//   cyl_refit   one workgroup per cluster (one wave for small clusters, launches
+//               per step for large ones): best hypothesis (max count, lowest
+//               index), inlier bit mask, LO-RANSAC refit (Gauss-Newton on the
+//               5-parameter geometric cylinder residual with inlier
+//               re-selection; FP32 residuals, TwoSum sums, FP64 solve).
 //
 // The inlier predicate is the reference's point-to-cylinder distance
 // (sloam/src/objects/cylinder.cpp:196-203, Cylinder::distance(const PointT&)):
@@ -56,16 +57,20 @@ struct HypOut {
   int valid;
 };
 
-__device__ inline void local_uvs(const CylFrame& f, float x, float y, float z, float* u, float* v,
-                                 float* s) {
-  const float dx = x - f.m[0];
-  const float dy = y - f.m[1];
-  const float dz = z - f.m[2];
-  const float uu = (dx * f.e1[0] + dy * f.e1[1]) + dz * f.e1[2];
-  const float vv = (dx * f.e2[0] + dy * f.e2[1]) + dz * f.e2[2];
+// the same of a point relative to the frame centre
+__device__ inline void rel_uvs(const CylFrame& f, const float d[3], float* u, float* v,
+                               float* s) {
+  const float uu = (d[0] * f.e1[0] + d[1] * f.e1[1]) + d[2] * f.e1[2];
+  const float vv = (d[0] * f.e2[0] + d[1] * f.e2[1]) + d[2] * f.e2[2];
   *u = uu;
   *v = vv;
   *s = uu * uu + vv * vv;
+}
+
+__device__ inline void local_uvs(const CylFrame& f, float x, float y, float z, float* u, float* v,
+                                 float* s) {
+  const float d[3] = {x - f.m[0], y - f.m[1], z - f.m[2]};
+  rel_uvs(f, d, u, v, s);
 }
 
 // Predicate parameters of the circle (cu, cv, r) of the local plane.
@@ -287,7 +292,7 @@ __global__ __launch_bounds__(kBlock) void cyl_seed_kernel(const float* __restric
 // by the CU's four SIMDs, has two operations per 64 pairs (count, add) instead
 // of three (and).  The loop was bound by those: 19.5 cycles per 64 pairs and
 // SIMD against 15.5 now, 16 being the issue of its four VALU instructions.
-// 2000 clusters x 1024 hypotheses, 2.20e9 pairs: PLACEHOLDER.  (The product
+// 2000 clusters x 1024 hypotheses, 2.20e9 pairs: 255 -> 227 us.  (The product
 // on v_mfma_f32_4x4x1_16b, which rounds like fmaf, takes 18.5: it does not
 // overlap the VALU.)
 // work item = {cluster, first hypothesis, hypothesis count, unused}
@@ -440,16 +445,17 @@ __global__ __launch_bounds__(kBlock) void cyl_score_kernel(
 // normal equations in FP64.  The order of every addition is fixed (no
 // atomics on values), so results do not depend on scheduling; the oracle
 // restates the same arithmetic.  Two launch forms give the same bits:
-//   per step  (large batches)  cyl_refit_init (best hypothesis, inlier mask,
-//             round-0 membership bits, initial model), then per Gauss-Newton
+//   team      (batches of clusters of up to 8,192 points, one-chunk clusters
+//             of the others, and every counted plan)
+//             cyl_refit_team: a wave or a workgroup walks every step of one
+//             cluster over its chunks, its first wave solving between steps
+//   per step  (the other clusters)  cyl_refit_init (best hypothesis, inlier
+//             mask, round-0 membership bits, initial model), then per Gauss-Newton
 //             step cyl_refit_step (one workgroup per chunk) and
 //             cyl_refit_solve (one wave per cluster: lane q sums term q over
 //             the chunks, lane 0 solves), then cyl_refit_final (the final
 //             inliers' centroid sums per chunk) and cyl_refit_finish (the
-//             output record, one wave per cluster);
-//   fused     (small batches, e.g. a keyframe's trees)  cyl_refit_init, then
-//             cyl_refit_fused: one workgroup walks every step of one cluster
-//             over its chunks, its first wave solving between steps.
+//             output record, one wave per cluster)
 // The kernels of the per-step form read the previous launch's results (no
 // fences between workgroups inside a launch).
 // ---------------------------------------------------------------------------
@@ -461,13 +467,17 @@ constexpr int kRefitGroups = kRefitBlock / kRefitGroup;
 constexpr int kRefitTerms = 20;  // 15 of J J^T (upper triangle), 5 of J d
 // largest cluster the plans take (points), and its chunks
 constexpr int kRefitMaxPoints = 1 << 17;
-constexpr int kRefitFusedChunks = kRefitMaxPoints / kRefitChunk;
-// the fused refit (a workgroup walks all steps of one cluster) takes a
-// host-planned batch of at most this many clusters of at most this many
-// chunks: beyond, one launch per step (every chunk of every cluster in
-// parallel) is faster; counted plans (a keyframe's trees) always take it
-constexpr int kRefitFusedPlanClusters = 512;
-constexpr int kRefitFusedPlanChunks = 4;
+constexpr int kRefitMaxChunks = kRefitMaxPoints / kRefitChunk;
+// A host-planned batch whose clusters have up to this many chunks goes to
+// cyl_refit_team.  A batch with larger ones has a launch per step (every chunk
+// of every cluster in parallel) for all of several chunks: the launches are
+// paid anyway (600 clusters of 2000..12000 points: 334 us for 380 with only
+// those above 4 chunks in them; without launches, 2000 clusters of up to 3
+// chunks take 336 us, with launches for 3 chunks 395).  Counted plans (a
+// keyframe's trees) always take the teams
+constexpr int kRefitTeamChunks = 4;
+// batches of up to this many clusters have a workgroup for each (four a CU)
+constexpr int kRefitTeamBlocks = 1024;
 // clusters (one wave each) per workgroup of the per-cluster solve and finish
 constexpr int kRefitWaveClusters = 4;
 
@@ -482,6 +492,7 @@ enum RefitStatus : int32_t {
 // plane orthogonal to its axis are made whenever the FP64 model changes.
 struct RefitState {
   double a[3], c[3], r;  // axis, axis point (relative to the frame centre), radius
+  double e1[3], e2[3];   // basis of the plane orthogonal to the axis
   float af[3], cf[3], rf, e1f[3], e2f[3];
   int32_t status;
   int32_t skip_round;  // round whose remaining steps are skipped (failed solve), -1
@@ -556,30 +567,82 @@ __device__ inline int block_sum_int(int v, int* lds) {
   return s;
 }
 
-// FP32 copy of the FP64 model and its basis.
+// The basis of the FP64 model and the FP32 copy of both.
 __device__ inline void refit_model_f32(RefitState& S) {
-  double e1[3], e2[3];
-  sl_basis(S.a, e1, e2);
+  sl_basis(S.a, S.e1, S.e2);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     S.af[i] = (float)S.a[i];
     S.cf[i] = (float)S.c[i];
-    S.e1f[i] = (float)e1[i];
-    S.e2f[i] = (float)e2[i];
+    S.e1f[i] = (float)S.e1[i];
+    S.e2f[i] = (float)S.e2[i];
   }
   S.rf = (float)S.r;
 }
 
-// FP32 distance of x (relative to the frame centre) to the model; w, h, rho out.
-__device__ inline float refit_dist(const RefitState& S, const float x[3], float w[3], float& h,
-                                   float& rho) {
-  const float q0 = x[0] - S.cf[0], q1 = x[1] - S.cf[1], q2 = x[2] - S.cf[2];
-  h = __builtin_fmaf(q2, S.af[2], __builtin_fmaf(q1, S.af[1], q0 * S.af[0]));
-  w[0] = __builtin_fmaf(-h, S.af[0], q0);
-  w[1] = __builtin_fmaf(-h, S.af[1], q1);
-  w[2] = __builtin_fmaf(-h, S.af[2], q2);
-  rho = sqrtf(__builtin_fmaf(w[2], w[2], __builtin_fmaf(w[1], w[1], w[0] * w[0])));
-  return rho - S.rf;
+// rho = sqrt(x) and inv = 1 / rho, both correctly rounded, from one v_rsq and
+// a Newton step each with exact residuals (Markstein 1990) instead of the
+// compiler's separate square root and divide: 9 instructions and 3 compares
+// for about 25.  Equal to sqrtf(x) and 1.0f / sqrtf(x) at every float of
+// [2^-96, 2^96) where e is not 2^-24 (all 1.6e9 tried on the card; the one
+// exception there is a rho whose mantissa is all ones).  False for the other
+// x, 0, infinity and NaN among them: they take sqrt_inv_any.
+__device__ inline bool sqrt_inv(float x, float& rho, float& inv) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float g = x * y;
+  rho = __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+  const float e = __builtin_fmaf(-rho, y, 1.0f);
+  inv = __builtin_fmaf(e, y, y);
+  return x >= 0x1p-96f && x < 0x1p96f && e != 0x1p-24f;
+}
+
+__device__ inline void sqrt_inv_any(float x, float& rho, float& inv) {
+  rho = sqrtf(x);
+  inv = 1.0f / rho;
+}
+
+// Of N points x (relative to the frame centre): w, the part of the offset to
+// the model's axis point orthogonal to the axis, h along it, rho = |w| and
+// 1 / rho.  Together, so that their chains overlap.
+template <int N>
+__device__ inline void refit_dist(const RefitState& S, const float (&x)[N][3], float (&w)[N][3],
+                                  float (&h)[N], float (&rho)[N], float (&inv)[N]) {
+  float ww[N];
+  bool ok = true;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const float q0 = x[k][0] - S.cf[0], q1 = x[k][1] - S.cf[1], q2 = x[k][2] - S.cf[2];
+    h[k] = __builtin_fmaf(q2, S.af[2], __builtin_fmaf(q1, S.af[1], q0 * S.af[0]));
+    w[k][0] = __builtin_fmaf(-h[k], S.af[0], q0);
+    w[k][1] = __builtin_fmaf(-h[k], S.af[1], q1);
+    w[k][2] = __builtin_fmaf(-h[k], S.af[2], q2);
+    ww[k] = __builtin_fmaf(w[k][2], w[k][2], __builtin_fmaf(w[k][1], w[k][1], w[k][0] * w[k][0]));
+    ok &= sqrt_inv(ww[k], rho[k], inv[k]);
+  }
+  if (!ok) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) sqrt_inv_any(ww[k], rho[k], inv[k]);
+  }
+}
+
+// Adds an inlier's Jacobian terms (15 of J J^T, 5 of J d) to g.
+__device__ inline void refit_add(const RefitState& S, const float (&w)[3], float hh, float inv,
+                                 float d, float (&g)[kRefitTerms]) {
+  const float n1 =
+      __builtin_fmaf(w[2], S.e1f[2], __builtin_fmaf(w[1], S.e1f[1], w[0] * S.e1f[0])) * inv;
+  const float n2 =
+      __builtin_fmaf(w[2], S.e2f[2], __builtin_fmaf(w[1], S.e2f[1], w[0] * S.e2f[0])) * inv;
+  const float J[5] = {-hh * n1, -hh * n2, -n1, -n2, -1.0f};
+  int t = 0;
+#pragma unroll
+  for (int a = 0; a < 5; ++a)
+#pragma unroll
+    for (int b = a; b < 5; ++b) {
+      g[t] = __builtin_fmaf(J[a], J[b], g[t]);
+      ++t;
+    }
+#pragma unroll
+  for (int a = 0; a < 5; ++a) g[15 + a] = __builtin_fmaf(J[a], d, g[15 + a]);
 }
 
 __device__ inline void write_invalid(double* out, double k) {
@@ -589,51 +652,29 @@ __device__ inline void write_invalid(double* out, double k) {
   out[7] = k;
 }
 
-// Cholesky solve of a symmetric positive definite N x N system, fully
-// unrolled so that every index is static (no private memory).
-template <int N>
-__device__ inline bool cholesky_solve(const double (&A)[N][N], const double (&b)[N],
-                                      double (&x)[N]) {
-  double L[N][N];
-  bool ok = true;
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    double s = A[j][j];
-#pragma unroll
-    for (int k = 0; k < j; ++k) s = s - L[j][k] * L[j][k];
-    ok = ok && (s > 0.0);
-    const double d = sqrt(s);
-    L[j][j] = d;
-#pragma unroll
-    for (int i = j + 1; i < N; ++i) {
-      double t = A[i][j];
-#pragma unroll
-      for (int k = 0; k < j; ++k) t = t - L[i][k] * L[j][k];
-      L[i][j] = t / d;
-    }
-  }
-  double y[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    double t = b[i];
-#pragma unroll
-    for (int k = 0; k < i; ++k) t = t - L[i][k] * y[k];
-    y[i] = t / L[i][i];
-  }
-#pragma unroll
-  for (int i = N - 1; i >= 0; --i) {
-    double t = y[i];
-#pragma unroll
-    for (int k = i + 1; k < N; ++k) t = t - L[k][i] * x[k];
-    x[i] = t / L[i][i];
-  }
-  return ok;
-}
-
 // Refit chunk ck = {cluster, first point (cluster-relative), points, chunk
 // index within the cluster}; cluster record cl = {first chunk id, chunks,
 // first membership word, 0}.  Membership words: two per 64 points of the
-// cluster, written by the wave that owns those 64 points.
+// cluster, written by the wave that owns those 64 points (the team form: a
+// byte per thread and chunk).
+
+// First membership word of cluster c, `start` points into the batch: 64 words
+// per chunk, at most (start / kRefitChunk + c) chunks before it.
+__host__ __device__ inline size_t member_word(int64_t start, int c) {
+  return (size_t)(kRefitChunk / 32) * (size_t)(start / kRefitChunk + c);
+}
+
+// Ors a wave's 64 bits b into the mask from bit `first` on: a lane for each of
+// the (up to three) words, which other waves and clusters share.
+__device__ inline void or_mask(uint32_t* __restrict__ mask, int first, uint64_t b) {
+  const int lane = threadIdx.x & 63;
+  if (b == 0 || lane >= 3) return;
+  const uint32_t sh = (uint32_t)first & 31u;
+  const uint32_t word = lane == 0   ? (uint32_t)b << sh
+                        : lane == 1 ? (uint32_t)((b << sh) >> 32)
+                                    : (sh ? (uint32_t)(b >> (64u - sh)) : 0u);
+  if (word) atomicOr(mask + (first >> 5) + lane, word);
+}
 
 // Round 0: best hypothesis, global mask bits, membership bits, initial model.
 // A flagged cluster (alt_flags) takes its hypotheses from the alternate set
@@ -646,13 +687,12 @@ __global__ __launch_bounds__(kRefitBlock) void cyl_refit_init_kernel(
     float max_radius, uint32_t k0, uint32_t k1, uint32_t tag, int refit_rounds, int refit_iters,
     const float* __restrict__ prop, const int32_t* __restrict__ active,
     const int32_t* __restrict__ alt_flags, const int32_t* __restrict__ alt_counts, int alt_n_hyp,
-    uint32_t alt_tag, int alt_rounds, int alt_iters, const int32_t* __restrict__ bcnt,
-    RefitState* __restrict__ state, uint32_t* __restrict__ member, uint32_t* __restrict__ mask,
+    uint32_t alt_tag, int alt_rounds, int alt_iters, RefitState* __restrict__ state,
+    uint32_t* __restrict__ member, uint32_t* __restrict__ mask,
     int32_t* __restrict__ best_out, double* __restrict__ model) {
   constexpr int W = kRefitBlock / 64;
   __shared__ long long redk[W];
   __shared__ HypOut best_h;
-  if (bcnt && (int)blockIdx.x >= bcnt[2]) return;  // past the batch's chunks
   const int4 ck = rchunks[blockIdx.x];
   const int c = ck.x;
   if (c < 0) return;  // padding of the per-XCD interleave
@@ -705,47 +745,31 @@ __global__ __launch_bounds__(kRefitBlock) void cyl_refit_init_kernel(
   __syncthreads();
   const HypOut h = best_h;
 
-  // membership bits of the chunk (cluster-relative, 64-aligned per wave)
+  // membership bits of the chunk (cluster-relative, 64-aligned per wave) and
+  // the global mask's
   const int4 cl = rclus[c];
   uint32_t* mem = member + cl.z;
   const int end = ck.y + ck.z;
+  float px[kRefitPerThread][3];
+#pragma unroll
+  for (int j = 0; j < kRefitPerThread; ++j) {
+    const int i = ck.y + kRefitBlock * j + (int)threadIdx.x;
+    const float* q = P + 3 * (size_t)min(i, end - 1);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) px[j][k] = q[k];
+  }
 #pragma unroll
   for (int j = 0; j < kRefitPerThread; ++j) {
     const int gbase = ck.y + kRefitBlock * j + 64 * wave;  // first point of this wave's group
-    const int i = gbase + lane;
-    bool in = false;
-    if (i < end) {
-      const float* q = P + 3 * (size_t)i;
-      float u, v, s;
-      local_uvs(f, q[0], q[1], q[2], &u, &v, &s);
-      in = is_inlier(u, v, s, h);
-    }
-    const uint64_t b = __builtin_amdgcn_ballot_w64(in);
+    float u, v, s;
+    local_uvs(f, px[j][0], px[j][1], px[j][2], &u, &v, &s);
+    const uint64_t b =
+        __builtin_amdgcn_ballot_w64(gbase + lane < end && is_inlier(u, v, s, h));
     if (lane == 0 && gbase < end) {
       mem[gbase >> 5] = (uint32_t)b;
       mem[(gbase >> 5) + 1] = (uint32_t)(b >> 32);
     }
-  }
-  if (mask) {
-    // global mask: 64-aligned global indices, so that each wave owns two whole
-    // 32-bit words (or-ed atomically: neighbouring chunks share boundary words)
-    const int gs = off + ck.y, ge = off + end;
-    for (int gb = (gs & ~63); gb < ge; gb += kRefitBlock) {
-      const int g = gb + (int)threadIdx.x;
-      bool in = false;
-      if (g >= gs && g < ge) {
-        const float* q = xyz + 3 * (size_t)g;
-        float u, v, s;
-        local_uvs(f, q[0], q[1], q[2], &u, &v, &s);
-        in = is_inlier(u, v, s, h);
-      }
-      const uint64_t b = __builtin_amdgcn_ballot_w64(in);
-      if (lane == 0 && b) {
-        const int w0 = (gb + wave * 64) >> 5;
-        if ((uint32_t)b) atomicOr(mask + w0, (uint32_t)b);
-        if ((uint32_t)(b >> 32)) atomicOr(mask + w0 + 1, (uint32_t)(b >> 32));
-      }
-    }
+    if (mask) or_mask(mask, off + gbase, b);
   }
   if (ck.w != 0 || threadIdx.x != 0) return;
   // the cluster's first chunk: initial model (the inlier count of the best
@@ -797,45 +821,37 @@ __device__ inline void refit_step_chunk(const float* __restrict__ P, const CylFr
       px[j][0] = q[0];
       px[j][1] = q[1];
       px[j][2] = q[2];
+    } else {
+      px[j][0] = px[j][1] = px[j][2] = 0.0f;
     }
   }
-#pragma unroll 2
-  for (int j = 0; j < kRefitPerThread; ++j) {
-    const int gbase = first + kRefitBlock * j + 64 * wave;
-    const int i = gbase + lane;
-    bool in = false;
-    float d = 0.f, hh = 0.f, rho = 0.f, w[3] = {0.f, 0.f, 0.f};
-    if (i < end) {
-      const float x[3] = {px[j][0] - f.m[0], px[j][1] - f.m[1], px[j][2] - f.m[2]};
-      d = refit_dist(S, x, w, hh, rho);
-      in = reselect ? (d < thr && d > -thr) : ((mem[i >> 5] >> (i & 31)) & 1u) != 0u;
-    }
-    if (reselect) {
-      const uint64_t b = __builtin_amdgcn_ballot_w64(in);
-      if (lane == 0 && gbase < end) {
-        mem[gbase >> 5] = (uint32_t)b;
-        mem[(gbase >> 5) + 1] = (uint32_t)(b >> 32);
+#pragma unroll
+  for (int j = 0; j < kRefitPerThread; j += 2) {
+    __builtin_amdgcn_sched_barrier(0);  // a pair at a time (registers)
+    float x[2][3], hh[2], rho[2], inv[2], w[2][3];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) x[e][k] = px[j + e][k] - f.m[k];
+    refit_dist<2>(S, x, w, hh, rho, inv);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int gbase = first + kRefitBlock * (j + e) + 64 * wave;
+      const int i = gbase + lane;
+      const float d = rho[e] - S.rf;
+      bool in = false;
+      if (i < end)
+        in = reselect ? (d < thr && d > -thr) : ((mem[i >> 5] >> (i & 31)) & 1u) != 0u;
+      if (reselect) {
+        const uint64_t b = __builtin_amdgcn_ballot_w64(in);
+        if (lane == 0 && gbase < end) {
+          mem[gbase >> 5] = (uint32_t)b;
+          mem[(gbase >> 5) + 1] = (uint32_t)(b >> 32);
+        }
       }
-    }
-    if (in) {
-      ++cnt;
-      if (rho > 0.0f) {
-        const float inv = 1.0f / rho;
-        const float n1 =
-            __builtin_fmaf(w[2], S.e1f[2], __builtin_fmaf(w[1], S.e1f[1], w[0] * S.e1f[0])) * inv;
-        const float n2 =
-            __builtin_fmaf(w[2], S.e2f[2], __builtin_fmaf(w[1], S.e2f[1], w[0] * S.e2f[0])) * inv;
-        const float J[5] = {-hh * n1, -hh * n2, -n1, -n2, -1.0f};
-        int t = 0;
-#pragma unroll
-        for (int a = 0; a < 5; ++a)
-#pragma unroll
-          for (int b = a; b < 5; ++b) {
-            g[t] = __builtin_fmaf(J[a], J[b], g[t]);
-            ++t;
-          }
-#pragma unroll
-        for (int a = 0; a < 5; ++a) g[15 + a] = __builtin_fmaf(J[a], d, g[15 + a]);
+      if (in) {
+        ++cnt;
+        if (rho[e] > 0.0f) refit_add(S, w[e], hh[e], inv[e], d, g);
       }
     }
   }
@@ -852,52 +868,6 @@ __device__ inline double refit_term(const Comp2* __restrict__ partial, int nck, 
   return (double)t.s + (double)t.e;
 }
 
-// The Gauss-Newton step's solve of one cluster (one thread) from its summed
-// terms gs and inlier count: the FP64 5x5 normal equations, the next model in
-// S.  Too few inliers stop the cluster; a failed factorisation skips the
-// rest of the round.
-__device__ inline void refit_solve_terms(RefitState& S, const double (&gs)[kRefitTerms],
-                                         int tot_cnt, int round) {
-  if (tot_cnt < 5) {
-    S.status = kRefitStopped;
-    return;
-  }
-  double A[5][5], rhs[5], dl[5];
-  {
-    int t = 0;
-#pragma unroll
-    for (int a = 0; a < 5; ++a)
-#pragma unroll
-      for (int bb = a; bb < 5; ++bb) {
-        A[a][bb] = gs[t];
-        A[bb][a] = gs[t];
-        ++t;
-      }
-#pragma unroll
-    for (int a = 0; a < 5; ++a) rhs[a] = -gs[15 + a];
-  }
-  if (!cholesky_solve<5>(A, rhs, dl)) {
-    S.skip_round = round;
-    return;
-  }
-  double e1[3], e2[3];
-  sl_basis(S.a, e1, e2);
-  double na[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) na[i] = S.a[i] + dl[0] * e1[i] + dl[1] * e2[i];
-  const double nl = sqrt(na[0] * na[0] + na[1] * na[1] + na[2] * na[2]);
-  RefitState N = S;
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    N.a[i] = na[i] / nl;
-    N.c[i] = S.c[i] + dl[2] * e1[i] + dl[3] * e2[i];
-  }
-  N.r = S.r + dl[4];
-  if (!(N.r > 0.0)) N.status = kRefitStopped;
-  refit_model_f32(N);
-  S = N;
-}
-
 // Sum of one int per lane over a wave (every lane gets it).
 __device__ inline int wave_sum_int(int v) {
 #pragma unroll
@@ -905,19 +875,81 @@ __device__ inline int wave_sum_int(int v) {
   return v;
 }
 
-// The solve by one wave: lane q < kRefitTerms sums term q over the chunks
-// (the loads of all terms in flight at once), lane 0 solves; S is lane 0's.
-__device__ inline void refit_solve_wave(RefitState& S, const Comp2* __restrict__ partial,
-                                        const int32_t* __restrict__ pcount, int nck, int round) {
+// d of lane `from` (uniform), as a scalar on every lane
+__device__ inline double lane_value(double d, int from) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(d), from);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(d), from);
+  return __hiloint2double(hi, lo);
+}
+
+// The Gauss-Newton step's solve of one cluster by one wave: lane q <
+// kRefitTerms sums term q over the chunks, then the FP64 5x5 normal equations
+// and the next model (lane 0 writes S).  Too few inliers stop the cluster; a
+// failed factorisation skips the rest of the round.  The operations and their
+// order are a scalar Cholesky's, with a row of the factor per lane (the right
+// side is row 5, so the forward substitution is part of it): a column's
+// divisions run at once, where one lane made the 25 divisions and roots of
+// the step one after the other.
+__device__ inline void refit_solve_wave(RefitState& S, const Comp2* part, const int32_t* pc, int nck,
+                                        int round) {
   const int lane = threadIdx.x & 63;
-  const double mine = lane < kRefitTerms ? refit_term(partial, nck, lane) : 0.0;
+  const double mine = lane < kRefitTerms ? refit_term(part, nck, lane) : 0.0;
   int cnt = 0;
-  for (int k = lane; k < nck; k += 64) cnt += pcount[k];
-  cnt = wave_sum_int(cnt);
-  double gs[kRefitTerms];
+  if (nck <= 4) {
+    for (int k = 0; k < nck; ++k) cnt += pc[k];
+  } else {
+    for (int k = lane; k < nck; k += 64) cnt += pc[k];
+    cnt = wave_sum_int(cnt);
+  }
+  if (cnt < 5) {
+    if (lane == 0) S.status = kRefitStopped;
+    return;
+  }
+  const int r = min(lane, 5);
+  double t, Lr[5], row[5], diag[5];
 #pragma unroll
-  for (int q = 0; q < kRefitTerms; ++q) gs[q] = __shfl(mine, q, 64);
-  if (lane == 0) refit_solve_terms(S, gs, cnt, round);
+  for (int c = 0; c < 5; ++c) {
+    const int lo = min(r, c), hi = max(r, c);
+    const double v = __shfl(mine, r == 5 ? 15 + c : lo * 5 - lo * (lo - 1) / 2 + (hi - lo), 64);
+    row[c] = r == 5 ? -v : v;
+  }
+  bool ok = true;
+#pragma unroll
+  for (int j = 0; j < 5; ++j) {
+    t = row[j];
+#pragma unroll
+    for (int k = 0; k < j; ++k) t = t - Lr[k] * lane_value(Lr[k], j);
+    const double s = lane_value(t, j);
+    ok = ok && (s > 0.0);
+    diag[j] = sqrt(s);
+    Lr[j] = t / diag[j];
+  }
+  if (!ok) {
+    if (lane == 0) S.skip_round = round;
+    return;
+  }
+  double x[5];
+#pragma unroll
+  for (int i = 4; i >= 0; --i) {
+    double u = lane_value(Lr[i], 5);
+#pragma unroll
+    for (int k = i + 1; k < 5; ++k) u = u - lane_value(Lr[i], k) * x[k];
+    x[i] = u / diag[i];
+  }
+  RefitState N = S;
+  double na[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) na[i] = N.a[i] + x[0] * N.e1[i] + x[1] * N.e2[i];
+  const double nl = sqrt(na[0] * na[0] + na[1] * na[1] + na[2] * na[2]);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    N.a[i] = na[i] / nl;
+    N.c[i] = N.c[i] + x[2] * N.e1[i] + x[3] * N.e2[i];
+  }
+  N.r = N.r + x[4];
+  if (!(N.r > 0.0)) N.status = kRefitStopped;
+  refit_model_f32(N);
+  if (lane == 0) S = N;
 }
 
 // The final pass over the chunk [first, end): the chunk sums of the final
@@ -945,13 +977,14 @@ __device__ inline void refit_final_chunk(const float* __restrict__ P, const CylF
     for (int j = 0; j < kRefitPerThread; ++j) {
       const int i = first + kRefitBlock * j + (int)threadIdx.x;
       if (i < end) {
-        const float x[3] = {px[j][0] - f.m[0], px[j][1] - f.m[1], px[j][2] - f.m[2]};
-        float w[3], hh, rho;
-        const float d = refit_dist(S, x, w, hh, rho);
+        const float x[1][3] = {{px[j][0] - f.m[0], px[j][1] - f.m[1], px[j][2] - f.m[2]}};
+        float w[1][3], hh[1], rho[1], inv[1];
+        refit_dist<1>(S, x, w, hh, rho, inv);
+        const float d = rho[0] - S.rf;
         if (d < thr && d > -thr) {
-          g[0] = g[0] + x[0];
-          g[1] = g[1] + x[1];
-          g[2] = g[2] + x[2];
+          g[0] = g[0] + x[0][0];
+          g[1] = g[1] + x[0][1];
+          g[2] = g[2] + x[0][2];
           ++cnt;
         }
       }
@@ -1004,10 +1037,9 @@ __global__ __launch_bounds__(kRefitBlock) void cyl_refit_step_kernel(
     const CylFrame* __restrict__ frames, const int4* __restrict__ rchunks,
     const int4* __restrict__ rclus, const RefitState* __restrict__ state,
     uint32_t* __restrict__ member, Comp2* __restrict__ partial, int32_t* __restrict__ pcount,
-    int step, float thr, const int32_t* __restrict__ bcnt) {
+    int step, float thr) {
   __shared__ RefitRed<kRefitTerms> red;
   __shared__ int cnt_w[kRefitBlock / 64];
-  if (bcnt && (int)blockIdx.x >= bcnt[2]) return;
   const int4 ck = rchunks[blockIdx.x];
   const int c = ck.x;
   if (c < 0) return;
@@ -1026,11 +1058,12 @@ __global__ __launch_bounds__(kRefitBlock) void cyl_refit_step_kernel(
 // The Gauss-Newton step's solve after the step's chunk partials, one wave
 // per cluster (kRefitWaveClusters per workgroup).
 __global__ __launch_bounds__(64 * kRefitWaveClusters) void cyl_refit_solve_kernel(
-    int n_clusters, const int4* __restrict__ rclus, RefitState* __restrict__ state,
-    const Comp2* __restrict__ partial, const int32_t* __restrict__ pcount, int step,
-    const int32_t* __restrict__ bcnt) {
-  const int c = blockIdx.x * kRefitWaveClusters + (int)(threadIdx.x >> 6);
-  if (c >= n_clusters || (bcnt && c >= bcnt[0])) return;
+    int n_big, const int4* __restrict__ big, const int4* __restrict__ rclus,
+    RefitState* __restrict__ state, const Comp2* __restrict__ partial,
+    const int32_t* __restrict__ pcount, int step) {
+  const int b = blockIdx.x * kRefitWaveClusters + (int)(threadIdx.x >> 6);
+  if (b >= n_big) return;
+  const int c = big[b].x;
   RefitState S = state[c];
   if (S.status != kRefitActive) return;
   if (step >= S.rounds * S.iters) return;
@@ -1046,11 +1079,9 @@ __global__ __launch_bounds__(kRefitBlock) void cyl_refit_final_kernel(
     const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
     const CylFrame* __restrict__ frames, const int4* __restrict__ rchunks,
     const int4* __restrict__ rclus, const RefitState* __restrict__ state,
-    Comp2* __restrict__ partial, int32_t* __restrict__ pcount, float thr,
-    const int32_t* __restrict__ bcnt) {
+    Comp2* __restrict__ partial, int32_t* __restrict__ pcount, float thr) {
   __shared__ RefitRed<3> red;
   __shared__ int cnt_w[kRefitBlock / 64];
-  if (bcnt && (int)blockIdx.x >= bcnt[2]) return;
   const int4 ck = rchunks[blockIdx.x];
   const int c = ck.x;
   if (c < 0) return;
@@ -1065,12 +1096,13 @@ __global__ __launch_bounds__(kRefitBlock) void cyl_refit_final_kernel(
 // The output record of each cluster from the final pass's chunk partials,
 // one wave per cluster (kRefitWaveClusters per workgroup).
 __global__ __launch_bounds__(64 * kRefitWaveClusters) void cyl_refit_finish_kernel(
-    int n_clusters, const CylFrame* __restrict__ frames, const int4* __restrict__ rclus,
-    const RefitState* __restrict__ state, const Comp2* __restrict__ partial,
-    const int32_t* __restrict__ pcount, const int32_t* __restrict__ bcnt,
+    int n_big, const int4* __restrict__ big, const CylFrame* __restrict__ frames,
+    const int4* __restrict__ rclus, const RefitState* __restrict__ state,
+    const Comp2* __restrict__ partial, const int32_t* __restrict__ pcount,
     double* __restrict__ model) {
-  const int c = blockIdx.x * kRefitWaveClusters + (int)(threadIdx.x >> 6);
-  if (c >= n_clusters || (bcnt && c >= bcnt[0])) return;
+  const int b = blockIdx.x * kRefitWaveClusters + (int)(threadIdx.x >> 6);
+  if (b >= n_big) return;
+  const int c = big[b].x;
   const RefitState S = state[c];
   if (S.status == kRefitInvalid || S.status == kRefitInactive) return;
   const int4 cl = rclus[c];
@@ -1078,65 +1110,394 @@ __global__ __launch_bounds__(64 * kRefitWaveClusters) void cyl_refit_finish_kern
                     model + (size_t)c * SLOAM_CYL_MODEL_STRIDE);
 }
 
-// Every Gauss-Newton step, the final pass and the output record of one
-// cluster in one workgroup: the workgroup of the cluster's first refit chunk
-// (the others exit) walks the cluster's chunks in order at every step, keeps
-// the chunk partials and counts in LDS and solves on its first thread
-// between steps.  Every sum is the same function over the same chunk as in
-// the launch-per-step sequence, so the records carry the same bits, without
-// its launches and per-cluster solve kernels.  Clusters of up to
-// kRefitFusedChunks chunks (every plan's bound).
-__global__ __launch_bounds__(kRefitBlock) void cyl_refit_fused_kernel(
-    const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
-    const CylFrame* __restrict__ frames, const int4* __restrict__ rchunks,
-    const int4* __restrict__ rclus, RefitState* __restrict__ state, uint32_t* __restrict__ member,
-    float thr, const int32_t* __restrict__ bcnt, double* __restrict__ model) {
-  __shared__ RefitRed<kRefitTerms> red;
-  __shared__ RefitRed<3> red3;
-  __shared__ int cnt_w[kRefitBlock / 64];
-  __shared__ Comp2 part[kRefitFusedChunks * kRefitTerms];
-  __shared__ int32_t pc[kRefitFusedChunks];
-  __shared__ RefitState s_next;
-  if (bcnt && (int)blockIdx.x >= bcnt[2]) return;
-  const int4 ck = rchunks[blockIdx.x];
-  const int c = ck.x;
-  if (c < 0 || ck.w != 0) return;  // one workgroup per cluster
-  RefitState S = state[c];
-  if (S.status == kRefitInvalid || S.status == kRefitInactive) return;
-  const int4 cl = rclus[c];
-  if (cl.y > kRefitFusedChunks) return;  // excluded by the plans' cluster bound
+// ---------------------------------------------------------------------------
+// The whole refit of one cluster by one team of NT threads (a wave or a
+// workgroup): best hypothesis, mask, every Gauss-Newton step, final pass and
+// output record.  The sums are the per-step form's, value for value: a team
+// of 64 plays the 256 threads of a chunk in four turns (virtual thread
+// 64 b + lane), sums with no points in them are skipped (TwoSum with zero
+// changes nothing), and the 5x5 solve is the same operations with a row per
+// lane.
+// ---------------------------------------------------------------------------
+// a wave takes clusters of up to this many points (up to 256 only: 3000
+// clusters of 40..700 points take 166 us for 149, up to 128: 178)
+constexpr int kWaveRefit = 512;
+
+template <int NT>
+struct TeamLds {
+  // rows of 36: a chain reads four values at a time, 16 chains distinct banks
+  alignas(16) float v[kRefitTerms][NT / kRefitGroup][kRefitGroup + 4];
+  Comp2 grp[kRefitTerms][kRefitGroups];
+  Comp2 part[(NT == kRefitBlock ? kRefitMaxChunks : 1) * kRefitTerms];
+  int pc[NT == kRefitBlock ? kRefitMaxChunks : 1];
+  RefitState S;
+  HypOut best;
+  long long redk[NT / 64];
+  int cnt[NT / 64];
+};
+
+// Orders LDS traffic within a team.
+template <int NT>
+__device__ inline void team_sync() {
+  if constexpr (NT == 64) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
+// The team's points of the chunk [first, end), relative to the frame centre m:
+// px[NVB * J] (turn b, point j of virtual
+// thread NT b + t at index b J + j).
+template <int NT>
+__device__ inline void team_load(const float* __restrict__ P, const float (&m)[3], int first,
+                                 int end, float (&px)[kRefitPerThread][3]) {
+  constexpr int NVB = kRefitBlock / NT, J = kRefitPerThread / NVB;
+  const int t = NT == 64 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+#pragma unroll
+  for (int b = 0; b < NVB; ++b)
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int i = first + kRefitBlock * j + NT * b + t;
+      if (i < end) {
+        const float* q = P + 3 * (size_t)i;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) px[b * J + j][k] = q[k] - m[k];
+      } else {
+        px[b * J + j][0] = px[b * J + j][1] = px[b * J + j][2] = 0.0f;
+      }
+    }
+}
+
+// TwoSum chains over the LDS values of turn b (NT threads' worth of groups).
+template <int NT, int K>
+__device__ inline void team_chains(TeamLds<NT>& L, int b, int used) {
+  constexpr int G = NT / kRefitGroup;  // groups of this turn
+  const int t = NT == 64 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+  if (t < K * G) {
+    const int k = t / G, q = t % G;
+    Comp2 s = {0.0f, 0.0f};
+    if ((NT * b + kRefitGroup * q) < used) {
+      const float4* row = reinterpret_cast<const float4*>(L.v[k][q]);
+#pragma unroll
+      for (int j = 0; j < kRefitGroup / 4; ++j) {
+        const float4 x = row[j];
+        comp_add(s, x.x);
+        comp_add(s, x.y);
+        comp_add(s, x.z);
+        comp_add(s, x.w);
+      }
+    }
+    L.grp[k][G * b + q] = s;
+  }
+}
+
+// Chunk partials from the group sums; count = inliers of this wave.
+template <int NT, int K>
+__device__ inline void team_close(TeamLds<NT>& L, int ck, int count) {
+  const int t = NT == 64 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+  if constexpr (NT != 64)
+    if ((t & 63) == 0) L.cnt[t >> 6] = count;
+  team_sync<NT>();
+  if (t < K) {
+    Comp2 s = {0.0f, 0.0f};
+#pragma unroll
+    for (int q = 0; q < kRefitGroups; ++q) comp_add(s, L.grp[t][q]);
+    L.part[ck * kRefitTerms + t] = s;
+  }
+  if (t == 0) {
+    if constexpr (NT != 64) {
+      count = 0;
+#pragma unroll
+      for (int w = 0; w < NT / 64; ++w) count += L.cnt[w];
+    }
+    L.pc[ck] = count;
+  }
+}
+
+template <int NT>
+__device__ inline void refit_team(const float* __restrict__ xyz, int off, int n, int c,
+                                  const CylFrame& f, const int32_t* __restrict__ cnts, int nh,
+                                  uint32_t tag, const float* pc_prop, int rounds, int iters,
+                                  float thr, float max_radius, uint32_t k0, uint32_t k1,
+                                  uint8_t* mem, uint32_t* __restrict__ mask,
+                                  int32_t* __restrict__ best_out, double* __restrict__ out,
+                                  TeamLds<NT>& L) {
+  constexpr int NVB = kRefitBlock / NT, J = kRefitPerThread / NVB, G = J < 4 ? J : 4;
+  const int t = NT == 64 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+  const int lane = t & 63, wave = t >> 6;
+  const float* P = xyz + 3 * (size_t)off;
+  const int nck = NT == 64 ? 1 : max(1, (n + kRefitChunk - 1) / kRefitChunk);
+  if (nck > (NT == 64 ? 1 : kRefitMaxChunks)) return;  // excluded by the plans' cluster bound
+  float px[kRefitPerThread][3];
+  if (nck == 1) team_load<NT>(P, f.m, 0, n, px);
+
+  // best hypothesis: key = count * 2^32 + (2^32 - 1 - index), max wins
+  long long key = -1;
+  for (int h = t; h < nh; h += NT) {
+    const long long kk =
+        ((long long)cnts[h] << 32) | (long long)(0xFFFFFFFFu - (uint32_t)h);
+    key = kk > key ? kk : key;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const long long other = __shfl_xor(key, o, 64);
+    key = other > key ? other : key;
+  }
+  if constexpr (NT != 64) {
+    if (lane == 0) L.redk[wave] = key;
+    __syncthreads();
+    key = L.redk[0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) key = L.redk[w] > key ? L.redk[w] : key;
+  }
+  const int best = (n >= 3 && nh > 0) ? (int)(0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFll)) : -1;
+  if (wave == 0) {
+    // every lane of the wave makes the same hypothesis and model
+    HypOut h;
+    if (best >= 0) {
+      int32_t idx[3];
+      h = hyp_for(P, n, c, best, f, thr, max_radius, k0, k1, tag, idx, pc_prop);
+    } else {
+      h.valid = 0;
+      h.A = h.B = 0.f;
+      h.L = INFINITY;
+      h.U = -INFINITY;
+      h.cu = h.cv = h.r = 0.f;
+    }
+    // the inlier count of the best hypothesis is its score
+    const int kin = best >= 0 ? cnts[best] : 0;
+    RefitState S;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      S.a[i] = f.axis[i];
+      S.c[i] = (double)h.cu * (double)f.e1[i] + (double)h.cv * (double)f.e2[i];
+    }
+    S.r = (double)h.r;
+    S.status = kRefitActive;
+    S.skip_round = -1;
+    if (kin < 3 || !h.valid) {
+      S.status = kRefitInvalid;
+      if (lane == 0) write_invalid(out, (double)kin);
+    }
+    refit_model_f32(S);
+    if (lane == 0) {
+      L.best = h;
+      L.S = S;
+      if (best_out) *best_out = best;
+    }
+  }
+  // group sums of turns without points stay zero
+  for (int q = t; q < kRefitTerms * kRefitGroups; q += NT)
+    L.grp[q / kRefitGroups][q % kRefitGroups] = Comp2{0.0f, 0.0f};
+  team_sync<NT>();
+  const HypOut h = L.best;
+
+  // round-0 membership: the inliers of the best hypothesis.  bit b J + j of a
+  // thread's byte of a chunk; mem holds the bytes of a cluster of several
+  uint32_t bits = 0;
+#pragma unroll 1
+  for (int ck = 0; ck < nck; ++ck) {
+    const int first = ck * kRefitChunk, end = min(n, first + kRefitChunk);
+    if (nck > 1) team_load<NT>(P, f.m, first, end, px);
+    bits = 0;
+#pragma unroll
+    for (int v = 0; v < kRefitPerThread; ++v) {
+      const int i = first + kRefitBlock * (v % J) + NT * (v / J) + t;
+      float uu, vv, ss;
+      rel_uvs(f, px[v], &uu, &vv, &ss);
+      const bool in = i < end && is_inlier(uu, vv, ss, h);
+      bits |= in ? 1u << v : 0u;
+      if (mask) or_mask(mask, off + i - lane, __builtin_amdgcn_ballot_w64(in));
+    }
+    if (nck > 1) mem[ck * kRefitBlock + t] = (uint8_t)bits;
+  }
+  if (L.S.status == kRefitInvalid) return;
+
+  // the FP32 model, uniform over the team
+  RefitState M;
+  auto fetch = [&]() {
+    auto uni = [](float v) {
+      return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+    };
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      M.af[i] = uni(L.S.af[i]);
+      M.cf[i] = uni(L.S.cf[i]);
+      M.e1f[i] = uni(L.S.e1f[i]);
+      M.e2f[i] = uni(L.S.e2f[i]);
+    }
+    M.rf = uni(L.S.rf);
+  };
+  const int steps = rounds * iters;
+  for (int step = 0; step < steps && L.S.status == kRefitActive; ++step) {
+    const int round = step / iters, it = step % iters;
+    if (L.S.skip_round == round) continue;
+    fetch();
+    const bool reselect = round > 0 && it == 0;
+    for (int ck = 0; ck < nck; ++ck) {
+      const int first = ck * kRefitChunk, end = min(n, first + kRefitChunk);
+      if (nck > 1) team_load<NT>(P, f.m, first, end, px);
+      if (nck > 1) bits = mem[ck * kRefitBlock + t];
+      int count = 0;
+#pragma unroll
+      for (int b = 0; b < NVB; ++b) {
+        if (first + NT * b >= end) break;
+        float g[kRefitTerms];
+#pragma unroll
+        for (int q = 0; q < kRefitTerms; ++q) g[q] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < J; j += G) {
+          // G points at a time: more of them in flight take too many registers
+          __builtin_amdgcn_sched_barrier(0);
+          const int i = first + kRefitBlock * j + NT * b + t, v = b * J + j;
+          if (i - t >= end) break;  // no point of the team's turn
+          float x[G][3], hh[G], rho[G], inv[G], w[G][3], d[G];
+#pragma unroll
+          for (int e = 0; e < G; ++e)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) x[e][k] = px[v + e][k];
+          refit_dist<G>(M, x, w, hh, rho, inv);
+#pragma unroll
+          for (int e = 0; e < G; ++e) d[e] = rho[e] - M.rf;
+          if (reselect) {
+#pragma unroll
+            for (int e = 0; e < G; ++e) {
+              const bool in = i + kRefitBlock * e < end && d[e] < thr && d[e] > -thr;
+              bits = (bits & ~(1u << (v + e))) | (in ? 1u << (v + e) : 0u);
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < G; ++e) {
+            const bool in = ((bits >> (v + e)) & 1u) != 0u;
+            count += __popcll(__builtin_amdgcn_ballot_w64(in));
+            if (in && rho[e] > 0.0f) refit_add(M, w[e], hh[e], inv[e], d[e], g);
+          }
+        }
+        const int tg = t / kRefitGroup, tl = t % kRefitGroup;
+        team_sync<NT>();
+#pragma unroll
+        for (int q = 0; q < kRefitTerms; ++q) L.v[q][tg][tl] = g[q];
+        team_sync<NT>();
+        team_chains<NT, kRefitTerms>(L, b, end - first);
+      }
+      if (nck > 1 && reselect) mem[ck * kRefitBlock + t] = (uint8_t)bits;
+      team_close<NT, kRefitTerms>(L, ck, count);
+    }
+    team_sync<NT>();
+    if (wave == 0) refit_solve_wave(L.S, L.part, L.pc, nck, round);
+    team_sync<NT>();
+  }
+
+  // final inliers' centroid and the record
+  fetch();
+  const bool pos = L.S.r > 0.0;
+  for (int ck = 0; ck < nck; ++ck) {
+    const int first = ck * kRefitChunk, end = min(n, first + kRefitChunk);
+    if (nck > 1) team_load<NT>(P, f.m, first, end, px);
+    int count = 0;
+#pragma unroll
+    for (int b = 0; b < NVB; ++b) {
+      if (first + NT * b >= end) break;
+      float g[3] = {0.0f, 0.0f, 0.0f};
+      if (pos)
+#pragma unroll
+        for (int j = 0; j < J; j += G) {
+          const int i = first + kRefitBlock * j + NT * b + t, v = b * J + j;
+          if (i - t >= end) break;
+          float x[G][3], hh[G], rho[G], inv[G], w[G][3];
+#pragma unroll
+          for (int e = 0; e < G; ++e)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) x[e][k] = px[v + e][k];
+          refit_dist<G>(M, x, w, hh, rho, inv);
+#pragma unroll
+          for (int e = 0; e < G; ++e) {
+            const float d = rho[e] - M.rf;
+            const bool in = i + kRefitBlock * e < end && d < thr && d > -thr;
+            count += __popcll(__builtin_amdgcn_ballot_w64(in));
+            if (in) {
+#pragma unroll
+              for (int k = 0; k < 3; ++k) g[k] = g[k] + x[e][k];
+            }
+          }
+        }
+      const int tg = t / kRefitGroup, tl = t % kRefitGroup;
+      team_sync<NT>();
+#pragma unroll
+      for (int q = 0; q < 3; ++q) L.v[q][tg][tl] = g[q];
+      team_sync<NT>();
+      team_chains<NT, 3>(L, b, end - first);
+    }
+    team_close<NT, 3>(L, ck, count);
+  }
+  team_sync<NT>();
+  if (wave == 0) {
+    refit_finish_wave(L.S, f, L.part, L.pc, nck, out);
+  }
+}
+
+// The whole refit, one team per cluster.  teams (host plans): per workgroup
+// either one cluster {c, -2, ..} or up to four of at most kWaveRefit points
+// {c0, c1, c2, c3} (-1: none), a wave each.  Without it workgroup b takes
+// cluster b.  A flagged cluster (alt_flags) takes its hypotheses from the
+// alternate set and refits with the alternate schedule; clusters not in
+// `active` are left alone.
+//
+// Latency-bound: a step of a 2048-point cluster is 3.0k cycles of distances
+// and products, 4k of TwoSum sums, 5k of FP64 solve.  Against a launch per step
+// and one per solve: 2000 clusters of 50..5000 points 164 -> 107 us, 4096 of
+// them 213 -> 176, 12 clusters of 90..1400 points (were one launch, too)
+// 53 -> 35.  In a batch the largest cluster is what ends last (90 us for 3
+// chunks); two teams of 1024 threads a CU, or more priority for it, were no
+// faster.
+__global__ __launch_bounds__(kRefitBlock, 4) void cyl_refit_team_kernel(
+    const float* __restrict__ xyz, const int32_t* __restrict__ offsets, int n_clusters,
+    const CylFrame* __restrict__ frames, const int32_t* __restrict__ counts,
+    const int4* __restrict__ teams, int n_hyp, float thr,
+    float max_radius, uint32_t k0, uint32_t k1, uint32_t tag, int refit_rounds, int refit_iters,
+    const float* __restrict__ prop, const int32_t* __restrict__ active,
+    const int32_t* __restrict__ alt_flags, const int32_t* __restrict__ alt_counts, int alt_n_hyp,
+    uint32_t alt_tag, int alt_rounds, int alt_iters, const int32_t* __restrict__ bcnt,
+    uint32_t* __restrict__ member, uint32_t* __restrict__ mask, int32_t* __restrict__ best_out,
+    double* __restrict__ model) {
+  constexpr int kW = kRefitBlock / 64;
+  union Lds {
+    TeamLds<kRefitBlock> block;
+    TeamLds<64> wave[kW];
+    __device__ Lds() {}
+  };
+  __shared__ Lds L;
+  int c = blockIdx.x;
+  bool by_wave = false;
+  if (teams) {
+    const int4 tm = teams[blockIdx.x];
+    by_wave = tm.y != -2;
+    const int w = threadIdx.x >> 6;
+    c = !by_wave || w == 0 ? tm.x : (w == 1 ? tm.y : (w == 2 ? tm.z : tm.w));
+  }
+  c = __builtin_amdgcn_readfirstlane(c);
+  if (c < 0 || c >= n_clusters || (bcnt && c >= bcnt[0]) || (active && !active[c])) return;
   const int off = offsets[c];
   const int n = offsets[c + 1] - off;
-  const float* P = xyz + 3 * (size_t)off;
   const CylFrame f = frames[c];
-  uint32_t* mem = member + cl.z;
-  const int steps = S.rounds * S.iters;
-  for (int step = 0; step < steps && S.status == kRefitActive; ++step) {
-    const int round = step / S.iters, it = step % S.iters;
-    if (S.skip_round == round) continue;
-    for (int k = 0; k < cl.y; ++k) {
-      const int first = k * kRefitChunk;
-      refit_step_chunk(P, f, S, mem, first, first + min(kRefitChunk, n - first),
-                       round > 0 && it == 0, thr, red, cnt_w, part + k * kRefitTerms, pc + k);
-    }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-      RefitState N = S;
-      refit_solve_wave(N, part, pc, cl.y, round);
-      if (threadIdx.x == 0) s_next = N;
-    }
-    __syncthreads();
-    S = s_next;
-  }
-  for (int k = 0; k < cl.y; ++k) {
-    const int first = k * kRefitChunk;
-    refit_final_chunk(P, f, S, first, first + min(kRefitChunk, n - first), thr, red3, cnt_w,
-                      part + k * kRefitTerms, pc + k);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) state[c] = S;
-  if (threadIdx.x < 64)
-    refit_finish_wave(S, f, part, pc, cl.y, model + (size_t)c * SLOAM_CYL_MODEL_STRIDE);
+  const bool alt = alt_flags && alt_flags[c];
+  const int nh = alt ? alt_n_hyp : n_hyp;
+  const int32_t* cnts = (alt ? alt_counts : counts) + (size_t)c * nh;
+  const uint32_t tg = alt ? alt_tag : tag;
+  const float* pc = alt ? nullptr : cluster_prop(prop, c);
+  const int rounds = alt ? alt_rounds : refit_rounds, iters = alt ? alt_iters : refit_iters;
+  int32_t* bo = best_out ? best_out + c : nullptr;
+  double* out = model + (size_t)c * SLOAM_CYL_MODEL_STRIDE;
+  if (by_wave)
+    refit_team<64>(xyz, off, n, c, f, cnts, nh, tg, pc, rounds, iters, thr, max_radius, k0, k1,
+                   nullptr, mask, bo, out, L.wave[threadIdx.x >> 6]);
+  else
+    refit_team<kRefitBlock>(xyz, off, n, c, f, cnts, nh, tg, pc, rounds, iters, thr, max_radius,
+                            k0, k1,
+                            reinterpret_cast<uint8_t*>(member + member_word(off - offsets[0], c)),
+                            mask, bo, out, L.block);
 }
 
 }  // namespace
@@ -1170,13 +1531,16 @@ struct sloam_cyl_plan {
   int n_xcd = 1;
   // counted plans: the layout is made on the device at every exec from the
   // offsets and the cluster count at d_n (at most cap clusters and
-  // cap_points points); n_clusters, n_work and n_rchunks are then the grid
+  // cap_points points); n_clusters and n_work are then the grid
   // sizes, d_cnt the batch's own {clusters, work items, refit chunks,
   // overflow}
   bool counted = false;
-  // refit in one workgroup per cluster (cyl_refit_fused) instead of one
-  // launch per Gauss-Newton step
-  bool fused = true;
+  // refit: the clusters of cyl_refit_team (largest first), and the large ones
+  // (big: their number) with one launch per Gauss-Newton step, whose chunks are
+  // d_rchunks; d_big lists them, as teams too (for a few of them at a time)
+  int n_teams = 0, n_big = 0;
+  int4* d_teams = nullptr;
+  int4* d_big = nullptr;
   const int32_t* d_n = nullptr;
   int64_t cap_points = 0;
   int cpc = 0;  // work items per cluster
@@ -1195,139 +1559,101 @@ struct sloam_cyl_plan {
 
 static int round_up(int x, int m) { return (x + m - 1) / m * m; }
 
-// Launches the refit of plan p: the init pass, then either the fused refit
-// (one workgroup per cluster) or one launch per Gauss-Newton step (as many as
-// the longest schedule among the clusters) and the final pass.
+// Launches the refit of plan p: one team per cluster, and for the large
+// clusters the init pass, one launch per Gauss-Newton step (as many as the
+// longest schedule among the clusters) and the final pass.
 // alt_flags (nullable) marks the clusters that take their best hypothesis
 // from alt_counts (alt_n_hyp hypotheses of sample stream alt_tag, no
 // proposal) and refit with alt_rounds x alt_iters steps, instead of counts.
+// few: only a few clusters are active, the large ones take a team each too.
 static int launch_refit(sloam_cyl_plan* p, const float* d_xyz, const int32_t* d_offsets,
                         const int32_t* counts, const float* d_proposal, const int32_t* d_active,
                         const int32_t* alt_flags, const int32_t* alt_counts, int alt_n_hyp,
                         uint32_t alt_tag, int alt_rounds, int alt_iters, uint32_t* d_mask,
-                        int32_t* d_best, double* d_model, bool force_fused = false) {
+                        int32_t* d_best, double* d_model, bool few = false) {
   sloam_ctx* ctx = p->ctx;
   const sloam_cyl_fit_cfg& cfg = p->cfg;
-  if (p->n_rchunks == 0) return SLOAM_OK;
+  if (p->n_clusters == 0) return SLOAM_OK;
   const uint32_t k0 = (uint32_t)cfg.seed;
   const uint32_t k1 = (uint32_t)(cfg.seed >> 32);
   const uint32_t tag = (uint32_t)cfg.stream_tag;
-  const dim3 grid(p->n_rchunks), block(kRefitBlock);
+  const dim3 block(kRefitBlock);
   const int32_t* cnt = p->counted ? p->d_cnt : nullptr;
+  auto team = [&](const int4* teams, int n) -> int {
+    if (n == 0) return SLOAM_OK;
+    hipLaunchKernelGGL(cyl_refit_team_kernel, dim3(n), block, 0, ctx->stream, d_xyz, d_offsets,
+                       p->n_clusters, p->d_frames, counts, teams, cfg.n_hyp, cfg.thr,
+                       cfg.max_radius, k0, k1, tag, cfg.refit_rounds, cfg.refit_iters, d_proposal,
+                       d_active, alt_flags, alt_counts, alt_n_hyp, alt_tag, alt_rounds, alt_iters,
+                       cnt, p->d_member, d_mask, d_best, d_model);
+    SLOAM_HIP(ctx, hipGetLastError());
+    return SLOAM_OK;
+  };
+  if (p->counted) return team(nullptr, p->n_clusters);
+  int st = team(p->d_teams, p->n_teams);
+  if (st || p->n_big == 0) return st;
+  if (few) return team(p->d_big, p->n_big);
+  const dim3 grid(p->n_rchunks);
   hipLaunchKernelGGL(cyl_refit_init_kernel, grid, block, 0, ctx->stream, d_xyz, d_offsets,
                      p->d_frames, counts, p->d_rchunks, p->d_rclus, cfg.n_hyp, cfg.thr,
                      cfg.max_radius, k0, k1, tag, cfg.refit_rounds, cfg.refit_iters, d_proposal,
                      d_active, alt_flags, alt_counts, alt_n_hyp, alt_tag, alt_rounds, alt_iters,
-                     cnt, p->d_state, p->d_member, d_mask, d_best, d_model);
+                     p->d_state, p->d_member, d_mask, d_best, d_model);
   SLOAM_HIP(ctx, hipGetLastError());
-  if (p->fused || force_fused) {
-    hipLaunchKernelGGL(cyl_refit_fused_kernel, grid, block, 0, ctx->stream, d_xyz, d_offsets,
-                       p->d_frames, p->d_rchunks, p->d_rclus, p->d_state, p->d_member, cfg.thr,
-                       cnt, d_model);
-    SLOAM_HIP(ctx, hipGetLastError());
-    return SLOAM_OK;
-  }
   // one wave per cluster
-  const dim3 cgrid((std::max(p->n_clusters, 1) + kRefitWaveClusters - 1) / kRefitWaveClusters),
+  const dim3 cgrid((p->n_big + kRefitWaveClusters - 1) / kRefitWaveClusters),
       cblock(64 * kRefitWaveClusters);
   int steps = cfg.refit_rounds * cfg.refit_iters;
   if (alt_flags) steps = std::max(steps, alt_rounds * alt_iters);
   for (int s = 0; s < steps; ++s) {
     hipLaunchKernelGGL(cyl_refit_step_kernel, grid, block, 0, ctx->stream, d_xyz, d_offsets,
                        p->d_frames, p->d_rchunks, p->d_rclus, p->d_state, p->d_member,
-                       p->d_partial, p->d_pcount, s, cfg.thr, cnt);
+                       p->d_partial, p->d_pcount, s, cfg.thr);
     SLOAM_HIP(ctx, hipGetLastError());
-    hipLaunchKernelGGL(cyl_refit_solve_kernel, cgrid, cblock, 0, ctx->stream, p->n_clusters,
-                       p->d_rclus, p->d_state, p->d_partial, p->d_pcount, s, cnt);
+    hipLaunchKernelGGL(cyl_refit_solve_kernel, cgrid, cblock, 0, ctx->stream, p->n_big, p->d_big,
+                       p->d_rclus, p->d_state, p->d_partial, p->d_pcount, s);
     SLOAM_HIP(ctx, hipGetLastError());
   }
   hipLaunchKernelGGL(cyl_refit_final_kernel, grid, block, 0, ctx->stream, d_xyz, d_offsets,
                      p->d_frames, p->d_rchunks, p->d_rclus, p->d_state, p->d_partial,
-                     p->d_pcount, cfg.thr, cnt);
+                     p->d_pcount, cfg.thr);
   SLOAM_HIP(ctx, hipGetLastError());
-  hipLaunchKernelGGL(cyl_refit_finish_kernel, cgrid, cblock, 0, ctx->stream, p->n_clusters,
-                     p->d_frames, p->d_rclus, p->d_state, p->d_partial, p->d_pcount, cnt,
-                     d_model);
+  hipLaunchKernelGGL(cyl_refit_finish_kernel, cgrid, cblock, 0, ctx->stream, p->n_big, p->d_big,
+                     p->d_frames, p->d_rclus, p->d_state, p->d_partial, p->d_pcount, d_model);
   SLOAM_HIP(ctx, hipGetLastError());
   return SLOAM_OK;
 }
 
 // Layout of a counted plan, made on the device: the work list (cluster c's
-// hypothesis chunks at c * cpc .. c * cpc + cpc - 1, clusters in index order),
-// the refit chunks and per-cluster records (prefix sums over the clusters),
-// and cnt = {clusters, work items, refit chunks, overflow}.  A batch beyond
-// the capacities sets overflow and zero counts (nothing runs).  One
-// workgroup of 256 threads.
+// hypothesis chunks at c * cpc .. c * cpc + cpc - 1, clusters in index order)
+// and cnt = {clusters, work items, refit chunks, overflow}.  A batch beyond the
+// capacities, or with a cluster beyond the host plans' bound, sets overflow
+// and zero counts (nothing runs).  One workgroup of 256 threads.
 __global__ __launch_bounds__(256) void cyl_layout_kernel(
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ d_n, int cap,
-    long long cap_points, int n_hyp, int hcap, int cpc, int cap_rchunks, long long cap_words,
-    int4* __restrict__ work, int4* __restrict__ rchunks, int4* __restrict__ rclus,
+    long long cap_points, int n_hyp, int hcap, int cpc, int4* __restrict__ work,
     int32_t* __restrict__ cnt) {
-  __shared__ int wck[4], wwd[4];
-  __shared__ long long s_ck, s_wd;
-  __shared__ int s_over;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nin = *d_n;
   const int n = min(max(nin, 0), cap);
-  if (tid == 0) {
-    s_ck = 0;
-    s_wd = 0;
-    s_over = (nin > cap || nin < 0) ? 1 : 0;
-  }
+  bool over = nin > cap || nin < 0;
+  __shared__ int chunks;
+  if (threadIdx.x == 0) chunks = 0;
   __syncthreads();
-  for (int c0 = 0; c0 < n; c0 += 256) {
-    const int c = c0 + tid;
-    int len = 0, nck = 0, nw = 0;
-    if (c < n) {
-      len = offsets[c + 1] - offsets[c];
-      nck = max(1, (len + kRefitChunk - 1) / kRefitChunk);
-      nw = 2 * ((len + 63) / 64);
-      if (len > kRefitMaxPoints || len < 0) s_over = 1;  // the host plans' bound
-    }
-    // inclusive wave scans, then the waves' totals
-    int sc = nck, sw = nw;
-    for (int o = 1; o < 64; o <<= 1) {
-      const int a = __shfl_up(sc, o, 64), b = __shfl_up(sw, o, 64);
-      if (lane >= o) {
-        sc += a;
-        sw += b;
-      }
-    }
-    if (lane == 63) {
-      wck[wave] = sc;
-      wwd[wave] = sw;
-    }
-    __syncthreads();
-    long long cb = s_ck, wb = s_wd;
-    for (int w = 0; w < wave; ++w) {
-      cb += wck[w];
-      wb += wwd[w];
-    }
-    cb += sc - nck;
-    wb += sw - nw;
-    if (c < n) {
-      rclus[c] = make_int4((int)cb, nck, (int)wb, 0);
-      for (int k = 0; k < nck; ++k)
-        if (cb + k < cap_rchunks)
-          rchunks[cb + k] = make_int4(c, k * kRefitChunk, min(kRefitChunk, len - k * kRefitChunk), k);
-      for (int j = 0; j < cpc; ++j)
-        work[(size_t)c * cpc + j] = make_int4(c, j * hcap, min(hcap, n_hyp - j * hcap), len);
-    }
-    __syncthreads();
-    if (tid == 0) {
-      for (int w = 0; w < 4; ++w) {
-        s_ck += wck[w];
-        s_wd += wwd[w];
-      }
-    }
-    __syncthreads();
+  int nck = 0;
+  for (int c = threadIdx.x; c < n; c += 256) {
+    const int len = offsets[c + 1] - offsets[c];
+    over = over || len > kRefitMaxPoints || len < 0;
+    nck += max(1, (len + kRefitChunk - 1) / kRefitChunk);
+    for (int j = 0; j < cpc; ++j)
+      work[(size_t)c * cpc + j] = make_int4(c, j * hcap, min(hcap, n_hyp - j * hcap), len);
   }
-  if (tid == 0) {
-    const bool over = s_over || s_ck > cap_rchunks || s_wd > cap_words ||
-                      (long long)offsets[n] - (long long)offsets[0] > cap_points;
+  if (nck) atomicAdd(&chunks, nck);
+  over = __syncthreads_or(over) ||
+         (long long)offsets[n] - (long long)offsets[0] > cap_points;
+  if (threadIdx.x == 0) {
     cnt[0] = over ? 0 : n;
     cnt[1] = over ? 0 : n * cpc;
-    cnt[2] = over ? 0 : (int)s_ck;
+    cnt[2] = over ? 0 : chunks;
     cnt[3] = over ? 1 : 0;
   }
 }
@@ -1336,10 +1662,9 @@ __global__ __launch_bounds__(256) void cyl_layout_kernel(
 static int layout_counted(sloam_cyl_plan* p, const int32_t* d_offsets) {
   if (!p->counted) return SLOAM_OK;
   sloam_ctx* ctx = p->ctx;
-  const long long cap_words = (long long)p->cap_member;
   hipLaunchKernelGGL(cyl_layout_kernel, dim3(1), dim3(256), 0, ctx->stream, d_offsets, p->d_n,
                      p->n_clusters, (long long)p->cap_points, p->cfg.n_hyp, p->hcap, p->cpc,
-                     p->n_rchunks, cap_words, p->d_work, p->d_rchunks, p->d_rclus, p->d_cnt);
+                     p->d_work, p->d_cnt);
   SLOAM_HIP(ctx, hipGetLastError());
   return SLOAM_OK;
 }
@@ -1443,7 +1768,7 @@ static int plan_layout(sloam_cyl_plan* p, const int32_t* h_offsets, int32_t n_cl
     // no chunk asked for: 256 hypotheses a workgroup (each workgroup takes the
     // cluster's points into the local frame, for all its hypotheses), fewer
     // where that would leave CUs idle, down to one pass of each wave.  12
-    // trees x 1024 hypotheses: 48 workgroups took 34 us, 384 take PLACEHOLDER2.
+    // trees x 1024 hypotheses: 48 workgroups took 34 us, 384 take 8.
     const int least = kWaves * kHB;
     p->hcap = std::min(256, round_up(cfg.n_hyp, least));
     while (p->hcap > least &&
@@ -1502,16 +1827,21 @@ static int plan_layout(sloam_cyl_plan* p, const int32_t* h_offsets, int32_t n_cl
   std::vector<long long> rload(n_xcd, 0);
   std::vector<int4> rclus(n_clusters);
   int n_chunk_ids = 0;
-  size_t n_words = 0;
   for (int c = 0; c < n_clusters; ++c) {
     const int len = h_offsets[c + 1] - h_offsets[c];
     const int nck = std::max(1, (len + kRefitChunk - 1) / kRefitChunk);
-    rclus[c] = make_int4(n_chunk_ids, nck, (int)n_words, 0);
+    rclus[c] = make_int4(n_chunk_ids, nck, (int)member_word(h_offsets[c], c), 0);
     n_chunk_ids += nck;
-    n_words += 2 * (size_t)((len + 63) / 64);
   }
+  const size_t n_words = member_word(h_offsets[n_clusters], n_clusters);
+  int team_chunks = 0;
+  for (int c = 0; c < n_clusters; ++c) team_chunks = std::max(team_chunks, rclus[c].y);
+  if (team_chunks > kRefitTeamChunks) team_chunks = 1;
+  std::vector<int4> big;
   for (int c : order) {
     const int len = h_offsets[c + 1] - h_offsets[c];
+    if (rclus[c].y <= team_chunks) continue;
+    big.push_back(make_int4(c, -2, 0, 0));
     const int x = (int)(std::min_element(rload.begin(), rload.end()) - rload.begin());
     for (int k = 0; k < rclus[c].y; ++k) {
       const int first = k * kRefitChunk;
@@ -1527,12 +1857,32 @@ static int plan_layout(sloam_cyl_plan* p, const int32_t* h_offsets, int32_t n_cl
     for (int x = 0; x < n_xcd; ++x)
       rchunks.push_back(k < rbins[x].size() ? rbins[x][k] : make_int4(-1, 0, 0, 0));
   p->n_rchunks = (int)rchunks.size();
-  int max_chunks = 0;
-  for (int c = 0; c < n_clusters; ++c) max_chunks = std::max(max_chunks, rclus[c].y);
-  p->fused = n_clusters <= kRefitFusedPlanClusters && max_chunks <= kRefitFusedPlanChunks;
+  // teams, largest clusters first: a workgroup each, and of a batch that has
+  // more clusters than the chip holds workgroups the small ones a wave each
+  std::vector<int4> teams;
+  int4 four = make_int4(-1, -1, -1, -1);
+  int in_four = 0;
+  for (int c : order) {
+    if (rclus[c].y > team_chunks) continue;
+    if (n_clusters <= kRefitTeamBlocks || h_offsets[c + 1] - h_offsets[c] > kWaveRefit) {
+      teams.push_back(make_int4(c, -2, 0, 0));
+      continue;
+    }
+    (in_four == 0 ? four.x : in_four == 1 ? four.y : in_four == 2 ? four.z : four.w) = c;
+    if (++in_four == 4) {
+      teams.push_back(four);
+      four = make_int4(-1, -1, -1, -1);
+      in_four = 0;
+    }
+  }
+  if (in_four) teams.push_back(four);
+  p->n_teams = (int)teams.size();
+  p->n_big = (int)big.size();
   const size_t wb = sizeof(int4) * work.size(), cb = sizeof(int4) * rchunks.size(),
-               lb = sizeof(int4) * rclus.size(), sb = sizeof(int32_t) * seed.size();
-  int st = grow(ctx, &p->d_tables, &p->cap_tables, wb + cb + lb + sb, 1);
+               lb = sizeof(int4) * rclus.size(), eb = sizeof(int4) * teams.size(),
+               bb = sizeof(int4) * big.size(), sb = sizeof(int32_t) * seed.size();
+  const size_t tb = wb + cb + lb + eb + bb + sb;
+  int st = grow(ctx, &p->d_tables, &p->cap_tables, tb, 1);
   if (!st) st = grow(ctx, (void**)&p->d_frames, &p->cap_frames, n_clusters, sizeof(CylFrame));
   if (!st)
     st = grow(ctx, (void**)&p->d_counts, &p->cap_counts, (size_t)n_clusters * cfg.n_hyp,
@@ -1553,10 +1903,12 @@ static int plan_layout(sloam_cyl_plan* p, const int32_t* h_offsets, int32_t n_cl
   p->d_work = static_cast<int4*>(p->d_tables);
   p->d_rchunks = reinterpret_cast<int4*>(static_cast<char*>(p->d_tables) + wb);
   p->d_rclus = reinterpret_cast<int4*>(static_cast<char*>(p->d_tables) + wb + cb);
-  p->d_seed_order = reinterpret_cast<int32_t*>(static_cast<char*>(p->d_tables) + wb + cb + lb);
+  p->d_teams = reinterpret_cast<int4*>(static_cast<char*>(p->d_tables) + wb + cb + lb);
+  p->d_big = p->d_teams + teams.size();
+  p->d_seed_order =
+      reinterpret_cast<int32_t*>(static_cast<char*>(p->d_tables) + wb + cb + lb + eb + bb);
   // the tables through the pinned staging buffer, in one copy (the caller
   // has made sure that no earlier upload from it is pending)
-  const size_t tb = wb + cb + lb + sb;
   if (tb > p->cap_stage) {
     if (p->h_stage) (void)hipHostFree(p->h_stage);
     p->h_stage = nullptr;
@@ -1570,7 +1922,9 @@ static int plan_layout(sloam_cyl_plan* p, const int32_t* h_offsets, int32_t n_cl
   if (wb) std::memcpy(stage, work.data(), wb);
   if (cb) std::memcpy(stage + wb, rchunks.data(), cb);
   if (lb) std::memcpy(stage + wb + cb, rclus.data(), lb);
-  if (sb) std::memcpy(stage + wb + cb + lb, seed.data(), sb);
+  if (eb) std::memcpy(stage + wb + cb + lb, teams.data(), eb);
+  if (bb) std::memcpy(stage + wb + cb + lb + eb, big.data(), bb);
+  if (sb) std::memcpy(stage + wb + cb + lb + eb + bb, seed.data(), sb);
   if (tb) SLOAM_HIP(ctx, hipMemcpyAsync(p->d_tables, stage, tb, hipMemcpyHostToDevice, ctx->stream));
   return SLOAM_OK;
 }
@@ -1648,37 +2002,27 @@ int sloam_cyl_plan_create_counted(sloam_ctx* ctx, int32_t cap_clusters, int64_t 
   sloam_cyl_plan* p = plan_new(ctx, cfg, &st);
   if (!p) return st;
   p->counted = true;
-  p->fused = true;
   p->d_n = d_n_clusters;
   p->cap_points = cap_points;
   p->cpc = (cfg->n_hyp + p->hcap - 1) / p->hcap;
   p->n_clusters = cap_clusters;
   p->n_points = cap_points;
   p->n_work = cap_clusters * p->cpc;
-  p->n_rchunks = (int)(cap_clusters + cap_points / kRefitChunk + 1);
-  const size_t words = (size_t)(cap_points / 32) + 2 * (size_t)cap_clusters + 2;
-  const size_t tb = sizeof(int4) * ((size_t)p->n_work + p->n_rchunks + cap_clusters);
+  const size_t words = member_word(cap_points, cap_clusters);
+  const size_t tb = sizeof(int4) * (size_t)p->n_work;
   st = grow(ctx, &p->d_tables, &p->cap_tables, tb, 1);
   if (!st) st = grow(ctx, (void**)&p->d_frames, &p->cap_frames, cap_clusters, sizeof(CylFrame));
   if (!st)
     st = grow(ctx, (void**)&p->d_counts, &p->cap_counts, (size_t)cap_clusters * cfg->n_hyp,
               sizeof(int32_t));
-  if (!st)
-    st = grow(ctx, (void**)&p->d_state, &p->cap_state, cap_clusters, sizeof(RefitState));
   if (!st) st = grow(ctx, (void**)&p->d_member, &p->cap_member, words, sizeof(uint32_t));
   if (!st) st = grow(ctx, (void**)&p->d_rescue, &p->cap_rescue, cap_clusters, sizeof(int32_t));
-  if (!st)
-    st = grow(ctx, (void**)&p->d_partial, &p->cap_partial, p->n_rchunks,
-              sizeof(Comp2) * kRefitTerms);
-  if (!st) st = sloam_dev_alloc(ctx, (void**)&p->d_pcount, sizeof(int32_t) * p->cap_partial);
   if (!st) st = sloam_dev_alloc(ctx, (void**)&p->d_cnt, sizeof(int32_t) * 4);
   if (st) {
     sloam_cyl_plan_destroy(p);
     return st;
   }
   p->d_work = static_cast<int4*>(p->d_tables);
-  p->d_rchunks = p->d_work + p->n_work;
-  p->d_rclus = p->d_rchunks + p->n_rchunks;
   *out = p;
   return SLOAM_OK;
 }
@@ -1703,6 +2047,8 @@ int sloam_cyl_plan_reset(sloam_cyl_plan* p, const int32_t* h_offsets, int32_t n_
     p->n_points = 0;
     p->n_work = 0;
     p->n_rchunks = 0;
+    p->n_teams = 0;
+    p->n_big = 0;
   }
   return st;
 }
@@ -1809,7 +2155,7 @@ int sloam_cyl_learned_exec(sloam_cyl_plan* verify, sloam_cyl_plan* plain, const 
     // rescue: the verified clusters whose refit failed or kept fewer than
     // min_inlier_ratio * n inliers take the plain method's fit after all
     // (scored with the plain hypotheses in the same seed frames, refitted
-    // alone in the fused form)
+    // alone)
     SloamKernelScope ks(ctx, "cyl_rescue");
     hipLaunchKernelGGL(cyl_rescue_kernel, dim3((S + 255) / 256), dim3(256), 0, ctx->stream,
                        d_offsets, S, d_model, min_inlier_ratio, vcnt, d_fallback,
@@ -1828,7 +2174,7 @@ int sloam_cyl_learned_exec(sloam_cyl_plan* verify, sloam_cyl_plan* plain, const 
     const int st = launch_refit(verify, d_xyz, d_offsets, cv, nullptr, verify->d_rescue,
                                 verify->d_rescue, cp, pc.n_hyp, (uint32_t)pc.stream_tag,
                                 pc.refit_rounds, pc.refit_iters, nullptr, d_best, d_model,
-                                /*force_fused=*/true);
+                                /*few=*/true);
     if (st) return st;
   }
   return SLOAM_OK;

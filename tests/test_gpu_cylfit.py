@@ -105,6 +105,35 @@ def test_large_cluster_takes_per_step_refit(ctx):
         _compare(g, o, o_off[-1])
 
 
+EDGES = [0, 2, 3, 63, 64, 65, 127, 255, 256, 257, 511, 512, 513, 2047, 2048, 2049]
+
+
+@pytest.mark.parametrize("sizes", [
+    EDGES + [4096, 4097, 8191, 8192],        # a workgroup each, up to 4 chunks
+    EDGES + [6143] + [20] * 1020,            # the small ones four to a workgroup
+    EDGES + [4097, 8193],                    # several chunks: a launch per step
+], ids=["teams", "waves", "steps"])
+def test_refit_forms_at_their_edges(ctx, sizes):
+    """Each form of the refit at the sizes where a wave's, a turn's, a chunk's
+    or a team's points end; one cluster of 1e-17 m (squared distances below
+    the range of the joint root and reciprocal).  Bit-exact as everywhere."""
+    rng = np.random.default_rng(len(sizes))
+    pts = []
+    for k, n in enumerate(sizes):
+        p, _ = synth.trunk_points(rng, n, np.array([5.0 + k % 7, 1.0, 0.0]),
+                                  np.array([0.0, 0.05, 1.0]), 0.3, 4.0, 0.02, 0.2)
+        pts.append(p)
+    pts.append(pts[sizes.index(257)] * 1e-17)
+    d = {"xyz": np.concatenate(pts).astype(np.float32),
+         "offsets": np.cumsum([0] + [len(p) for p in pts]).astype(np.int32)}
+    _run_both(d, 96)
+    g = fit_cylinders(ctx, d["xyz"], d["offsets"], n_hyp=96, counts=True, samples=True,
+                      mask=True, best=True)
+    o = oracle.cyl_fit_batch(d["xyz"], d["offsets"], 96, samples=True, threads=8)
+    assert (o["model"][:, 6] > 0).sum() >= len(pts) - 12 and o["model"][-1, 6] > 0
+    _compare(g, o, d["offsets"][-1])
+
+
 @pytest.mark.parametrize("hyp_chunk,tile", [(32, 64), (96, 512), (1024, 4096)])
 def test_launch_shapes_do_not_change_results(ctx, hyp_chunk, tile):
     d = synth.make_clusters(40, seed=9)
