@@ -66,19 +66,16 @@ void sloam_ctx_pin_slots(sloam_ctx* ctx, uint32_t slots, int delta);
 int sloam_project_noalloc_init(sloam_ctx* ctx);
 
 // Pose solves whose problem count is in device memory (*d_n_problems <=
-// max_problems): LM state set-up and the fused LM kernel of
-// sloam_pose_plan_exec over a work list built on the device (d_work: int4
-// {problem, first residual, end residual, 0} per chunk of at most 2048
-// residuals, d_first: first chunk of each problem).  d_state holds
-// max_problems LM states (sloam_pose_state_bytes each); d_cyl_tab / d_pl_tab
-// the landmark tables (per cylinder / plane: 32 / 16 bytes at cfg->precision
+// max_problems): the fused LM kernel of sloam_pose_plan_exec over a work list
+// built on the device (d_work: int4 {problem, first residual, end residual, 0}
+// per chunk of at most 2048 residuals, d_first: first chunk of each problem).
+// d_cyl_tab / d_pl_tab take the landmark tables (per cylinder / plane: 32 / 16 bytes at cfg->precision
 // 0, 64 / 32 bytes at precision 1).
-size_t sloam_pose_state_bytes();
 int sloam_pose_fused_device(sloam_ctx* ctx, int max_problems, const int32_t* d_n_problems,
                             const float* d_points, const int32_t* d_work, const int32_t* d_first,
                             const double* d_cyl, const int32_t* d_cyl_off, const double* d_planes,
                             const int32_t* d_pl_off, const double* d_pose_in,
-                            const int32_t* d_free_mask, const sloam_pose_cfg* cfg, void* d_state,
+                            const int32_t* d_free_mask, const sloam_pose_cfg* cfg,
                             void* d_cyl_tab, void* d_pl_tab, double* d_pose_out,
                             double* d_params_out, int32_t* d_status, double* d_cost);
 
@@ -318,6 +315,34 @@ __host__ __device__ inline void sl_basis(const double a[3], double e1[3], double
   e2[0] = a[1] * z - a[2] * y;
   e2[1] = a[2] * x - a[0] * z;
   e2[2] = a[0] * y - a[1] * x;
+}
+
+// rho = sqrt(x) and inv = 1 / rho, both correctly rounded, from one v_rsq and
+// a Newton step each with exact residuals (Markstein 1990) instead of the
+// compiler's separate square root and divide: 9 instructions and 3 compares
+// for about 25.  Equal to sqrtf(x) and 1.0f / sqrtf(x) at every float of
+// [2^-96, 2^96) where e is not 2^-24 (all 1.6e9 tried on the card; the one
+// exception there is a rho whose mantissa is all ones).  False for the other
+// x, 0, infinity and NaN among them: they take sl_sqrt_inv_any.
+__device__ inline bool sl_sqrt_inv(float x, float& rho, float& inv) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float g = x * y;
+  rho = __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+  const float e = __builtin_fmaf(-rho, y, 1.0f);
+  inv = __builtin_fmaf(e, y, y);
+  return x >= 0x1p-96f && x < 0x1p96f && e != 0x1p-24f;
+}
+
+__device__ inline void sl_sqrt_inv_any(float x, float& rho, float& inv) {
+  rho = sqrtf(x);
+  inv = 1.0f / rho;
+}
+
+// d of lane `from` (uniform), as a scalar on every lane
+__device__ inline double sl_lane_value(double d, int from) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(d), from);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(d), from);
+  return __hiloint2double(hi, lo);
 }
 
 // ---------------------------------------------------------------------------

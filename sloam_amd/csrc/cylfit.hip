@@ -580,27 +580,6 @@ __device__ inline void refit_model_f32(RefitState& S) {
   S.rf = (float)S.r;
 }
 
-// rho = sqrt(x) and inv = 1 / rho, both correctly rounded, from one v_rsq and
-// a Newton step each with exact residuals (Markstein 1990) instead of the
-// compiler's separate square root and divide: 9 instructions and 3 compares
-// for about 25.  Equal to sqrtf(x) and 1.0f / sqrtf(x) at every float of
-// [2^-96, 2^96) where e is not 2^-24 (all 1.6e9 tried on the card; the one
-// exception there is a rho whose mantissa is all ones).  False for the other
-// x, 0, infinity and NaN among them: they take sqrt_inv_any.
-__device__ inline bool sqrt_inv(float x, float& rho, float& inv) {
-  const float y = __builtin_amdgcn_rsqf(x);
-  const float g = x * y;
-  rho = __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
-  const float e = __builtin_fmaf(-rho, y, 1.0f);
-  inv = __builtin_fmaf(e, y, y);
-  return x >= 0x1p-96f && x < 0x1p96f && e != 0x1p-24f;
-}
-
-__device__ inline void sqrt_inv_any(float x, float& rho, float& inv) {
-  rho = sqrtf(x);
-  inv = 1.0f / rho;
-}
-
 // Of N points x (relative to the frame centre): w, the part of the offset to
 // the model's axis point orthogonal to the axis, h along it, rho = |w| and
 // 1 / rho.  Together, so that their chains overlap.
@@ -617,11 +596,11 @@ __device__ inline void refit_dist(const RefitState& S, const float (&x)[N][3], f
     w[k][1] = __builtin_fmaf(-h[k], S.af[1], q1);
     w[k][2] = __builtin_fmaf(-h[k], S.af[2], q2);
     ww[k] = __builtin_fmaf(w[k][2], w[k][2], __builtin_fmaf(w[k][1], w[k][1], w[k][0] * w[k][0]));
-    ok &= sqrt_inv(ww[k], rho[k], inv[k]);
+    ok &= sl_sqrt_inv(ww[k], rho[k], inv[k]);
   }
   if (!ok) {
 #pragma unroll
-    for (int k = 0; k < N; ++k) sqrt_inv_any(ww[k], rho[k], inv[k]);
+    for (int k = 0; k < N; ++k) sl_sqrt_inv_any(ww[k], rho[k], inv[k]);
   }
 }
 
@@ -875,13 +854,6 @@ __device__ inline int wave_sum_int(int v) {
   return v;
 }
 
-// d of lane `from` (uniform), as a scalar on every lane
-__device__ inline double lane_value(double d, int from) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(d), from);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(d), from);
-  return __hiloint2double(hi, lo);
-}
-
 // The Gauss-Newton step's solve of one cluster by one wave: lane q <
 // kRefitTerms sums term q over the chunks, then the FP64 5x5 normal equations
 // and the next model (lane 0 writes S).  Too few inliers stop the cluster; a
@@ -918,8 +890,8 @@ __device__ inline void refit_solve_wave(RefitState& S, const Comp2* part, const 
   for (int j = 0; j < 5; ++j) {
     t = row[j];
 #pragma unroll
-    for (int k = 0; k < j; ++k) t = t - Lr[k] * lane_value(Lr[k], j);
-    const double s = lane_value(t, j);
+    for (int k = 0; k < j; ++k) t = t - Lr[k] * sl_lane_value(Lr[k], j);
+    const double s = sl_lane_value(t, j);
     ok = ok && (s > 0.0);
     diag[j] = sqrt(s);
     Lr[j] = t / diag[j];
@@ -931,9 +903,9 @@ __device__ inline void refit_solve_wave(RefitState& S, const Comp2* part, const 
   double x[5];
 #pragma unroll
   for (int i = 4; i >= 0; --i) {
-    double u = lane_value(Lr[i], 5);
+    double u = sl_lane_value(Lr[i], 5);
 #pragma unroll
-    for (int k = i + 1; k < 5; ++k) u = u - lane_value(Lr[i], k) * x[k];
+    for (int k = i + 1; k < 5; ++k) u = u - sl_lane_value(Lr[i], k) * x[k];
     x[i] = u / diag[i];
   }
   RefitState N = S;

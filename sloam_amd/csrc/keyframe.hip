@@ -799,7 +799,6 @@ struct sloam_kf_estimator {
   double* params_out = nullptr;
   int32_t* status = nullptr;
   double* cost = nullptr;
-  void* lm_state = nullptr;
   void* cyl_tab = nullptr;  // pose landmark tables, FP64 size
   void* pl_tab = nullptr;
   size_t r_off[7] = {};  // byte offsets of the result regions
@@ -844,8 +843,7 @@ int sloam_kf_estimator_create(sloam_ctx* ctx, const sloam_kf_params* p, int32_t 
                o_work = take(16 * (size_t)e->cap_work), o_first = take(4 * 4),
                o_np = take(4), o_pose_out = take(8 * 14), o_params = take(8 * 12),
                o_status = take(4 * 4), o_cost = take(8 * 4),
-               o_lm_state = take(2 * sloam_pose_state_bytes()), o_cylf = take(8 * 8 * T),
-               o_plf = take(8 * 4 * Cc);
+               o_cylf = take(8 * 8 * T), o_plf = take(8 * 4 * Cc);
   int st = sloam_dev_alloc(ctx, &e->dev, off);
   if (st) {
     delete e;
@@ -903,7 +901,6 @@ int sloam_kf_estimator_create(sloam_ctx* ctx, const sloam_kf_params* p, int32_t 
   e->params_out = reinterpret_cast<double*>(d + o_params);
   e->status = reinterpret_cast<int32_t*>(d + o_status);
   e->cost = reinterpret_cast<double*>(d + o_cost);
-  e->lm_state = d + o_lm_state;
   e->cyl_tab = d + o_cylf;
   e->pl_tab = d + o_plf;
   b.pose_out = e->pose_out;
@@ -1006,7 +1003,7 @@ int sloam_kf_estimator_exec(sloam_kf_estimator* e, const sloam_kf_inputs* in) {
     SloamKernelScope ks(ctx, "kf_pose");
     const int st = sloam_pose_fused_device(
         ctx, 2, b.n_problems, b.res, b.work, b.first, b.cyl, b.cyl_off, b.pl, b.pl_off, b.pose_in,
-        b.free_mask, &c, e->lm_state, e->cyl_tab, e->pl_tab, e->pose_out, e->params_out, e->status,
+        b.free_mask, &c, e->cyl_tab, e->pl_tab, e->pose_out, e->params_out, e->status,
         e->cost);
     if (st) return st;
   }

@@ -5,7 +5,8 @@
 // CylinderCost (sloam/include/objects/cylinder.h:90-132) and PlaneCost
 // (sloam/include/objects/plane.h:76-116), HuberLoss(0.1), Ceres LM.
 //
-// Per LM iteration two kernels run on the context stream:
+// Per LM iteration pose_eval and, for large problem sets, pose_solve run on the
+// context stream (else pose_eval makes the step of the evaluation before it):
 //   pose_eval   one workgroup per chunk of 256 * kRpt residuals of one problem:
 //               FP32 residual r, 1x6 Jacobian [d/dt, d/dtheta] (left
 //               perturbation), Huber IRLS weight w = min(1, delta/|r|); sums
@@ -14,14 +15,14 @@
 //               28 (sum, compensation) pairs go to HBM as FP64.
 //   pose_solve  one wave per problem: FP64 sum of the chunk partials in chunk
 //               order, then the LM trust-region logic and the FP64 6x6
-//               Cholesky solve of (J'WJ + D/radius) dx = -J'Wr; writes the next
-//               pose to evaluate.
+//               Cholesky solve of (J'WJ + D/radius) dx = -J'Wr, a row per lane;
+//               writes the next pose to evaluate.
 // pose_fused    one workgroup per problem runs every iteration in one launch:
 //               the same chunk evaluations and the same FP64 sum of chunk
-//               partials in chunk order, then the same LM step in thread 0,
-//               so its results are bit-identical to the two-kernel loop.  It
+//               partials in chunk order, then the same LM step in its first
+//               wave, so its results are bit-identical to the loop's.  It
 //               serves small problems (a keyframe's solve), where the loop's
-//               2 * (max_iters + 1) launches cost more than the work.
+//               max_iters + 2 launches cost more than the work.
 // Coordinates are evaluated relative to a per-problem anchor (the initial
 // translation) so that FP32 residuals keep sub-micrometre resolution.
 //
@@ -52,14 +53,15 @@ static_assert(kSums * kParts <= kPBlock && kPBlock % kParts == 0, "chunk reducti
 
 // LDS of the chunk reduction: every thread's sums, then the partials
 struct ChunkRed {
-  float x[kSums][kPBlock + 1];
+  // rows of 260: a chain reads four values at a time, 16 chains distinct banks
+  alignas(16) float x[kSums][kPBlock + 4];
   float ps[kSums][kParts];
   float pc[kSums][kParts];
 };
 
 // the same in FP64 (plain sums in the same order)
 struct ChunkRed64 {
-  double x[kSums][kPBlock + 1];
+  alignas(16) double x[kSums][kPBlock + 2];
   double ps[kSums][kParts];
 };
 
@@ -189,43 +191,6 @@ __device__ inline void left_jacobian(const double w[3], double J[3][3]) {
     }
 }
 
-__device__ inline bool chol6(const double A[6][6], const double b[6], double x[6]) {
-  double L[6][6];
-  bool ok = true;
-#pragma unroll
-  for (int j = 0; j < 6; ++j) {
-    double s = A[j][j];
-#pragma unroll
-    for (int k = 0; k < j; ++k) s = s - L[j][k] * L[j][k];
-    ok = ok && (s > 0.0);
-    const double d = sqrt(s);
-    L[j][j] = d;
-#pragma unroll
-    for (int i = j + 1; i < 6; ++i) {
-      double t = A[i][j];
-#pragma unroll
-      for (int k = 0; k < j; ++k) t = t - L[i][k] * L[j][k];
-      L[i][j] = t / d;
-    }
-  }
-  double y[6];
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    double t = b[i];
-#pragma unroll
-    for (int k = 0; k < i; ++k) t = t - L[i][k] * y[k];
-    y[i] = t / L[i][i];
-  }
-#pragma unroll
-  for (int i = 5; i >= 0; --i) {
-    double t = y[i];
-#pragma unroll
-    for (int k = i + 1; k < 6; ++k) t = t - L[k][i] * x[k];
-    x[i] = t / L[i][i];
-  }
-  return ok;
-}
-
 // error-free transformation: a + b = s + e exactly
 __device__ inline void two_sum(float a, float b, float* s, float* e) {
   const float ss = a + b;
@@ -238,21 +203,23 @@ __device__ inline void two_sum(float a, float b, float* s, float* e) {
 // prep: LM state init + landmark tables: FP32 relative to the anchor, or FP64
 // absolute (F64)
 // --------------------------------------------------------------------------
-// d_n_problems (nullable): the problem count in device memory (a grid of
-// n_problems workgroups then serves any count up to n_problems)
+// Of problem k by one workgroup: its landmarks' entries and its state S.
+struct PoseIn {
+  const double* pose;
+  const int32_t* free_mask;  // nullable
+  const double* cyl;
+  const int32_t* cyl_off;
+  const double* pl;
+  const int32_t* pl_off;
+};
+
 template <bool F64>
-__global__ __launch_bounds__(kPBlock) void pose_prep_kernel(
-    int n_problems, const int32_t* __restrict__ d_n_problems, const double* __restrict__ pose_in,
-    const int32_t* __restrict__ free_mask, const double* __restrict__ cyl,
-    const int32_t* __restrict__ cyl_off, const double* __restrict__ pl,
-    const int32_t* __restrict__ pl_off, PoseCfgDev cfg, LMState* __restrict__ st,
-    void* __restrict__ cyl_tab, void* __restrict__ pl_tab) {
-  const int k = blockIdx.x;
-  if (k >= n_problems || (d_n_problems && k >= *d_n_problems)) return;
-  const double* x0 = pose_in + 7 * (size_t)k;
+__device__ inline void pose_prep(int k, const PoseIn& in, const PoseCfgDev& cfg, LMState* S,
+                                 void* cyl_tab, void* pl_tab) {
+  const double* x0 = in.pose + 7 * (size_t)k;
   const double ax = x0[0], ay = x0[1], az = x0[2];
-  for (int i = cyl_off[k] + (int)threadIdx.x; i < cyl_off[k + 1]; i += kPBlock) {
-    const double* c = cyl + 8 * (size_t)i;
+  for (int i = in.cyl_off[k] + (int)threadIdx.x; i < in.cyl_off[k + 1]; i += kPBlock) {
+    const double* c = in.cyl + 8 * (size_t)i;
     const double rn = sqrt(c[3] * c[3] + c[4] * c[4] + c[5] * c[5]);
     if constexpr (F64) {
       double4* t = static_cast<double4*>(cyl_tab) + 2 * (size_t)i;
@@ -264,8 +231,8 @@ __global__ __launch_bounds__(kPBlock) void pose_prep_kernel(
       t[1] = make_float4((float)(c[3] / rn), (float)(c[4] / rn), (float)(c[5] / rn), 0.f);
     }
   }
-  for (int i = pl_off[k] + (int)threadIdx.x; i < pl_off[k + 1]; i += kPBlock) {
-    const double* q = pl + 4 * (size_t)i;
+  for (int i = in.pl_off[k] + (int)threadIdx.x; i < in.pl_off[k + 1]; i += kPBlock) {
+    const double* q = in.pl + 4 * (size_t)i;
     const double nn = sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
     if constexpr (F64) {
       static_cast<double4*>(pl_tab)[i] = make_double4(q[0] / nn, q[1] / nn, q[2] / nn, q[3] / nn);
@@ -294,7 +261,7 @@ __global__ __launch_bounds__(kPBlock) void pose_prep_kernel(
     s.term = 1;
     s.done = 0;
     s.phase = 0;
-    s.free_mask = free_mask ? free_mask[k] : 0x3f;
+    s.free_mask = in.free_mask ? in.free_mask[k] : 0x3f;
     s.pad = 0;
     s.aa[0] = s.aae[0] = x0[0];
     s.aa[1] = s.aae[1] = x0[1];
@@ -304,8 +271,18 @@ __global__ __launch_bounds__(kPBlock) void pose_prep_kernel(
       quat_to_aa(x0 + 3, w);
       for (int i = 0; i < 3; ++i) s.aa[3 + i] = s.aae[3 + i] = w[i];
     }
-    st[k] = s;
+    *S = s;
   }
+}
+
+template <bool F64>
+__global__ __launch_bounds__(kPBlock) void pose_prep_kernel(int n_problems, PoseIn in,
+                                                            PoseCfgDev cfg,
+                                                            LMState* __restrict__ st,
+                                                            void* __restrict__ cyl_tab,
+                                                            void* __restrict__ pl_tab) {
+  const int k = blockIdx.x;
+  if (k < n_problems) pose_prep<F64>(k, in, cfg, st + k, cyl_tab, pl_tab);
 }
 
 // --------------------------------------------------------------------------
@@ -353,8 +330,8 @@ __device__ inline void eval_frame(const LMState& s, int param, EvalFrame& F) {
 // 16 bytes of HBM).  kSub false (the quaternion parametrization, all
 // parameters free) drops the left-Jacobian map and the masks, whose identity
 // and unit factors change no bit.  The divides and the square root stay
-// correctly rounded: the hardware reciprocals would save ~35 instructions per
-// residual but move the LM path of small ill-conditioned problems by more
+// correctly rounded (a root and its reciprocal from one v_rsq): the hardware
+// reciprocals alone would move the LM path of small ill-conditioned problems by more
 // than 1e-4 within a fixed iteration count.
 template <bool kSub>
 __device__ inline double eval_chunk(const float4* __restrict__ pts, int b, int e,
@@ -408,9 +385,11 @@ __device__ inline double eval_chunk(const float4* __restrict__ pts, int b, int e
       const float w0 = __builtin_fmaf(-h, L1.x, v0);
       const float w1 = __builtin_fmaf(-h, L1.y, v1);
       const float w2 = __builtin_fmaf(-h, L1.z, v2);
-      const float rho = sqrtf(__builtin_fmaf(w0, w0, __builtin_fmaf(w1, w1, w2 * w2)));
+      const float ww = __builtin_fmaf(w0, w0, __builtin_fmaf(w1, w1, w2 * w2));
+      float rho, inv;
+      if (!sl_sqrt_inv(ww, rho, inv)) sl_sqrt_inv_any(ww, rho, inv);
       r = rho - L0.w;
-      const float inv = rho > 0.f ? 1.0f / rho : 0.f;
+      inv = rho > 0.f ? inv : 0.f;
       dir[0] = w0 * inv;
       dir[1] = w1 * inv;
       dir[2] = w2 * inv;
@@ -480,13 +459,23 @@ __device__ inline double eval_chunk(const float4* __restrict__ pts, int b, int e
   __syncthreads();
   if (threadIdx.x < kSums * kParts) {
     const int i = threadIdx.x % kSums, part = threadIdx.x / kSums;
-    const float* row = &red.x[i][part * (kPBlock / kParts)];
-    float sm = row[0], c = 0.f;
-    for (int j = 1; j < kPBlock / kParts; ++j) {
-      float ns, err;
-      two_sum(sm, row[j], &ns, &err);
-      sm = ns;
-      c += err;
+    const float4* row = reinterpret_cast<const float4*>(&red.x[i][part * (kPBlock / kParts)]);
+    float sm = 0.f, c = 0.f;
+#pragma unroll
+    for (int j = 0; j < kPBlock / kParts / 4; ++j) {
+      const float4 q = row[j];
+      const float v[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (j == 0 && u == 0) {
+          sm = v[0];
+          continue;
+        }
+        float ns, err;
+        two_sum(sm, v[u], &ns, &err);
+        sm = ns;
+        c += err;
+      }
     }
     red.ps[i][part] = sm;
     red.pc[i][part] = c;
@@ -637,9 +626,14 @@ __device__ inline double eval_chunk64(const float4* __restrict__ pts, int b, int
   __syncthreads();
   if (threadIdx.x < kSums * kParts) {
     const int i = threadIdx.x % kSums, part = threadIdx.x / kSums;
-    const double* row = &red.x[i][part * (kPBlock / kParts)];
-    double sm = row[0];
-    for (int j = 1; j < kPBlock / kParts; ++j) sm += row[j];
+    const double2* row = reinterpret_cast<const double2*>(&red.x[i][part * (kPBlock / kParts)]);
+    double sm = 0.0;
+#pragma unroll
+    for (int j = 0; j < kPBlock / kParts / 2; ++j) {
+      const double2 q = row[j];
+      sm = j == 0 ? q.x : sm + q.x;
+      sm += q.y;
+    }
     red.ps[i][part] = sm;
   }
   __syncthreads();
@@ -682,146 +676,167 @@ struct PoseEval<true> {
   }
 };
 
-// work item = {problem, first residual, end residual, unused}
-template <bool F64>
-__global__ __launch_bounds__(kPBlock) void pose_eval_kernel(
-    const float4* __restrict__ pts, const int4* __restrict__ work, const LMState* __restrict__ st,
-    const void* __restrict__ cyl_tab, const void* __restrict__ pl_tab, double delta, int param,
-    double* __restrict__ partials) {
-  using E = PoseEval<F64>;
-  __shared__ typename E::Red red;
-  const int4 w = work[blockIdx.x];
-  const int k = w.x;
-  if (st[k].done) return;
-  typename E::Frame F;
-  E::frame(st[k], param, F);
-  const double p = E::chunk(pts, w.y, w.z, F, cyl_tab, pl_tab, delta, red);
-  if (threadIdx.x < kSums) partials[(size_t)blockIdx.x * kSums + threadIdx.x] = p;
-}
-
 // --------------------------------------------------------------------------
 // solve: LM trust-region logic and the FP64 6x6 step on the summed evaluation
-// tot[28] of the pose S.xe (one thread)
+// tot[28] of the pose S.xe, by one whole wave (S and tot in LDS).  The values
+// are a scalar program's; the Cholesky factor has a row per lane (the right
+// side is row 6, so that the forward substitution is part of it) and a
+// column's divisions run at once: with one lane for all, the loop's solve kernel
+// took 9 us for 5, a keyframe's pair of solves 48 for 39.
 // --------------------------------------------------------------------------
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 __device__ inline void lm_step(LMState& S, const double* tot, const PoseCfgDev& cfg) {
-  // evaluation result of S.xe
-  double A[6][6], g[6];
-  {
-    int tt = 0;
-    for (int a = 0; a < 6; ++a)
-      for (int b = a; b < 6; ++b) {
-        A[a][b] = tot[tt];
-        A[b][a] = tot[tt];
-        ++tt;
-      }
-    for (int a = 0; a < 6; ++a) g[a] = tot[21 + a];
-  }
+  const int lane = threadIdx.x & 63;
   const double Fe = tot[27];
-  auto store_eval = [&]() {
-    int tt = 0;
-    for (int a = 0; a < 6; ++a)
-      for (int b = a; b < 6; ++b) S.A[tt++] = A[a][b];
-    for (int a = 0; a < 6; ++a) S.g[a] = g[a];
-    S.F = Fe;
-  };
-  bool done = false;
+  double radius = S.radius, factor = S.factor, F = S.F, F0 = S.F0;
+  int term = S.term, iter = S.iter;
+  bool done = false, accept = false;
+  double gmax = 0.0;
+#pragma unroll
+  for (int a = 0; a < 6; ++a) gmax = fmax(gmax, fabs(tot[21 + a]));
   if (S.phase == 0) {
-    store_eval();
-    S.F0 = Fe;
-    double gmax = 0.0;
-    for (int a = 0; a < 6; ++a) gmax = fmax(gmax, fabs(g[a]));
+    accept = true;
+    F = F0 = Fe;
     if (gmax <= cfg.gtol) {
-      S.term = 0;
+      term = 0;
       if (cfg.stop_conv) done = true;
     }
   } else {
-    const double change = S.F - Fe;
-    const double q = S.model > 0.0 ? change / S.model : -1.0;
+    const double change = F - Fe, dn = S.dn, xn = S.xn, model = S.model;
+    const double q = model > 0.0 ? change / model : -1.0;
     if (isfinite(Fe) && q > cfg.min_rel) {
-      for (int i = 0; i < 7; ++i) S.x[i] = S.xe[i];
-      for (int i = 0; i < 6; ++i) S.aa[i] = S.aae[i];
-      const double Fprev = S.F;
-      store_eval();
+      accept = true;
+      const double Fprev = F;
+      F = Fe;
       const double c3 = 2.0 * q - 1.0;
-      S.radius = S.radius / fmax(1.0 / 3.0, 1.0 - c3 * c3 * c3);
-      S.radius = fmin(S.radius, 1e16);
-      S.factor = 2.0;
-      double gmax = 0.0;
-      for (int a = 0; a < 6; ++a) gmax = fmax(gmax, fabs(S.g[a]));
+      radius = radius / fmax(1.0 / 3.0, 1.0 - c3 * c3 * c3);
+      radius = fmin(radius, 1e16);
+      factor = 2.0;
       if (fabs(change) <= cfg.ftol * Fprev || gmax <= cfg.gtol ||
-          S.dn <= cfg.ptol * (S.xn + cfg.ptol)) {
-        S.term = 0;
+          dn <= cfg.ptol * (xn + cfg.ptol)) {
+        term = 0;
         if (cfg.stop_conv) done = true;
       }
     } else {
-      S.radius = S.radius / S.factor;
-      S.factor = S.factor * 2.0;
-      if (S.dn <= cfg.ptol * (S.xn + cfg.ptol)) {
-        S.term = 0;
+      radius = radius / factor;
+      factor = factor * 2.0;
+      if (dn <= cfg.ptol * (xn + cfg.ptol)) {
+        term = 0;
         if (cfg.stop_conv) done = true;
       }
     }
   }
+  if (accept) {
+    if (S.phase != 0) {
+      if (lane < 7) S.x[lane] = S.xe[lane];
+      if (lane < 6) S.aa[lane] = S.aae[lane];
+    }
+    if (lane < 21) S.A[lane] = tot[lane];
+    if (lane < 6) S.g[lane] = tot[21 + lane];
+  }
+  wave_fence();
   // next candidate
+  const int r = min(lane, 6);
+  double arow[6], g[6], dx[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    const int lo = min(min(r, 5), c), hi = max(min(r, 5), c);
+    arow[c] = S.A[lo * 6 - lo * (lo - 1) / 2 + (hi - lo)];
+    g[c] = S.g[c];
+  }
+  double dg = arow[0];
+#pragma unroll
+  for (int c = 1; c < 6; ++c) dg = r == c ? arow[c] : dg;
+  dg = dg < 1e-6 ? 1e-6 : (dg > 1e32 ? 1e32 : dg);
   bool have_candidate = false;
-  while (!done && S.iter < cfg.max_iters) {
-    S.iter += 1;
-    double Acur[6][6], Aug[6][6], rhs[6], dx[6];
-    {
-      int tt = 0;
-      for (int a = 0; a < 6; ++a)
-        for (int b = a; b < 6; ++b) {
-          Acur[a][b] = S.A[tt];
-          Acur[b][a] = S.A[tt];
-          ++tt;
-        }
+  while (!done && iter < cfg.max_iters) {
+    iter += 1;
+    const double damp = dg / radius;
+    double L[6], diag[6];
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      double t = r == 6 ? -g[j] : arow[j];
+      if (r == j) t += damp;
+#pragma unroll
+      for (int k = 0; k < j; ++k) t = t - L[k] * sl_lane_value(L[k], j);
+      const double s = sl_lane_value(t, j);
+      ok = ok && (s > 0.0);
+      diag[j] = sqrt(s);
+      L[j] = t / diag[j];
     }
-    for (int a = 0; a < 6; ++a) {
-      for (int b = 0; b < 6; ++b) Aug[a][b] = Acur[a][b];
-      double dg = Acur[a][a];
-      dg = dg < 1e-6 ? 1e-6 : (dg > 1e32 ? 1e32 : dg);
-      Aug[a][a] += dg / S.radius;
-      rhs[a] = -S.g[a];
-    }
-    if (!chol6(Aug, rhs, dx)) {
-      S.radius = S.radius / S.factor;
-      S.factor = S.factor * 2.0;
+    if (!ok) {
+      radius = radius / factor;
+      factor = factor * 2.0;
       continue;
     }
-    double gdx = 0.0, dAd = 0.0;
-    for (int a = 0; a < 6; ++a) {
-      gdx += S.g[a] * dx[a];
-      double tt = 0.0;
-      for (int b = 0; b < 6; ++b) tt += Acur[a][b] * dx[b];
-      dAd += dx[a] * tt;
-    }
-    S.model = -(gdx + 0.5 * dAd);
-    double xn = 0.0, dn = 0.0;
-    if (cfg.param == 1) {
-      for (int a = 0; a < 6; ++a) xn += S.aa[a] * S.aa[a];
-    } else {
-      for (int a = 0; a < 7; ++a) xn += S.x[a] * S.x[a];
-    }
-    for (int a = 0; a < 6; ++a) dn += dx[a] * dx[a];
-    S.xn = sqrt(xn);
-    S.dn = sqrt(dn);
-    if (cfg.param == 1) {
-      for (int a = 0; a < 6; ++a) S.aae[a] = S.aa[a] + dx[a];
-      double qn[4];
-      aa_to_quat(S.aae + 3, qn);
-      for (int a = 0; a < 3; ++a) S.xe[a] = S.aae[a];
-      for (int a = 0; a < 4; ++a) S.xe[3 + a] = qn[a];
-    } else {
-      for (int a = 0; a < 3; ++a) S.xe[a] = S.x[a] + dx[a];
-      double qn[4];
-      quat_left_update(S.x + 3, dx + 3, qn);
-      for (int a = 0; a < 4; ++a) S.xe[3 + a] = qn[a];
+#pragma unroll
+    for (int i = 5; i >= 0; --i) {
+      double t = sl_lane_value(L[i], 6);
+#pragma unroll
+      for (int k = i + 1; k < 6; ++k) t = t - sl_lane_value(L[i], k) * dx[k];
+      dx[i] = t / diag[i];
     }
     have_candidate = true;
     break;
   }
-  S.phase = 1;
-  if (!have_candidate) S.done = 1;
+  if (have_candidate) {
+    double gdx = 0.0, dAd = 0.0, rowdot = 0.0, xn = 0.0, dn = 0.0;
+#pragma unroll
+    for (int b = 0; b < 6; ++b) rowdot += arow[b] * dx[b];
+#pragma unroll
+    for (int a = 0; a < 6; ++a) {
+      gdx += g[a] * dx[a];
+      dAd += dx[a] * sl_lane_value(rowdot, a);
+      dn += dx[a] * dx[a];
+    }
+    double xe[7], aae[6];
+    if (cfg.param == 1) {
+#pragma unroll
+      for (int a = 0; a < 6; ++a) {
+        xn += S.aa[a] * S.aa[a];
+        aae[a] = S.aa[a] + dx[a];
+      }
+#pragma unroll
+      for (int a = 0; a < 3; ++a) xe[a] = aae[a];
+      aa_to_quat(aae + 3, xe + 3);
+    } else {
+      double q[4];
+#pragma unroll
+      for (int a = 0; a < 7; ++a) xn += S.x[a] * S.x[a];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) xe[a] = S.x[a] + dx[a];
+#pragma unroll
+      for (int a = 0; a < 4; ++a) q[a] = S.x[3 + a];
+      quat_left_update(q, dx + 3, xe + 3);
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int a = 0; a < 7; ++a) S.xe[a] = xe[a];
+      if (cfg.param == 1) {
+#pragma unroll
+        for (int a = 0; a < 6; ++a) S.aae[a] = aae[a];
+      }
+      S.model = -(gdx + 0.5 * dAd);
+      S.xn = sqrt(xn);
+      S.dn = sqrt(dn);
+    }
+  }
+  if (lane == 0) {
+    S.F = F;
+    S.F0 = F0;
+    S.radius = radius;
+    S.factor = factor;
+    S.term = term;
+    S.iter = iter;
+    S.phase = 1;
+    if (!have_candidate) S.done = 1;
+  }
+  wave_fence();
 }
 
 __device__ inline void write_outputs(const LMState& S, int k, const PoseCfgDev& cfg,
@@ -850,59 +865,112 @@ __device__ inline void write_outputs(const LMState& S, int k, const PoseCfgDev& 
   }
 }
 
-// FP64 chunk sums in chunk order, one wave per problem
+// The chunks' sums of problem k added in chunk order into tot, by one wave;
+// loaded eight at a time so that the loads overlap.
+__device__ inline void chunk_total(const int32_t* __restrict__ first_work,
+                                   const double* __restrict__ partials, int k, double* tot) {
+  const int lane = threadIdx.x & 63;
+  if (lane >= kSums) return;
+  double s = 0.0;
+  const int w0 = first_work[k], w1 = first_work[k + 1];
+  for (int wk = w0; wk < w1; wk += 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      v[u] = wk + u < w1 ? partials[(size_t)(wk + u) * kSums + lane] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (wk + u < w1) s += v[u];
+  }
+  tot[lane] = s;
+}
+
+// State copies by one wave (8-byte words).
+static_assert(sizeof(LMState) % 8 == 0, "LMState is copied in 8-byte words");
+__device__ inline void copy_state(LMState* __restrict__ dst, const LMState* __restrict__ src) {
+  const double* a = reinterpret_cast<const double*>(src);
+  double* b = reinterpret_cast<double*>(dst);
+  for (int i = threadIdx.x & 63; i < (int)(sizeof(LMState) / 8); i += 64) b[i] = a[i];
+}
+
+// work item = {problem, first residual, end residual, unused}.  prev_partials
+// (nullable): the previous evaluation's; its LM step is made here, by every
+// workgroup of the problem alike, instead of in a kernel between the two
+// evaluations, and the problem's first workgroup writes the state to st_out
+// (64 problems of 31000 residuals: 16.3 us an iteration for 12.8 + 9).
+template <bool F64>
+__global__ __launch_bounds__(kPBlock) void pose_eval_kernel(
+    const float4* __restrict__ pts, const int4* __restrict__ work,
+    const int32_t* __restrict__ first_work, const LMState* __restrict__ st,
+    const double* __restrict__ prev_partials, LMState* __restrict__ st_out,
+    const void* __restrict__ cyl_tab, const void* __restrict__ pl_tab, PoseCfgDev cfg,
+    double* __restrict__ partials) {
+  using E = PoseEval<F64>;
+  __shared__ typename E::Red red;
+  __shared__ LMState S;
+  __shared__ double tot[kSums];
+  const int4 w = work[blockIdx.x];
+  const int k = w.x;
+  if (threadIdx.x < 64) {
+    copy_state(&S, st + k);
+    if (prev_partials) {
+      chunk_total(first_work, prev_partials, k, tot);
+      wave_fence();
+      if (!S.done) lm_step(S, tot, cfg);
+      if ((int)blockIdx.x == first_work[k]) copy_state(st_out + k, &S);
+    }
+  }
+  __syncthreads();
+  if (S.done) return;
+  typename E::Frame F;
+  E::frame(S, cfg.param, F);
+  const double p = E::chunk(pts, w.y, w.z, F, cyl_tab, pl_tab, cfg.delta, red);
+  if (threadIdx.x < kSums) partials[(size_t)blockIdx.x * kSums + threadIdx.x] = p;
+}
+
+// The LM step of the last evaluation and the outputs (or, between evaluations,
+// only the step: pose_out null), one wave per problem.
 __global__ __launch_bounds__(64) void pose_solve_kernel(
     int n_problems, const int32_t* __restrict__ first_work, const double* __restrict__ partials,
     PoseCfgDev cfg, LMState* __restrict__ st, double* __restrict__ pose_out,
     int32_t* __restrict__ status, double* __restrict__ cost, double* __restrict__ params_out) {
   __shared__ double tot[kSums];
+  __shared__ LMState S;
   const int k = blockIdx.x;
   if (k >= n_problems) return;
-  if (st[k].done) return;
-  if (threadIdx.x < kSums) {
-    // the chunks' sums added in chunk order; loaded eight at a time so that
-    // the loads overlap
-    double s = 0.0;
-    const int w0 = first_work[k], w1 = first_work[k + 1];
-    for (int wk = w0; wk < w1; wk += 8) {
-      double v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        v[u] = wk + u < w1 ? partials[(size_t)(wk + u) * kSums + threadIdx.x] : 0.0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (wk + u < w1) s += v[u];
-    }
-    tot[threadIdx.x] = s;
+  copy_state(&S, st + k);
+  chunk_total(first_work, partials, k, tot);
+  wave_fence();
+  if (!S.done) {
+    lm_step(S, tot, cfg);
+    copy_state(st + k, &S);
   }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  LMState S = st[k];
-  lm_step(S, tot, cfg);
-  st[k] = S;
-  write_outputs(S, k, cfg, pose_out, status, cost, params_out);
+  if (pose_out && threadIdx.x == 0) write_outputs(S, k, cfg, pose_out, status, cost, params_out);
 }
 
 // --------------------------------------------------------------------------
 // fused: every iteration of one problem in one workgroup
 // --------------------------------------------------------------------------
+// d_n_problems (nullable): the problem count in device memory (a grid of
+// n_problems workgroups then serves any count up to n_problems).  The landmark
+// tables are written here and read back (no __restrict__): a preparation
+// launch of its own was 4.7 us and the gap after it.
 template <bool F64>
 __global__ __launch_bounds__(kPBlock) void pose_fused_kernel(
-    int n_problems, const int32_t* __restrict__ d_n_problems, const float4* __restrict__ pts,
-    const int4* __restrict__ work, const int32_t* __restrict__ first_work,
-    const void* __restrict__ cyl_tab, const void* __restrict__ pl_tab, PoseCfgDev cfg,
-    LMState* __restrict__ st, double* __restrict__ pose_out, int32_t* __restrict__ status,
-    double* __restrict__ cost, double* __restrict__ params_out) {
+    int n_problems, const int32_t* __restrict__ d_n_problems, PoseIn in,
+    const float4* __restrict__ pts, const int4* __restrict__ work,
+    const int32_t* __restrict__ first_work, void* cyl_tab, void* pl_tab, PoseCfgDev cfg,
+    double* __restrict__ pose_out, int32_t* __restrict__ status, double* __restrict__ cost,
+    double* __restrict__ params_out) {
   using E = PoseEval<F64>;
   __shared__ typename E::Red red;
   __shared__ double tot[kSums];
   __shared__ LMState sS;
   const int k = blockIdx.x;
   if (k >= n_problems || (d_n_problems && k >= *d_n_problems)) return;
-  if (threadIdx.x == 0) sS = st[k];
+  pose_prep<F64>(k, in, cfg, &sS, cyl_tab, pl_tab);
   __syncthreads();
   const int w0 = first_work[k], w1 = first_work[k + 1];
-  bool ran = false;
   for (int it = 0; it <= cfg.max_iters; ++it) {
     if (sS.done) break;
     typename E::Frame F;
@@ -915,19 +983,10 @@ __global__ __launch_bounds__(kPBlock) void pose_fused_kernel(
     }
     if (threadIdx.x < kSums) tot[threadIdx.x] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) {
-      LMState S = sS;
-      lm_step(S, tot, cfg);
-      sS = S;
-    }
-    ran = true;
+    if (threadIdx.x < 64) lm_step(sS, tot, cfg);
     __syncthreads();
   }
-  if (threadIdx.x == 0 && ran) {
-    const LMState S = sS;
-    st[k] = S;
-    write_outputs(S, k, cfg, pose_out, status, cost, params_out);
-  }
+  if (threadIdx.x == 0) write_outputs(sS, k, cfg, pose_out, status, cost, params_out);
 }
 
 }  // namespace
@@ -958,6 +1017,14 @@ namespace {
 // a problem set whose largest problem has at most this many chunks is solved
 // by pose_fused in AUTO mode
 constexpr int kFusedAutoChunks = 8;
+// The evaluations make the LM steps themselves where all their workgroups run
+// at once (four a CU, so the step's latency is paid once) and a problem has
+// few chunks (every workgroup sums its problem's).  10 iterations, joint
+// against two kernels: 64 problems of 16 chunks 179 / 194 us, 4 of 103
+// 186 / 199, 1 of 293 308 / 319; 16 of 126 (2016 workgroups) 489 / 385, 2 of
+// 586 1004 / 612.
+constexpr int kJointBlocks = 1024;
+constexpr int kJointChunks = 256;
 
 int grow(sloam_ctx* ctx, void** p, size_t* cap, size_t want, size_t elem) {
   if (want <= *cap) return SLOAM_OK;
@@ -1001,9 +1068,10 @@ int plan_build(sloam_pose_plan* p, const int32_t* h_res_offsets, int32_t n_probl
   p->n_work = (int)p->h_work.size();
   int st = grow(ctx, (void**)&p->d_work, &p->cap_work, p->h_work.size(), sizeof(int4));
   if (!st) st = grow(ctx, (void**)&p->d_first, &p->cap_first, p->h_first.size(), sizeof(int32_t));
-  if (!st) st = grow(ctx, (void**)&p->d_state, &p->cap_state, (size_t)n_problems, sizeof(LMState));
   if (!st)
-    st = grow(ctx, (void**)&p->d_partials, &p->cap_partials, (size_t)kSums * p->h_work.size(),
+    st = grow(ctx, (void**)&p->d_state, &p->cap_state, 2 * (size_t)n_problems, sizeof(LMState));
+  if (!st)
+    st = grow(ctx, (void**)&p->d_partials, &p->cap_partials, 2 * (size_t)kSums * p->h_work.size(),
               sizeof(double));
   // landmark table entries: 2 float4 / 2 double4 per cylinder, 1 per plane
   const size_t tab = p->cfg.precision == 1 ? sizeof(double4) : sizeof(float4);
@@ -1043,30 +1111,16 @@ static PoseCfgDev pose_cfg_dev(const sloam_pose_cfg& c) {
   return dc;
 }
 
-size_t sloam_pose_state_bytes() { return sizeof(LMState); }
-
 namespace {
 
-// pose_prep + pose_fused of one precision
 template <bool F64>
-void launch_prep(sloam_ctx* ctx, int grid, int n_problems, const int32_t* d_n_problems,
-                 const double* d_pose_in, const int32_t* d_free_mask, const double* d_cyl,
-                 const int32_t* d_cyl_off, const double* d_planes, const int32_t* d_pl_off,
-                 const PoseCfgDev& dc, LMState* st, void* cyl_tab, void* pl_tab) {
-  hipLaunchKernelGGL(pose_prep_kernel<F64>, dim3(grid), dim3(kPBlock), 0, ctx->stream,
-                     n_problems, d_n_problems, d_pose_in, d_free_mask, d_cyl, d_cyl_off, d_planes,
-                     d_pl_off, dc, st, cyl_tab, pl_tab);
-}
-
-template <bool F64>
-void launch_fused(sloam_ctx* ctx, int grid, int n_problems, const int32_t* d_n_problems,
+void launch_fused(sloam_ctx* ctx, int grid, const int32_t* d_n_problems, const PoseIn& in,
                   const float* d_points, const int4* d_work, const int32_t* d_first,
-                  const void* cyl_tab, const void* pl_tab, const PoseCfgDev& dc, LMState* st,
-                  double* d_pose_out, int32_t* d_status, double* d_cost, double* d_params_out) {
-  hipLaunchKernelGGL(pose_fused_kernel<F64>, dim3(grid), dim3(kPBlock), 0, ctx->stream,
-                     n_problems, d_n_problems, reinterpret_cast<const float4*>(d_points), d_work,
-                     d_first, cyl_tab, pl_tab, dc, st, d_pose_out, d_status, d_cost,
-                     d_params_out);
+                  void* cyl_tab, void* pl_tab, const PoseCfgDev& dc, double* d_pose_out,
+                  int32_t* d_status, double* d_cost, double* d_params_out) {
+  hipLaunchKernelGGL(pose_fused_kernel<F64>, dim3(grid), dim3(kPBlock), 0, ctx->stream, grid,
+                     d_n_problems, in, reinterpret_cast<const float4*>(d_points), d_work, d_first,
+                     cyl_tab, pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
 }
 
 }  // namespace
@@ -1075,27 +1129,17 @@ int sloam_pose_fused_device(sloam_ctx* ctx, int max_problems, const int32_t* d_n
                             const float* d_points, const int32_t* d_work, const int32_t* d_first,
                             const double* d_cyl, const int32_t* d_cyl_off, const double* d_planes,
                             const int32_t* d_pl_off, const double* d_pose_in,
-                            const int32_t* d_free_mask, const sloam_pose_cfg* cfg, void* d_state,
+                            const int32_t* d_free_mask, const sloam_pose_cfg* cfg,
                             void* d_cyl_tab, void* d_pl_tab, double* d_pose_out,
                             double* d_params_out, int32_t* d_status, double* d_cost) {
   if (max_problems <= 0) return SLOAM_OK;
   if (!valid_cfg(cfg)) return SLOAM_ERR_INVALID_ARG;
   const PoseCfgDev dc = pose_cfg_dev(*cfg);
-  LMState* st = static_cast<LMState*>(d_state);
+  const PoseIn in{d_pose_in, d_free_mask, d_cyl, d_cyl_off, d_planes, d_pl_off};
   const int4* work = reinterpret_cast<const int4*>(d_work);
-  if (cfg->precision == 1) {
-    launch_prep<true>(ctx, max_problems, max_problems, d_n_problems, d_pose_in, d_free_mask, d_cyl,
-                      d_cyl_off, d_planes, d_pl_off, dc, st, d_cyl_tab, d_pl_tab);
-    SLOAM_HIP(ctx, hipGetLastError());
-    launch_fused<true>(ctx, max_problems, max_problems, d_n_problems, d_points, work, d_first,
-                       d_cyl_tab, d_pl_tab, dc, st, d_pose_out, d_status, d_cost, d_params_out);
-  } else {
-    launch_prep<false>(ctx, max_problems, max_problems, d_n_problems, d_pose_in, d_free_mask,
-                       d_cyl, d_cyl_off, d_planes, d_pl_off, dc, st, d_cyl_tab, d_pl_tab);
-    SLOAM_HIP(ctx, hipGetLastError());
-    launch_fused<false>(ctx, max_problems, max_problems, d_n_problems, d_points, work, d_first,
-                        d_cyl_tab, d_pl_tab, dc, st, d_pose_out, d_status, d_cost, d_params_out);
-  }
+  auto launch = cfg->precision == 1 ? launch_fused<true> : launch_fused<false>;
+  launch(ctx, max_problems, d_n_problems, in, d_points, work, d_first, d_cyl_tab, d_pl_tab, dc,
+         d_pose_out, d_status, d_cost, d_params_out);
   SLOAM_HIP(ctx, hipGetLastError());
   return SLOAM_OK;
 }
@@ -1175,47 +1219,47 @@ int sloam_pose_plan_exec(sloam_pose_plan* p, const float* d_points, const double
   const sloam_pose_cfg& c = p->cfg;
   const PoseCfgDev dc = pose_cfg_dev(c);
   const bool f64 = c.precision == 1;
-  {
-    SloamKernelScope ks(ctx, "pose_prep");
-    if (f64)
-      launch_prep<true>(ctx, p->n_problems, p->n_problems, nullptr, d_pose_in, d_free_mask, d_cyl,
-                        d_cyl_offsets, d_planes, d_plane_offsets, dc, p->d_state, p->d_cyl_tab,
-                        p->d_pl_tab);
-    else
-      launch_prep<false>(ctx, p->n_problems, p->n_problems, nullptr, d_pose_in, d_free_mask,
-                         d_cyl, d_cyl_offsets, d_planes, d_plane_offsets, dc, p->d_state,
-                         p->d_cyl_tab, p->d_pl_tab);
-  }
-  SLOAM_HIP(ctx, hipGetLastError());
+  const PoseIn in{d_pose_in, d_free_mask, d_cyl, d_cyl_offsets, d_planes, d_plane_offsets};
   if (sloam_pose_plan_uses_fused(p)) {
     SloamKernelScope ks(ctx, "pose_fused");
-    if (f64)
-      launch_fused<true>(ctx, p->n_problems, p->n_problems, nullptr, d_points, p->d_work,
-                         p->d_first, p->d_cyl_tab, p->d_pl_tab, dc, p->d_state, d_pose_out,
-                         d_status, d_cost, d_params_out);
-    else
-      launch_fused<false>(ctx, p->n_problems, p->n_problems, nullptr, d_points, p->d_work,
-                          p->d_first, p->d_cyl_tab, p->d_pl_tab, dc, p->d_state, d_pose_out,
-                          d_status, d_cost, d_params_out);
+    auto launch = f64 ? launch_fused<true> : launch_fused<false>;
+    launch(ctx, p->n_problems, nullptr, in, d_points, p->d_work, p->d_first, p->d_cyl_tab,
+           p->d_pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
     SLOAM_HIP(ctx, hipGetLastError());
     return SLOAM_OK;
   }
+  {
+    SloamKernelScope ks(ctx, "pose_prep");
+    auto kern = f64 ? pose_prep_kernel<true> : pose_prep_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3(p->n_problems), dim3(kPBlock), 0, ctx->stream, p->n_problems,
+                       in, dc, p->d_state, p->d_cyl_tab, p->d_pl_tab);
+  }
+  SLOAM_HIP(ctx, hipGetLastError());
+  // an evaluation makes the step of the one before it, from the other halves
+  // of the state and partials buffers
+  const bool joint = p->n_work <= kJointBlocks && p->max_chunks <= kJointChunks;
+  auto half = [&](int it) { return joint && (it & 1) ? 1 : 0; };
+  auto state = [&](int it) { return p->d_state + (size_t)half(it) * p->n_problems; };
+  auto partials = [&](int it) { return p->d_partials + (size_t)half(it) * kSums * p->n_work; };
   for (int it = 0; it <= c.max_iters; ++it) {
+    const bool step = joint && it > 0;
     {
       SloamKernelScope ks(ctx, "pose_eval");
       auto kern = f64 ? pose_eval_kernel<true> : pose_eval_kernel<false>;
       hipLaunchKernelGGL(kern, dim3(p->n_work), dim3(kPBlock), 0, ctx->stream,
-                         reinterpret_cast<const float4*>(d_points), p->d_work, p->d_state,
+                         reinterpret_cast<const float4*>(d_points), p->d_work, p->d_first,
+                         step ? state(it - 1) : state(it),
+                         step ? partials(it - 1) : static_cast<const double*>(nullptr), state(it),
                          static_cast<const void*>(p->d_cyl_tab),
-                         static_cast<const void*>(p->d_pl_tab), c.huber_delta, c.parametrization,
-                         p->d_partials);
+                         static_cast<const void*>(p->d_pl_tab), dc, partials(it));
     }
     SLOAM_HIP(ctx, hipGetLastError());
+    if (joint && it < c.max_iters) continue;
     {
       SloamKernelScope ks(ctx, "pose_solve");
       hipLaunchKernelGGL(pose_solve_kernel, dim3(p->n_problems), dim3(64), 0, ctx->stream,
-                         p->n_problems, p->d_first, p->d_partials, dc, p->d_state, d_pose_out,
-                         d_status, d_cost, d_params_out);
+                         p->n_problems, p->d_first, partials(it), dc, state(it),
+                         it == c.max_iters ? d_pose_out : nullptr, d_status, d_cost, d_params_out);
     }
     SLOAM_HIP(ctx, hipGetLastError());
   }

@@ -142,6 +142,21 @@ def test_fused_matches_batched_bitwise(ctx, name, make, kw, precision):
         assert np.array_equal(b[k], f[k]), k
 
 
+@pytest.mark.parametrize("problems,n_cyl,n_planes,chunks", [
+    (1, 8735, 3, 256), (1, 8735, 4, 257), (204, 150, 1, 1020), (205, 150, 1, 1025)])
+def test_joint_step_limits(ctx, problems, n_cyl, n_planes, chunks):
+    """On both sides of the limits up to which an evaluation makes the LM step
+    of the one before it (256 chunks a problem, 1024 in all): the one-launch
+    kernel's bits."""
+    prob = synth.make_pose_problems(problems, n_cyl=n_cyl, n_planes=n_planes, seed=38)
+    assert int(np.sum(-(-np.diff(prob["res_offsets"]) // 2048))) == chunks
+    for kw in (dict(max_iters=0), dict(max_iters=3), dict(max_iters=12, stop_on_convergence=True)):
+        b = solve_poses(ctx, prob, mode=1, **kw)
+        f = solve_poses(ctx, prob, mode=2, **kw)
+        for k in ("pose", "params", "status", "cost"):
+            assert np.array_equal(b[k], f[k]), (k, kw)
+
+
 def test_auto_mode_choice(ctx):
     import torch
     from sloam_amd.gpu import PosePlan
