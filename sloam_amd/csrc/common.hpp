@@ -354,8 +354,46 @@ __device__ inline double sl_wave_sum(double v) {
   return v;
 }
 
+// One step of a wave reduction: the value of the lane that `kCtrl` names (a
+// DPP row shift or row broadcast), `none` where there is none.
+template <int kCtrl, int kRows>
+__device__ inline int sl_dpp(int none, int v) {
+  return __builtin_amdgcn_update_dpp(none, v, kCtrl, kRows, 0xf, false);
+}
+
+// Sums, minima and maxima over a wave, on every lane: row shifts by 1, 2, 4, 8,
+// then the rows' last lanes broadcast; lane 63 ends with all of them.  These
+// run on the SIMDs; shuffles go through the LDS unit, which a CU has once
+// (nine 64-bit sums of every wave kept it busy for 3k cycles a workgroup).
+template <int kCtrl, int kRows>
+__device__ inline long long sl_dpp_add(long long v) {
+  const int lo = sl_dpp<kCtrl, kRows>(0, (int)v), hi = sl_dpp<kCtrl, kRows>(0, (int)(v >> 32));
+  return v + (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
+}
+
 __device__ inline long long sl_wave_sum_i64(long long v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v = sl_dpp_add<0x111, 0xf>(v);
+  v = sl_dpp_add<0x112, 0xf>(v);
+  v = sl_dpp_add<0x114, 0xf>(v);
+  v = sl_dpp_add<0x118, 0xf>(v);
+  v = sl_dpp_add<0x142, 0xa>(v);
+  v = sl_dpp_add<0x143, 0xc>(v);
+  const int lo = __builtin_amdgcn_readlane((int)v, 63);
+  const int hi = __builtin_amdgcn_readlane((int)(v >> 32), 63);
+  return (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
+}
+
+template <bool kMax>
+__device__ inline float sl_wave_extreme(float v) {
+  auto step = [&](int other) {
+    const float o = __int_as_float(other);
+    v = kMax ? fmaxf(v, o) : fminf(v, o);
+  };
+  step(sl_dpp<0x111, 0xf>(__float_as_int(v), __float_as_int(v)));
+  step(sl_dpp<0x112, 0xf>(__float_as_int(v), __float_as_int(v)));
+  step(sl_dpp<0x114, 0xf>(__float_as_int(v), __float_as_int(v)));
+  step(sl_dpp<0x118, 0xf>(__float_as_int(v), __float_as_int(v)));
+  step(sl_dpp<0x142, 0xa>(__float_as_int(v), __float_as_int(v)));
+  step(sl_dpp<0x143, 0xc>(__float_as_int(v), __float_as_int(v)));
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }

@@ -39,6 +39,10 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kHB = 8;  // hypotheses held in registers per pass over a tile
+constexpr int kSeedPts = 8;  // points of a thread in flight in cyl_seed
+// clusters from which on the seed axes have a launch of their own (200: 122 us
+// for 121 without, 500: 123 / 125, 1200: 127 / 132, 4096: 589 / 606)
+constexpr int kAxisClusters = 384;
 constexpr int kScoreFill = 2048;  // score workgroups that fill the chip (8 a CU)
 constexpr int kMaxLds = 65536;  // LDS bytes per workgroup this kernel asks for
 
@@ -161,101 +165,9 @@ __device__ inline const float* cluster_prop(const float* prop, int c) {
   return q[7] > 0.0f ? q : nullptr;
 }
 
-// order (nullable): the cluster of each workgroup, -1 for padding (the plans'
-// largest-first order dealt to the XCDs as the scoring work list deals them,
-// so a cluster's points are read through the L2 its scoring will read them
-// through); without it workgroup b seeds cluster b
-__global__ __launch_bounds__(kBlock) void cyl_seed_kernel(const float* __restrict__ xyz,
-                                                          const int32_t* __restrict__ offsets,
-                                                          int n_clusters,
-                                                          const int32_t* __restrict__ active,
-                                                          const int32_t* __restrict__ bcnt,
-                                                          CylFrame* __restrict__ frames,
-                                                          const int32_t* __restrict__ order) {
-  __shared__ float red_f[kWaves][6];
-  __shared__ long long red_i[kWaves][9];
-  const int c = order ? order[blockIdx.x] : (int)blockIdx.x;
-  if (c < 0 || c >= n_clusters || (bcnt && c >= bcnt[0])) return;
-  if (active && !active[c]) return;
-  const int off = offsets[c];
-  const int n = offsets[c + 1] - off;
-  const float* P = xyz + 3 * (size_t)off;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-
-  float mn[3] = {INFINITY, INFINITY, INFINITY};
-  float mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-  for (int i = threadIdx.x; i < n; i += kBlock) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const float q = P[3 * (size_t)i + k];
-      mn[k] = fminf(mn[k], q);
-      mx[k] = fmaxf(mx[k], q);
-    }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      mn[k] = fminf(mn[k], __shfl_xor(mn[k], o, 64));
-      mx[k] = fmaxf(mx[k], __shfl_xor(mx[k], o, 64));
-    }
-  }
-  if (lane == 0) {
-    for (int k = 0; k < 3; ++k) {
-      red_f[wave][k] = mn[k];
-      red_f[wave][3 + k] = mx[k];
-    }
-  }
-  __syncthreads();
-  float m[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    float a = red_f[0][k], b = red_f[0][3 + k];
-    for (int w = 1; w < kWaves; ++w) {
-      a = fminf(a, red_f[w][k]);
-      b = fmaxf(b, red_f[w][3 + k]);
-    }
-    m[k] = n > 0 ? 0.5f * (a + b) : 0.0f;
-  }
-
-  // integer-exact sums of q = rint((p - m) * 2^16), |q| < 2^23
-  long long s[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  for (int i = threadIdx.x; i < n; i += kBlock) {
-    long long q[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      double d = ((double)P[3 * (size_t)i + k] - (double)m[k]) * 65536.0;
-      d = rint(d);
-      if (d > 8388607.0) d = 8388607.0;
-      if (d < -8388607.0) d = -8388607.0;
-      q[k] = (long long)d;
-    }
-    s[0] += q[0];
-    s[1] += q[1];
-    s[2] += q[2];
-    s[3] += q[0] * q[0];
-    s[4] += q[0] * q[1];
-    s[5] += q[0] * q[2];
-    s[6] += q[1] * q[1];
-    s[7] += q[1] * q[2];
-    s[8] += q[2] * q[2];
-  }
-#pragma unroll
-  for (int k = 0; k < 9; ++k) s[k] = sl_wave_sum_i64(s[k]);
-  if (lane == 0)
-    for (int k = 0; k < 9; ++k) red_i[wave][k] = s[k];
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  long long t[9];
-  for (int k = 0; k < 9; ++k) {
-    t[k] = red_i[0][k];
-    for (int w = 1; w < kWaves; ++w) t[k] += red_i[w][k];
-  }
-  CylFrame f;
-  f.m[0] = m[0];
-  f.m[1] = m[1];
-  f.m[2] = m[2];
+// Axis and basis of n points from the sums t of their quantised offsets and
+// of the products (xx, xy, xz, yy, yz, zz).
+__device__ inline void seed_axis(const long long (&t)[9], int n, CylFrame& f) {
   f.n = n;
   f.reserved = 0.0;
   double axis[3] = {0.0, 0.0, 1.0};
@@ -280,6 +192,146 @@ __global__ __launch_bounds__(kBlock) void cyl_seed_kernel(const float* __restric
     f.e1[k] = (float)e1[k];
     f.e2[k] = (float)e2[k];
   }
+}
+
+// Two passes over the points, kSeedPts of them in flight a thread (one pass
+// over memory up to 2048 points), then the eigen-solver, a serial chain of
+// about 7 us: sums (nullable) takes the sums instead, and cyl_axis solves a
+// large batch a lane each.  13.5e6 points in 1500 clusters (162 MB, the larger
+// ones read twice): 121 us with a point in flight and 64-bit products, 66 now;
+// 4096 clusters, 4.4e6 points: 59 -> 37; a keyframe's 12: 11.7 -> 9.
+//
+// order (nullable): the cluster of each workgroup, -1 for padding (the plans'
+// largest-first order dealt to the XCDs as the scoring work list deals them,
+// so a cluster's points are read through the L2 its scoring will read them
+// through); without it workgroup b seeds cluster b
+__global__ __launch_bounds__(kBlock) void cyl_seed_kernel(const float* __restrict__ xyz,
+                                                          const int32_t* __restrict__ offsets,
+                                                          int n_clusters,
+                                                          const int32_t* __restrict__ active,
+                                                          const int32_t* __restrict__ bcnt,
+                                                          CylFrame* __restrict__ frames,
+                                                          long long* __restrict__ sums,
+                                                          const int32_t* __restrict__ order) {
+  __shared__ float red_f[kWaves][6];
+  __shared__ long long red_i[kWaves][9];
+  const int c = order ? order[blockIdx.x] : (int)blockIdx.x;
+  if (c < 0 || c >= n_clusters || (bcnt && c >= bcnt[0])) return;
+  if (active && !active[c]) return;
+  const int off = offsets[c];
+  const int n = offsets[c + 1] - off;
+  const float* P = xyz + 3 * (size_t)off;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+
+  float mn[3] = {INFINITY, INFINITY, INFINITY};
+  float mx[3] = {-INFINITY, -INFINITY, -INFINITY};
+  float px[kSeedPts][3];
+  // points first + kBlock j + thread; past the end the last point again
+  auto load = [&](int first) {
+#pragma unroll
+    for (int j = 0; j < kSeedPts; ++j) {
+      const float* q = P + 3 * (size_t)min(first + kBlock * j + (int)threadIdx.x, n - 1);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) px[j][k] = q[k];
+    }
+  };
+  for (int first = 0; first < n; first += kBlock * kSeedPts) {
+    load(first);
+#pragma unroll
+    for (int j = 0; j < kSeedPts; ++j)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        mn[k] = fminf(mn[k], px[j][k]);
+        mx[k] = fmaxf(mx[k], px[j][k]);
+      }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    mn[k] = sl_wave_extreme<false>(mn[k]);
+    mx[k] = sl_wave_extreme<true>(mx[k]);
+  }
+  if (lane == 0) {
+    for (int k = 0; k < 3; ++k) {
+      red_f[wave][k] = mn[k];
+      red_f[wave][3 + k] = mx[k];
+    }
+  }
+  __syncthreads();
+  float m[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    float a = red_f[0][k], b = red_f[0][3 + k];
+    for (int w = 1; w < kWaves; ++w) {
+      a = fminf(a, red_f[w][k]);
+      b = fmaxf(b, red_f[w][3 + k]);
+    }
+    m[k] = n > 0 ? 0.5f * (a + b) : 0.0f;
+  }
+
+  // integer-exact sums of q = rint((p - m) * 2^16), |q| < 2^23
+  long long s[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  for (int first = 0; first < n; first += kBlock * kSeedPts) {
+    if (n > kBlock * kSeedPts) load(first);
+    int32_t s1[3] = {0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < kSeedPts; ++j) {
+      if (first + kBlock * j >= n) break;
+      int32_t q[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        double d = rint(((double)px[j][k] - (double)m[k]) * 65536.0);
+        if (d > 8388607.0) d = 8388607.0;
+        if (d < -8388607.0) d = -8388607.0;
+        q[k] = first + kBlock * j + (int)threadIdx.x < n ? (int32_t)d : 0;
+        s1[k] += q[k];
+      }
+      s[3] += (int64_t)q[0] * q[0];
+      s[4] += (int64_t)q[0] * q[1];
+      s[5] += (int64_t)q[0] * q[2];
+      s[6] += (int64_t)q[1] * q[1];
+      s[7] += (int64_t)q[1] * q[2];
+      s[8] += (int64_t)q[2] * q[2];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) s[k] += s1[k];
+  }
+#pragma unroll
+  for (int k = 0; k < 9; ++k) s[k] = sl_wave_sum_i64(s[k]);
+  if (lane == 0)
+    for (int k = 0; k < 9; ++k) red_i[wave][k] = s[k];
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  long long t[9];
+  for (int k = 0; k < 9; ++k) {
+    t[k] = red_i[0][k];
+    for (int w = 1; w < kWaves; ++w) t[k] += red_i[w][k];
+  }
+  if (sums) {
+    CylFrame& f = frames[c];
+    for (int k = 0; k < 3; ++k) f.m[k] = m[k];
+    for (int k = 0; k < 9; ++k) sums[9 * (size_t)c + k] = t[k];
+    return;
+  }
+  CylFrame f;
+  for (int k = 0; k < 3; ++k) f.m[k] = m[k];
+  seed_axis(t, n, f);
+  frames[c] = f;
+}
+
+// The axes of a batch whose sums cyl_seed left in `sums`, a lane per cluster.
+__global__ __launch_bounds__(64) void cyl_axis_kernel(const int32_t* __restrict__ offsets,
+                                                      int n_clusters,
+                                                      const int32_t* __restrict__ active,
+                                                      const long long* __restrict__ sums,
+                                                      CylFrame* __restrict__ frames) {
+  const int c = blockIdx.x * 64 + (int)threadIdx.x;
+  if (c >= n_clusters || (active && !active[c])) return;
+  long long t[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) t[k] = sums[9 * (size_t)c + k];
+  CylFrame f = frames[c];
+  seed_axis(t, offsets[c + 1] - offsets[c], f);
   frames[c] = f;
 }
 
@@ -1531,6 +1583,25 @@ struct sloam_cyl_plan {
 
 static int round_up(int x, int m) { return (x + m - 1) / m * m; }
 
+// Launches the axis seeds of plan p.  The sums of a large batch pass through
+// the refit states' memory, which the refit writes later.
+static void launch_seed(sloam_cyl_plan* p, const float* d_xyz, const int32_t* d_offsets,
+                        const int32_t* d_active) {
+  hipStream_t stream = p->ctx->stream;
+  const bool ord = !p->counted && p->n_seed > 0;
+  static_assert(sizeof(RefitState) >= 9 * sizeof(long long), "sums fit the refit states");
+  long long* sums = !p->counted && p->n_clusters >= kAxisClusters
+                        ? reinterpret_cast<long long*>(p->d_state)
+                        : nullptr;
+  hipLaunchKernelGGL(cyl_seed_kernel, dim3(ord ? p->n_seed : p->n_clusters), dim3(kBlock), 0,
+                     stream, d_xyz, d_offsets, p->n_clusters, d_active,
+                     p->counted ? p->d_cnt : nullptr, p->d_frames, sums,
+                     ord ? p->d_seed_order : nullptr);
+  if (sums)
+    hipLaunchKernelGGL(cyl_axis_kernel, dim3((p->n_clusters + 63) / 64), dim3(64), 0, stream,
+                       d_offsets, p->n_clusters, d_active, sums, p->d_frames);
+}
+
 // Launches the refit of plan p: one team per cluster, and for the large
 // clusters the init pass, one launch per Gauss-Newton step (as many as the
 // longest schedule among the clusters) and the final pass.
@@ -2078,10 +2149,7 @@ int sloam_cyl_learned_exec(sloam_cyl_plan* verify, sloam_cyl_plan* plain, const 
   {
     // one axis seed per cluster serves both hypothesis sets
     SloamKernelScope ks(ctx, "cyl_seed");
-    const bool ord = !verify->counted && verify->n_seed > 0;
-    hipLaunchKernelGGL(cyl_seed_kernel, dim3(ord ? verify->n_seed : S), dim3(kBlock), 0,
-                       ctx->stream, d_xyz, d_offsets, S, nullptr, vcnt, verify->d_frames,
-                       ord ? verify->d_seed_order : nullptr);
+    launch_seed(verify, d_xyz, d_offsets, nullptr);
   }
   SLOAM_HIP(ctx, hipGetLastError());
   if (verify->n_work > 0) {
@@ -2272,10 +2340,7 @@ int sloam_cyl_plan_exec_ex(sloam_cyl_plan* p, const float* d_xyz, const int32_t*
   }
   {
     SloamKernelScope ks(ctx, "cyl_seed");
-    const bool ord = !p->counted && p->n_seed > 0;
-    hipLaunchKernelGGL(cyl_seed_kernel, dim3(ord ? p->n_seed : p->n_clusters), dim3(kBlock), 0,
-                       ctx->stream, d_xyz, d_offsets, p->n_clusters, d_active, cnt, p->d_frames,
-                       ord ? p->d_seed_order : nullptr);
+    launch_seed(p, d_xyz, d_offsets, d_active);
   }
   SLOAM_HIP(ctx, hipGetLastError());
   if (p->n_work > 0) {
