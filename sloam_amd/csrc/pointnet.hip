@@ -493,20 +493,37 @@ __global__ __launch_bounds__(kFB) void pn_head_kernel(const float* __restrict__ 
 // FP32-level accuracy with FP32 accumulation.
 // ---------------------------------------------------------------------------
 constexpr int kQT = 32;        // active points per tile (the K of one MFMA)
+constexpr int kQB = 8;         // of them whose loads a thread has in flight
 constexpr int kSQ = kQT + 8;   // row stride (bf16) of the [channel][point] tiles
 constexpr int kSJ = kC2 + 8;   // row stride (bf16) of the [point][channel] tiles
 // four waves: wave w owns dz1 channels 16w.. and dW2 rows 32w..; two
 // threads per layer-2 channel fill the dz2 tile
-static_assert(kFB == 256 && kC1 == 4 * 16 && kC2 == 4 * 32 && kFB == 2 * kC2 && kQT == 32,
+static_assert(kFB == 256 && kC1 == 4 * 16 && kC2 == 4 * 32 && kFB == 2 * kC2 && kQT == 32 &&
+                  kQT % (kQB * kFB / kC2) == 0 && kC3 == kFB && kP == 2 * kFB,
               "backward tile layout");
 
+// Four consecutive floats at a 4-byte aligned address (a cluster's gradients
+// start at any multiple of 4 bytes), as one store.
+struct __attribute__((packed, aligned(4))) Float4U {
+  float x, y, z, w;
+};
+__device__ inline void store4(float* p, float x, float y, float z, float w) {
+  *reinterpret_cast<Float4U*>(p) = Float4U{x, y, z, w};
+}
+
+// One workgroup a CU and a wave a SIMD: what it takes is latency.  250
+// clusters: 117 us with the active points and their channels listed by one
+// thread and one gather in flight at a time, 61 now (75 MB of gradients
+// written, 15 us of it).
 __global__ __launch_bounds__(kFB) void pn_bwd_kernel(
     const float* __restrict__ prm, const float4* __restrict__ X, const PnMeta* __restrict__ meta,
     const float* __restrict__ act, const unsigned short* __restrict__ H1,
     const unsigned short* __restrict__ H2, const double* __restrict__ targets, LossCfg lc,
     int n_clusters, float* __restrict__ G, float* __restrict__ loss_out) {
-  __shared__ float f[kC3], dz3[kC3], h4[kC4], dz4[kC4], dout[8];
-  __shared__ int fidx[kC3];
+  __shared__ __align__(16) float f[kC3];
+  __shared__ float dz3[kC3], h4[kC4], dz4[kC4], dout[8];
+  __shared__ __align__(16) int fidx[kC3];
+  __shared__ int wcount[2 * kFB / 64];
   __shared__ int slot_of[kP];
   __shared__ int plist[kC3];
   __shared__ int ccount[kC3 + 1], cstart[kC3 + 1], corder[kC3];
@@ -583,11 +600,16 @@ __global__ __launch_bounds__(kFB) void pn_bwd_kernel(
     dz4[t] = h4[t] > 0.f ? s : 0.f;
   }
   __syncthreads();
-  for (int i = t; i < kC4 * kC3; i += kFB) Gc[kW4 + i] = dz4[i / kC3] * f[i % kC3];
+  for (int i = 4 * t; i < kC4 * kC3; i += 4 * kFB) {
+    const float4 fv = *reinterpret_cast<const float4*>(f + i % kC3);
+    const float z = dz4[i / kC3];
+    store4(Gc + kW4 + i, z * fv.x, z * fv.y, z * fv.z, z * fv.w);
+  }
   if (t < kC4) Gc[kB4 + t] = dz4[t];
   // df, dz3 (the max-pool passes the gradient to the argmax point)
   for (int k = t; k < kC3; k += kFB) {
     float s = 0.f;
+#pragma unroll 16
     for (int o = 0; o < kC4; ++o) s += bf_round(prm[kW4 + o * kC3 + k]) * dz4[o];
     dz3[k] = fidx[k] >= 0 ? s : 0.f;
   }
@@ -596,48 +618,78 @@ __global__ __launch_bounds__(kFB) void pn_bwd_kernel(
   for (int k = t; k < kC3; k += kFB)
     if (fidx[k] >= 0) slot_of[fidx[k]] = 0;
   __syncthreads();
-  if (t == 0) {
-    int s = 0;
-    for (int p = 0; p < kP; ++p)
-      if (slot_of[p] == 0) {
-        slot_of[p] = s;
-        plist[s] = p;
-        ++s;
-      } else {
-        slot_of[p] = -1;
+  const int lane = t & 63, wave = t >> 6;
+  const uint64_t below = (1ull << lane) - 1;
+  {
+    bool on[2];
+    uint64_t b[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      on[u] = slot_of[kFB * u + t] == 0;
+      b[u] = __builtin_amdgcn_ballot_w64(on[u]);
+      if (lane == 0) wcount[kFB / 64 * u + wave] = __popcll(b[u]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      int s = __popcll(b[u] & below);
+      for (int w = 0; w < kFB / 64 * u + wave; ++w) s += wcount[w];
+      if (on[u]) {
+        slot_of[kFB * u + t] = s;
+        plist[s] = kFB * u + t;
       }
-    nact = s;
+    }
+    if (t == 0) {
+      int s = 0;
+      for (int w = 0; w < 2 * kFB / 64; ++w) s += wcount[w];
+      nact = s;
+    }
   }
   __syncthreads();
   const int P = nact;
-  for (int k = t; k < kC3; k += kFB)
-    if (fidx[k] >= 0) atomicAdd(&ccount[slot_of[fidx[k]]], 1);
+  if (fidx[t] >= 0) atomicAdd(&ccount[slot_of[fidx[t]]], 1);
   __syncthreads();
-  if (t == 0) {
-    int s = 0;
-    for (int q = 0; q < P; ++q) {
-      cstart[q] = s;
-      s += ccount[q];
+  {
+    // exclusive sums of the points' channel counts (zero beyond P)
+    int v = ccount[t];
+    const int mine = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(v, o, 64);
+      if (lane >= o) v += u;
     }
-    cstart[P] = s;
+    if (lane == 63) wcount[wave] = v;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) v += wcount[w];
+    cstart[t] = v - mine;
+    if (t == kFB - 1) cstart[kC3] = v;
   }
   __syncthreads();
-  for (int k = t; k < kC3; k += kFB) {
-    if (fidx[k] < 0) continue;
+  if (fidx[t] >= 0) {
+    const int mine = fidx[t];
     int before = 0;
-    for (int k2 = 0; k2 < k; ++k2) before += (fidx[k2] == fidx[k]) ? 1 : 0;
-    corder[cstart[slot_of[fidx[k]]] + before] = k;
+    for (int k2 = 0; k2 < kC3; k2 += 4) {
+      const int4 o = *reinterpret_cast<const int4*>(fidx + k2);
+      before += (o.x == mine && k2 < t) + (o.y == mine && k2 + 1 < t) +
+                (o.z == mine && k2 + 2 < t) + (o.w == mine && k2 + 3 < t);
+    }
+    corder[cstart[slot_of[mine]] + before] = t;
   }
   __syncthreads();
   // layer 3 weights: dW3[ch][k] = dz3[ch] h2[argmax ch][k]
-  for (int i = t; i < kC3 * kC2; i += kFB) {
+#pragma unroll 8
+  for (int i = 4 * t; i < kC3 * kC2; i += 4 * kFB) {
     const int ch = i / kC2, k = i % kC2;
-    Gc[kW3 + i] = fidx[ch] >= 0 ? dz3[ch] * bf_val(H2c[(size_t)fidx[ch] * kC2 + k]) : 0.f;
+    const bool on = fidx[ch] >= 0;
+    const ushort4 h = *reinterpret_cast<const ushort4*>(H2c + (on ? fidx[ch] : 0) * kC2 + k);
+    const float z = dz3[ch];
+    store4(Gc + kW3 + i, on ? z * bf_val(h.x) : 0.f, on ? z * bf_val(h.y) : 0.f,
+           on ? z * bf_val(h.z) : 0.f, on ? z * bf_val(h.w) : 0.f);
   }
   if (t < kC3) Gc[kB3 + t] = dz3[t];
   // layer-2 weight fragments for dz1 = dz2 W2 (B operand: column k = 16 wave
   // + lr, rows j = 32 ks + 8 lg + e), BF16-rounded as in the forward pass
-  const int lane = t & 63, wave = t >> 6, lr = lane & 15, lg = lane >> 4;
+  const int lr = lane & 15, lg = lane >> 4;
   bf16x8 w2b[kC2 / 32];
 #pragma unroll
   for (int ks = 0; ks < kC2 / 32; ++ks) {
@@ -666,25 +718,50 @@ __global__ __launch_bounds__(kFB) void pn_bwd_kernel(
   for (int q0 = 0; q0 < P; q0 += kQT) {
     // dz2 of the tile's points (zero beyond P): the max-pool's channels of
     // each point back through W3, then ReLU'
-    for (int qi = qpar; qi < kQT; qi += kFB / kC2) {
-      const int q = q0 + qi;
-      float v = 0.f;
-      if (q < P) {
-        float sm = 0.f;
-        for (int r = cstart[q]; r < cstart[q + 1]; ++r) {
-          const int ch = corder[r];
-          sm += bf_round(prm[kW3 + ch * kC2 + jj]) * dz3[ch];
-        }
-        const float h2 = bf_val(H2c[(size_t)plist[q] * kC2 + jj]);
-        v = h2 > 0.f ? sm : 0.f;
+#pragma unroll
+    for (int qb = 0; qb < kQT; qb += kQB * kFB / kC2) {
+      // the activation and the first channel's weight of kQB points at once,
+      // then each point's other channels, four at a time
+      unsigned short h2b[kQB];
+      float w0[kQB], z0[kQB];
+#pragma unroll
+      for (int u = 0; u < kQB; ++u) {
+        const int q = min(q0 + qb + u * (kFB / kC2) + qpar, P - 1);
+        const int ch = corder[cstart[q]];
+        h2b[u] = H2c[(size_t)plist[q] * kC2 + jj];
+        w0[u] = prm[kW3 + ch * kC2 + jj];
+        z0[u] = dz3[ch];
       }
-      db2 += v;
-      const unsigned short hi = bf_bits(v);
-      const unsigned short lo = bf_bits(v - bf_val(hi));
-      zq_hi[qi * kSJ + jj] = hi;
-      zq_lo[qi * kSJ + jj] = lo;
-      zj_hi[jj * kSQ + qi] = hi;
-      zj_lo[jj * kSQ + qi] = lo;
+#pragma unroll
+      for (int u = 0; u < kQB; ++u) {
+        const int qi = qb + u * (kFB / kC2) + qpar, q = q0 + qi;
+        float v = 0.f;
+        if (q < P) {
+          float sm = 0.f;
+          sm += bf_round(w0[u]) * z0[u];
+          const int r1 = cstart[q + 1];
+          for (int r = cstart[q] + 1; r < r1; r += 4) {
+            float w[4], z[4];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              const int ch = corder[min(r + x, r1 - 1)];
+              w[x] = prm[kW3 + ch * kC2 + jj];
+              z[x] = dz3[ch];
+            }
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+              if (r + x < r1) sm += bf_round(w[x]) * z[x];
+          }
+          v = bf_val(h2b[u]) > 0.f ? sm : 0.f;
+        }
+        db2 += v;
+        const unsigned short hi = bf_bits(v);
+        const unsigned short lo = bf_bits(v - bf_val(hi));
+        zq_hi[qi * kSJ + jj] = hi;
+        zq_lo[qi * kSJ + jj] = lo;
+        zj_hi[jj * kSQ + qi] = hi;
+        zj_lo[jj * kSQ + qi] = lo;
+      }
     }
     for (int i = t; i < kQT * kC1; i += kFB) {
       const int qi = i / kC1, k = i % kC1, q = q0 + qi;

@@ -70,6 +70,31 @@ def test_forward_and_gradient_vs_oracle(ctx):
     assert rel < 3e-2 and cos > 0.999
 
 
+@pytest.mark.parametrize("n,spread", [(3, 1.0), (33, 1.0), (512, 1.0), (2000, 1.0), (64, 0.0)])
+def test_gradient_of_one_cluster(ctx, n, spread):
+    """The backward's list of active points and of their channels at its ends:
+    a point for all channels (coincident points), three, and as many as there
+    are.  Tolerance as for the batch above (BF16 activations)."""
+    d, t = _batch(1, seed=21)
+    rng = np.random.default_rng(n)
+    xyz = rng.normal(0.0, 1.0, (n, 3)) * spread * np.array([0.4, 0.4, 2.0]) + d["xyz"][0]
+    d = dict(xyz=xyz.astype(np.float32), offsets=np.array([0, n], np.int32))
+    p = proposal.init_params(seed=6)
+    print(f"[pn] gradient of one cluster of {n} points, spread {spread}", flush=True)
+    net = proposal.ProposalNet(ctx, p)
+    x, o, tt = _dev(d, t)
+    cfg = proposal.train_cfg()
+    loss, grad = net.loss_grad(x, o, tt, cfg)
+    ctx.sync()
+    rl, rg = oracle.pn_loss_grad(p, d["xyz"], d["offsets"], t,
+                                 weights=(cfg.w_axis, cfg.w_centre, cfg.w_radius), emulate=True)
+    assert np.linalg.norm(rg) > 0
+    assert np.allclose(loss.cpu().numpy(), rl, rtol=2e-2, atol=1e-4)
+    rel = np.linalg.norm(grad.cpu().numpy() - rg) / np.linalg.norm(rg)
+    print(f"[pn] gradient relative error {rel:.2e}", flush=True)
+    assert rel < 3e-2
+
+
 def test_training_reduces_loss(ctx):
     d, t = _batch(64, seed=12)
     net = proposal.ProposalNet(ctx, proposal.init_params(seed=5))
