@@ -44,7 +44,7 @@ constexpr int kS1 = kC1 + 8;         // LDS row strides (bf16), 16-byte multiple
 constexpr int kS2 = kC2 + 8;
 constexpr int kFB = 256;             // backward / prep workgroup
 constexpr int kFW = 512;             // forward workgroup (8 waves)
-constexpr int kHC = 8;               // clusters per head workgroup
+constexpr int kHeadSmall = 512;      // largest batch with 2 clusters per head workgroup
 
 // parameter offsets (weight [out][in], then bias)
 constexpr int kW1 = 0, kB1 = kW1 + kC1 * 3;
@@ -378,21 +378,22 @@ __global__ __launch_bounds__(kFW) void pn_fwd_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// head: 256 -> 128 (ReLU) -> 7 for kHC clusters per workgroup (each weight row
+// head: 256 -> 128 (ReLU) -> 7 for HC clusters per workgroup (each weight row
 // read once per workgroup), proposals in the world frame (prop nullable)
 // ---------------------------------------------------------------------------
+template <int HC>
 __global__ __launch_bounds__(kFB) void pn_head_kernel(const float* __restrict__ prm,
                                                       const PnMeta* __restrict__ meta,
                                                       int n_clusters,
                                                       const int32_t* __restrict__ d_n,
                                                       float* __restrict__ act,
                                                       float* __restrict__ prop) {
-  __shared__ float fs[kHC][kC3];
-  __shared__ float h4s[kHC][kC4];
-  __shared__ float outs[kHC][8];
+  __shared__ float fs[HC][kC3];
+  __shared__ float h4s[HC][kC4];
+  __shared__ float outs[HC][8];
   const int t = threadIdx.x;
-  const int c0 = blockIdx.x * kHC;
-  const int nc = min(kHC, pn_count(n_clusters, d_n) - c0);
+  const int c0 = blockIdx.x * HC;
+  const int nc = min(HC, pn_count(n_clusters, d_n) - c0);
   if (nc <= 0) return;
   for (int i = t; i < nc * kC3; i += kFB)
     fs[i / kC3][i % kC3] = act[(size_t)(c0 + i / kC3) * kAct + kAF + i % kC3];
@@ -402,9 +403,9 @@ __global__ __launch_bounds__(kFB) void pn_head_kernel(const float* __restrict__ 
   {
     const int o = t & (kC4 - 1);
     const int half = t / kC4;
-    float z[kHC];
+    float z[HC];
 #pragma unroll
-    for (int j = 0; j < kHC; ++j) z[j] = 0.f;
+    for (int j = 0; j < HC; ++j) z[j] = 0.f;
     const float4* w = reinterpret_cast<const float4*>(prm + kW4 + o * kC3 + half * (kC3 / 2));
     for (int q0 = 0; q0 < kC3 / 8; q0 += 16) {
       float4 wv[16];
@@ -418,24 +419,24 @@ __global__ __launch_bounds__(kFB) void pn_head_kernel(const float* __restrict__ 
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int j = 0; j < kHC; ++j) z[j] = __builtin_fmaf(wk[e], fs[j][k + e], z[j]);
+          for (int j = 0; j < HC; ++j) z[j] = __builtin_fmaf(wk[e], fs[j][k + e], z[j]);
       }
     }
     if (half == 1)
 #pragma unroll
-      for (int j = 0; j < kHC; ++j) h4s[j][o] = z[j];
+      for (int j = 0; j < HC; ++j) h4s[j][o] = z[j];
     __syncthreads();
     if (half == 0) {
       const float bias = bf_round(prm[kB4 + o]);
 #pragma unroll
-      for (int j = 0; j < kHC; ++j) {
+      for (int j = 0; j < HC; ++j) {
         const float v = bias + (z[j] + h4s[j][o]);
         h4s[j][o] = v > 0.f ? v : 0.f;
       }
     }
   }
   __syncthreads();
-  if (t < kOut * kHC) {
+  if (t < kOut * HC) {
     const int j = t / kOut, o = t % kOut;
     if (j < nc) {
       float z = bf_round(prm[kB5 + o]);
@@ -481,6 +482,17 @@ __global__ __launch_bounds__(kFB) void pn_head_kernel(const float* __restrict__ 
     pr[6] = ok ? r : 0.f;
     pr[7] = ok ? 1.f : 0.f;
   }
+}
+
+// The clusters of a head workgroup: 8 share a read of the weights in large
+// batches; where that leaves CUs idle, 2 (250 clusters: a training step 134 -> 129
+// us; 4096 clusters take 18 with 8).
+void launch_head(sloam_ctx* ctx, const float* prm, const PnMeta* meta, int n_clusters,
+                 const int32_t* d_n, float* act, float* prop) {
+  const int hc = n_clusters <= kHeadSmall ? 2 : 8;
+  auto kern = hc == 2 ? pn_head_kernel<2> : pn_head_kernel<8>;
+  hipLaunchKernelGGL(kern, dim3((n_clusters + hc - 1) / hc), dim3(kFB), 0, ctx->stream, prm, meta,
+                     n_clusters, d_n, act, prop);
 }
 
 // ---------------------------------------------------------------------------
@@ -964,8 +976,7 @@ int pn_loss_grad(sloam_ctx* ctx, const float* d_params, const float* d_xyz,
     SloamKernelScope ks(ctx, "pn_fwd");
     hipLaunchKernelGGL(pn_fwd_kernel<true>, dim3(fwd_grid(ctx, B)), dim3(kFW), 0, ctx->stream,
                        d_params, b->X, b->meta, B, (const int32_t*)nullptr, b->act, b->H1, b->H2);
-    hipLaunchKernelGGL(pn_head_kernel, dim3((B + kHC - 1) / kHC), dim3(kFB), 0, ctx->stream,
-                       d_params, b->meta, B, (const int32_t*)nullptr, b->act, (float*)nullptr);
+    launch_head(ctx, d_params, b->meta, B, nullptr, b->act, nullptr);
   }
   {
     SloamKernelScope ks(ctx, "pn_bwd");
@@ -1011,8 +1022,7 @@ static int pn_infer(sloam_ctx* ctx, const float* d_params, const float* d_xyz,
   }
   {
     SloamKernelScope ks(ctx, "pn_head");
-    hipLaunchKernelGGL(pn_head_kernel, dim3((n_clusters + kHC - 1) / kHC), dim3(kFB), 0,
-                       ctx->stream, d_params, b.meta, n_clusters, d_n, b.act, d_proposal);
+    launch_head(ctx, d_params, b.meta, n_clusters, d_n, b.act, d_proposal);
   }
   SLOAM_HIP(ctx, hipGetLastError());
   return SLOAM_OK;
