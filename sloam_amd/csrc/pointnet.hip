@@ -16,7 +16,8 @@
 //               columns 32w.. of layer 3), masked max-pool with the first
 //               maximising point kept per channel; persistent: a fixed grid
 //               loops over the clusters with the weight fragments loaded once
-//   pn_head     256 -> 128 -> 7 on the VALU for 8 clusters per workgroup
+//   pn_head     256 -> 128 -> 7 on the VALU for 8 (small batches: 2) clusters
+//               per workgroup
 //   pn_bwd      one workgroup per cluster: loss, head gradients, and the
 //               max-pool gradient routed to its argmax points only (at most
 //               256 of them), back through layers 3, 2, 1 from the
@@ -485,8 +486,8 @@ __global__ __launch_bounds__(kFB) void pn_head_kernel(const float* __restrict__ 
 }
 
 // The clusters of a head workgroup: 8 share a read of the weights in large
-// batches; where that leaves CUs idle, 2 (250 clusters: a training step 134 -> 129
-// us; 4096 clusters take 18 with 8).
+// batches; where that leaves CUs idle, 2 (a keyframe's trees 15 -> 9 us, 250
+// clusters 14 -> 9; 4096 clusters take 18 with 8).
 void launch_head(sloam_ctx* ctx, const float* prm, const PnMeta* meta, int n_clusters,
                  const int32_t* d_n, float* act, float* prop) {
   const int hc = n_clusters <= kHeadSmall ? 2 : 8;
