@@ -238,7 +238,10 @@ int sloam_cyl_fallback(sloam_ctx* ctx, const int32_t* d_offsets, int32_t n_clust
  * d_points, cylinders [cyl_offsets[k], ...) and planes [plane_offsets[k], ...).
  * d_points: 4 floats per residual: x, y, z (sensor frame) and the landmark
  *   reference as int32 bits: id >= 0 -> cylinder id, id < 0 -> plane -(id+1)
- *   (global indices into d_cyl / d_planes).
+ *   (global indices into d_cyl / d_planes).  A residual may name a landmark
+ *   listed under another problem of the plan; at precision 0 the two problems
+ *   must then start at the same translation (landmarks are held relative to
+ *   the initial translation of the problem that lists them).
  * d_cyl: 8 doubles per cylinder (map frame): root[3], ray[3], radius, unused.
  * d_planes: 4 doubles per plane (map frame): a, b, c, d of a x + b y + c z + d.
  * d_pose_in / d_pose_out: 7 doubles per problem: t[3], q[4] (x, y, z, w),

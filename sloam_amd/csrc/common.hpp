@@ -69,8 +69,10 @@ int sloam_project_noalloc_init(sloam_ctx* ctx);
 // max_problems): the fused LM kernel of sloam_pose_plan_exec over a work list
 // built on the device (d_work: int4 {problem, first residual, end residual, 0}
 // per chunk of at most 2048 residuals, d_first: first chunk of each problem).
-// d_cyl_tab / d_pl_tab take the landmark tables (per cylinder / plane: 32 / 16 bytes at cfg->precision
-// 0, 64 / 32 bytes at precision 1).
+// Every problem's residuals name its own landmarks only (each workgroup
+// prepares and reads its problem's part of the tables).  d_cyl_tab / d_pl_tab
+// take the landmark tables (per cylinder / plane: 32 / 16 bytes at
+// cfg->precision 0, 64 / 32 bytes at precision 1).
 int sloam_pose_fused_device(sloam_ctx* ctx, int max_problems, const int32_t* d_n_problems,
                             const float* d_points, const int32_t* d_work, const int32_t* d_first,
                             const double* d_cyl, const int32_t* d_cyl_off, const double* d_planes,

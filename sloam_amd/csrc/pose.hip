@@ -952,13 +952,17 @@ __global__ __launch_bounds__(64) void pose_solve_kernel(
 // fused: every iteration of one problem in one workgroup
 // --------------------------------------------------------------------------
 // d_n_problems (nullable): the problem count in device memory (a grid of
-// n_problems workgroups then serves any count up to n_problems).  The landmark
-// tables are written here and read back (no __restrict__): a preparation
-// launch of its own was 4.7 us and the gap after it.
+// n_problems workgroups then serves any count up to n_problems).
+// st (nullable): the states pose_prep left, with every problem's landmark
+// tables: residuals may name landmarks listed under another problem.  Without
+// it each workgroup prepares its own problem and reads only that back (no
+// __restrict__): for one problem, or several whose residuals are known to
+// name their own landmarks, where a preparation launch is 4.7 us and the gap
+// after it.
 template <bool F64>
 __global__ __launch_bounds__(kPBlock) void pose_fused_kernel(
     int n_problems, const int32_t* __restrict__ d_n_problems, PoseIn in,
-    const float4* __restrict__ pts, const int4* __restrict__ work,
+    const LMState* __restrict__ st, const float4* __restrict__ pts, const int4* __restrict__ work,
     const int32_t* __restrict__ first_work, void* cyl_tab, void* pl_tab, PoseCfgDev cfg,
     double* __restrict__ pose_out, int32_t* __restrict__ status, double* __restrict__ cost,
     double* __restrict__ params_out) {
@@ -968,7 +972,10 @@ __global__ __launch_bounds__(kPBlock) void pose_fused_kernel(
   __shared__ LMState sS;
   const int k = blockIdx.x;
   if (k >= n_problems || (d_n_problems && k >= *d_n_problems)) return;
-  pose_prep<F64>(k, in, cfg, &sS, cyl_tab, pl_tab);
+  if (!st)
+    pose_prep<F64>(k, in, cfg, &sS, cyl_tab, pl_tab);
+  else if (threadIdx.x < 64)
+    copy_state(&sS, st + k);
   __syncthreads();
   const int w0 = first_work[k], w1 = first_work[k + 1];
   for (int it = 0; it <= cfg.max_iters; ++it) {
@@ -1115,12 +1122,12 @@ namespace {
 
 template <bool F64>
 void launch_fused(sloam_ctx* ctx, int grid, const int32_t* d_n_problems, const PoseIn& in,
-                  const float* d_points, const int4* d_work, const int32_t* d_first,
+                  const LMState* st, const float* d_points, const int4* d_work, const int32_t* d_first,
                   void* cyl_tab, void* pl_tab, const PoseCfgDev& dc, double* d_pose_out,
                   int32_t* d_status, double* d_cost, double* d_params_out) {
   hipLaunchKernelGGL(pose_fused_kernel<F64>, dim3(grid), dim3(kPBlock), 0, ctx->stream, grid,
-                     d_n_problems, in, reinterpret_cast<const float4*>(d_points), d_work, d_first,
-                     cyl_tab, pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
+                     d_n_problems, in, st, reinterpret_cast<const float4*>(d_points), d_work,
+                     d_first, cyl_tab, pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
 }
 
 }  // namespace
@@ -1138,8 +1145,8 @@ int sloam_pose_fused_device(sloam_ctx* ctx, int max_problems, const int32_t* d_n
   const PoseIn in{d_pose_in, d_free_mask, d_cyl, d_cyl_off, d_planes, d_pl_off};
   const int4* work = reinterpret_cast<const int4*>(d_work);
   auto launch = cfg->precision == 1 ? launch_fused<true> : launch_fused<false>;
-  launch(ctx, max_problems, d_n_problems, in, d_points, work, d_first, d_cyl_tab, d_pl_tab, dc,
-         d_pose_out, d_status, d_cost, d_params_out);
+  launch(ctx, max_problems, d_n_problems, in, nullptr, d_points, work, d_first, d_cyl_tab,
+         d_pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
   SLOAM_HIP(ctx, hipGetLastError());
   return SLOAM_OK;
 }
@@ -1220,21 +1227,24 @@ int sloam_pose_plan_exec(sloam_pose_plan* p, const float* d_points, const double
   const PoseCfgDev dc = pose_cfg_dev(c);
   const bool f64 = c.precision == 1;
   const PoseIn in{d_pose_in, d_free_mask, d_cyl, d_cyl_offsets, d_planes, d_plane_offsets};
-  if (sloam_pose_plan_uses_fused(p)) {
-    SloamKernelScope ks(ctx, "pose_fused");
-    auto launch = f64 ? launch_fused<true> : launch_fused<false>;
-    launch(ctx, p->n_problems, nullptr, in, d_points, p->d_work, p->d_first, p->d_cyl_tab,
-           p->d_pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
-    SLOAM_HIP(ctx, hipGetLastError());
-    return SLOAM_OK;
-  }
-  {
+  const bool fused = sloam_pose_plan_uses_fused(p);
+  // one problem's workgroup prepares itself in the one launch
+  const bool prep = !fused || p->n_problems > 1;
+  if (prep) {
     SloamKernelScope ks(ctx, "pose_prep");
     auto kern = f64 ? pose_prep_kernel<true> : pose_prep_kernel<false>;
     hipLaunchKernelGGL(kern, dim3(p->n_problems), dim3(kPBlock), 0, ctx->stream, p->n_problems,
                        in, dc, p->d_state, p->d_cyl_tab, p->d_pl_tab);
+    SLOAM_HIP(ctx, hipGetLastError());
   }
-  SLOAM_HIP(ctx, hipGetLastError());
+  if (fused) {
+    SloamKernelScope ks(ctx, "pose_fused");
+    auto launch = f64 ? launch_fused<true> : launch_fused<false>;
+    launch(ctx, p->n_problems, nullptr, in, prep ? p->d_state : nullptr, d_points, p->d_work,
+           p->d_first, p->d_cyl_tab, p->d_pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
+    SLOAM_HIP(ctx, hipGetLastError());
+    return SLOAM_OK;
+  }
   // an evaluation makes the step of the one before it, from the other halves
   // of the state and partials buffers
   const bool joint = p->n_work <= kJointBlocks && p->max_chunks <= kJointChunks;
