@@ -76,10 +76,17 @@ __device__ inline int ground_cell(const float4& p, const GroundCfgDev& cfg) {
 constexpr int kSelCells = 255;   // cells (and the outside) are one 8-bit digit
 constexpr int kSelTile = 1024;   // points per workgroup of the partition
 constexpr int kSelWave = kSelTile / (kGB / 64);  // consecutive points per wave
-constexpr int kSelKeys = 4096;   // keys of a cell held in LDS
-constexpr int kSelCand = 2048;   // points sorted at once
+constexpr int kSelKeys = 4096;   // points of a cell whose keys are held in LDS
+constexpr int kSelCand = 2048;   // of them sorted at once
 constexpr int kSelBins = kGB;
 constexpr int kSelRank = 512;    // up to here sorted by counting smaller ones
+// larger cells: threads, bins of the threshold's search, points of its bin
+// that are sorted along, loads of a thread in flight
+constexpr int kBigB = 1024;
+constexpr int kBigW = kBigB / 64;
+constexpr int kBigBins = 2048;
+constexpr int kBigSlack = 8192;
+constexpr int kBigAhead = 16;
 // average points per cell up to which the selection is taken (more: two radix
 // sorts; a workgroup re-reads a larger cell from L2 several times)
 constexpr int kSelAvg = 16384;
@@ -210,28 +217,26 @@ struct GroundSel {
   int n_cand, bin, count, mode;
 };
 
-// The cell's first k points by (z, input order), k <= s, as input indices into
-// list.  Rounds of at most kSelCand points: the pending keys' range is cut
-// into 256 bins, the bins that reach k (or as many as fit) are gathered and
-// sorted as (key, position) pairs; a first bin that does not fit is cut
-// again, down to one key, whose points follow in input order.  The usual cell
-// (a few thousand points, 5 % kept) takes one round of ~100 candidates.
+// The first k points by (z, input order) of a cell of s <= kSelKeys points,
+// k <= s, as input indices into list.  Rounds of at most kSelCand points: the
+// pending keys' range is cut into 256 bins, the bins that reach k (or as many
+// as fit) are gathered and sorted as (key, position) pairs; a first bin that
+// does not fit is cut again, down to one key, whose points follow in input
+// order.  The usual cell (a few thousand points, 5 % kept) takes one round of
+// ~100 candidates.
 __device__ inline void ground_select(const uint32_t* __restrict__ gkey,
                                      const int32_t* __restrict__ gidx, int s, int k,
                                      int32_t* __restrict__ list, GroundSel& L) {
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const bool in_lds = s <= kSelKeys;
-  if (in_lds)
-    for (int i = t; i < s; i += kGB) L.keys[i] = gkey[i];
+  for (int i = t; i < s; i += kGB) L.keys[i] = gkey[i];
   __syncthreads();
-  auto key_at = [&](int i) -> uint32_t { return in_lds ? L.keys[i] : gkey[i]; };
   unsigned long long lo = 0;  // smallest pending key
   int done = 0;
   while (done < k) {
     const int rem = k - done;
     uint32_t kmin = 0xffffffffu, kmax = 0u;
     for (int i = t; i < s; i += kGB) {
-      const uint32_t q = key_at(i);
+      const uint32_t q = L.keys[i];
       if (q >= lo) {
         kmin = min(kmin, q);
         kmax = max(kmax, q);
@@ -264,7 +269,7 @@ __device__ inline void ground_select(const uint32_t* __restrict__ gkey,
       }
       __syncthreads();
       for (int i = t; i < s; i += kGB) {
-        const uint32_t q = key_at(i);
+        const uint32_t q = L.keys[i];
         if (q >= kmin && q <= kmax) atomicAdd(&L.hist[(q - kmin) >> shift], 1);
       }
       __syncthreads();
@@ -310,7 +315,7 @@ __device__ inline void ground_select(const uint32_t* __restrict__ gkey,
       int got = 0;
       for (int i0 = 0; i0 < s && got < rem; i0 += kGB) {
         const int i = i0 + t;
-        const bool f = i < s && key_at(i) == v;
+        const bool f = i < s && L.keys[i] == v;
         const uint64_t b = __builtin_amdgcn_ballot_w64(f);
         if (lane == 0) L.wtot[wave] = __builtin_popcountll(b);
         __syncthreads();
@@ -331,7 +336,7 @@ __device__ inline void ground_select(const uint32_t* __restrict__ gkey,
         min((unsigned long long)kmin + ((unsigned long long)(bin + 1) << shift),
             (unsigned long long)kmax + 1ull);
     for (int i = t; i < s; i += kGB) {
-      const uint32_t q = key_at(i);
+      const uint32_t q = L.keys[i];
       if (q >= kmin && q < bound) {
         const int o = atomicAdd(&L.n_cand, 1);
         L.cand[o] = ((unsigned long long)q << 32) | (unsigned)i;
@@ -370,6 +375,240 @@ __device__ inline void ground_select(const uint32_t* __restrict__ gkey,
     lo = bound;
     __syncthreads();
   }
+  __syncthreads();
+}
+
+struct GroundBig {
+  int hist[kBigBins];
+  int wc[kBigW][256];
+  uint32_t wmin[kBigW], wmax[kBigW];
+  int wtot[kBigW], bin, prev, count;
+};
+
+// Memory of a large cell's sort: two arrays of (key, position) pairs.
+struct GroundPairs {
+  uint32_t *key, *key2;
+  int32_t *pos, *pos2;
+};
+
+// inclusive wave scan
+__device__ inline int ground_scan(int v, int lane) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(v, o, 64);
+    if (lane >= o) v += u;
+  }
+  return v;
+}
+
+// Calls f(position, key) for the points [b, e) of a wave in order, 64 at a
+// time (key valid below e only), kBigAhead loads in flight.
+template <typename F>
+__device__ inline void ground_walk(const uint32_t* key, int b, int e, F f) {
+  const int lane = threadIdx.x & 63;
+  for (int i0 = b; i0 < e; i0 += 64 * kBigAhead) {
+    uint32_t q[kBigAhead];
+#pragma unroll
+    for (int u = 0; u < kBigAhead; ++u) q[u] = key[min(i0 + 64 * u + lane, e - 1)];
+#pragma unroll
+    for (int u = 0; u < kBigAhead; ++u)
+      if (i0 + 64 * u < e) f(i0 + 64 * u + lane, q[u]);
+  }
+}
+
+// The same for a cell of more than kSelKeys points, by kBigB threads, in a
+// bounded number of passes over the s keys whatever their distribution and k:
+// the range of the keys; the bin of the k-th key (cut again, at most twice,
+// while it holds more than kBigSlack points of more than one key; of one key
+// only the missing points are taken, the first in input order); the points up
+// to that bin in input order, each wave over consecutive ones; and a stable
+// sort of those, 8 bits a pass over the bits in which they differ.  Latency
+// and the LDS adds of one CU bound it (a pass over 262,144 keys 20 us, with
+// the adds 54).  262,144 points in one cell, 5 % kept, the whole call: 352 us;
+// in rounds of kSelCand points over all keys 4,709, by two radix sorts of the
+// cloud (ground_sort) 444.  65,536 points: 119 / 443 / 187.
+__device__ inline void ground_select_big(const uint32_t* __restrict__ gkey,
+                                         const int32_t* __restrict__ gidx, int s, int k,
+                                         int32_t* list, GroundPairs pairs, GroundBig& L) {
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const uint64_t below_lane = (1ull << lane) - 1ull;
+  // a wave's share of n points: consecutive, in multiples of 64
+  auto share = [&](int n, int& b, int& e) {
+    const int per = (n + kBigB - 1) / kBigB * 64;
+    b = min(n, wave * per);
+    e = min(n, b + per);
+  };
+  int wb, we;
+  share(s, wb, we);
+  // smallest and largest of the waves' values, on every thread
+  auto extremes = [&](uint32_t& a, uint32_t& b) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      a = min(a, (uint32_t)__shfl_xor((int)a, o, 64));
+      b = max(b, (uint32_t)__shfl_xor((int)b, o, 64));
+    }
+    if (lane == 0) {
+      L.wmin[wave] = a;
+      L.wmax[wave] = b;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kBigW; ++w) {
+      a = min(a, L.wmin[w]);
+      b = max(b, L.wmax[w]);
+    }
+  };
+  uint32_t kmin = 0xffffffffu, kmax = 0u;
+  ground_walk(gkey, wb, we, [&](int, uint32_t q) {  // past the end: the last key again
+    kmin = min(kmin, q);
+    kmax = max(kmax, q);
+  });
+  extremes(kmin, kmax);
+  // [lo, hi]: the bin of the k-th key, with `inside` points and `before`
+  // smaller ones
+  uint32_t lo = kmin, hi = kmax;
+  int before = 0, inside = s;
+  while (lo < hi && inside > kBigSlack && before + inside > k) {
+    const int shift = max(0, 21 - (int)__builtin_clz(hi - lo));  // ((hi - lo) >> shift) < kBigBins
+    for (int i = t; i < kBigBins; i += kBigB) L.hist[i] = 0;
+    __syncthreads();
+    uint32_t first = 0xffffffffu, last = 0u;
+    ground_walk(gkey, wb, we, [&](int i, uint32_t q) {
+      if (i < we && q >= lo && q <= hi) {
+        first = min(first, q);
+        last = max(last, q);
+        atomicAdd(&L.hist[(q - lo) >> shift], 1);
+      }
+    });
+    extremes(first, last);
+    if (first == last) {  // one key's points
+      lo = hi = first;
+      break;
+    }
+    constexpr int kPer = kBigBins / kBigB;
+    int h[kPer], mine = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      h[j] = L.hist[kPer * t + j];
+      mine += h[j];
+    }
+    int c = ground_scan(mine, lane);
+    if (lane == 63) L.wtot[wave] = c;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) c += L.wtot[w];
+    c += before - mine;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (c < k && c + h[j] >= k) {  // one thread finds it
+        L.bin = kPer * t + j;
+        L.prev = c;
+        L.count = h[j];
+      }
+      c += h[j];
+    }
+    __syncthreads();
+    before = L.prev;
+    inside = L.count;
+    lo += (uint32_t)L.bin << shift;
+    hi = min(hi, lo + ((1u << shift) - 1u));
+    __syncthreads();
+  }
+  __syncthreads();
+  // The smaller points and the bin's (of one key's only those missing), as
+  // (key - kmin, position), each wave's at the start of its own share.
+  int quota = inside;  // of the wave
+  if (lo == hi && before + inside > k) {
+    int n_in = 0;
+    ground_walk(gkey, wb, we, [&](int i, uint32_t q) {
+      n_in += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i < we && q == lo));
+    });
+    if (lane == 0) L.wtot[wave] = n_in;
+    __syncthreads();
+    quota = k - before;
+    for (int w = 0; w < wave; ++w) quota -= L.wtot[w];
+    quota = max(quota, 0);
+  }
+  int n = 0, n_in = 0;
+  ground_walk(gkey, wb, we, [&](int i, uint32_t q) {
+    const bool lt = i < we && q < lo, in = i < we && q >= lo && q <= hi;
+    const uint64_t bi = __builtin_amdgcn_ballot_w64(in);
+    const bool take = lt || (in && n_in + __builtin_popcountll(bi & below_lane) < quota);
+    const uint64_t bt = __builtin_amdgcn_ballot_w64(take);
+    const int dest = wb + n + __builtin_popcountll(bt & below_lane);
+    if (take) {
+      pairs.key[dest] = q - kmin;
+      pairs.pos[dest] = i;
+    }
+    n += __builtin_popcountll(bt);
+    n_in += __builtin_popcountll(bi);
+  });
+  const uint32_t range = hi - kmin;
+  const int bits = range ? 32 - (int)__builtin_clz(range) : 1;
+  int cb = wb, ce = wb + n;  // the wave's part of the pass's input
+  for (int bit = 0; bit < bits; bit += 8) {
+    for (int i = t; i < kBigW * 256; i += kBigB) L.wc[i >> 8][i & 255] = 0;
+    __syncthreads();  // the pairs, too
+    ground_walk(pairs.key, cb, ce, [&](int i, uint32_t q) {
+      if (i < ce) atomicAdd(&L.wc[wave][(q >> bit) & 255], 1);
+    });
+    __syncthreads();
+    int tot = 0;
+    if (t < 256) {
+#pragma unroll
+      for (int w = 0; w < kBigW; ++w) {
+        const int c = L.wc[w][t];
+        L.wc[w][t] = tot;
+        tot += c;
+      }
+    }
+    int off = ground_scan(tot, lane);
+    if (lane == 63) L.wtot[wave] = off;
+    __syncthreads();
+    if (t < 256) {
+      off -= tot;
+      for (int w = 0; w < wave; ++w) off += L.wtot[w];
+#pragma unroll
+      for (int w = 0; w < kBigW; ++w) L.wc[w][t] += off;
+    }
+    const int C = L.wtot[0] + L.wtot[1] + L.wtot[2] + L.wtot[3];
+    __syncthreads();
+    for (int i0 = cb; i0 < ce; i0 += 64 * kBigAhead) {
+      uint32_t qs[kBigAhead];
+      int32_t vs[kBigAhead];
+#pragma unroll
+      for (int u = 0; u < kBigAhead; ++u) {
+        const int i = min(i0 + 64 * u + lane, ce - 1);
+        qs[u] = pairs.key[i];
+        vs[u] = pairs.pos[i];
+      }
+#pragma unroll
+      for (int u = 0; u < kBigAhead; ++u) {
+        if (i0 + 64 * u >= ce) break;
+        const bool act = i0 + 64 * u + lane < ce;
+        const int d = (qs[u] >> bit) & 255;
+        uint64_t peers = __builtin_amdgcn_ballot_w64(act);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+          const uint64_t m = __builtin_amdgcn_ballot_w64(act && ((d >> b) & 1));
+          peers &= (d >> b) & 1 ? m : ~m;
+        }
+        const int r = __builtin_popcountll(peers & below_lane);
+        if (act) {
+          const int dest = L.wc[wave][d] + r;
+          __builtin_amdgcn_wave_barrier();
+          if (r == 0) L.wc[wave][d] += __builtin_popcountll(peers);
+          pairs.key2[dest] = qs[u];
+          pairs.pos2[dest] = vs[u];
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+    share(C, cb, ce);
+    pairs = {pairs.key2, pairs.key, pairs.pos2, pairs.pos};
+    __syncthreads();
+  }
+#pragma unroll 4
+  for (int j = t; j < k; j += kBigB) list[j] = gidx[pairs.pos[j]];
   __syncthreads();
 }
 
@@ -470,21 +709,23 @@ __device__ inline void gsum(double (&v)[K], double* lds) {
 // offsets (nullable): the cells' exclusive prefix of counts; without it
 // (few cells) each workgroup adds the counts of the cells before its own.
 // kSelect: by_idx and zkey are the points partitioned by cell, by_z receives
-// the cell's kept points where they are the lowest by z.
+// the cell's kept points where they are the lowest by z; pairs are the sort
+// buffers of the large cells, which all kBigB threads select (the first kGB do
+// the rest).
 template <bool kSelect>
-__global__ __launch_bounds__(kGB) void ground_fit_kernel(
+__global__ __launch_bounds__(kSelect ? kBigB : kGB) void ground_fit_kernel(
     const float4* __restrict__ pts, const int32_t* __restrict__ counts,
     const int32_t* __restrict__ offsets,
     const int32_t* __restrict__ by_idx, int32_t* __restrict__ by_z,
-    const uint32_t* __restrict__ zkey, GroundCfgDev cfg,
+    const uint32_t* __restrict__ zkey, GroundPairs pairs, GroundCfgDev cfg,
     int4* __restrict__ info, double* __restrict__ model, float4* __restrict__ features,
     int32_t* __restrict__ kept_index, int32_t* __restrict__ kept_offsets) {
   // the selection's memory serves the centroid's tiles afterwards
   struct Tiles {
     float v[3][kCentroidTile];
   };
-  constexpr size_t kLds = kSelect && sizeof(GroundSel) > sizeof(Tiles) ? sizeof(GroundSel)
-                                                                       : sizeof(Tiles);
+  constexpr size_t kLds =
+      kSelect ? std::max({sizeof(GroundSel), sizeof(GroundBig), sizeof(Tiles)}) : sizeof(Tiles);
   __shared__ __align__(16) unsigned char lds[kLds];
   float(*tile)[kCentroidTile] = reinterpret_cast<Tiles*>(lds)->v;
   __shared__ double red[(kGB / 64) * 6];
@@ -505,7 +746,20 @@ __global__ __launch_bounds__(kGB) void ground_fit_kernel(
     k = (int)((double)s / cfg.retain_num);
     k = min(k, s);
     list = by_z + off;
-    if constexpr (kSelect)
+  }
+  bool listed = false;  // kept_index holds the cell's points
+  if constexpr (kSelect) {
+    const bool reduced = cfg.retain_num < (double)s, big = reduced && s > kSelKeys;
+    if (big) {
+      ground_select_big(zkey + off, by_idx + off, s, k, by_z + off,
+                        {pairs.key + off, pairs.key2 + off, pairs.pos + off, pairs.pos2 + off},
+                        *reinterpret_cast<GroundBig*>(lds));
+      if (kept_index)
+        for (int j = threadIdx.x; j < s; j += kBigB) kept_index[off + j] = j < k ? list[j] : -1;
+      listed = true;
+    }
+    if (threadIdx.x >= kGB) return;  // no barrier waits for waves that ended
+    if (reduced && !big)
       ground_select(zkey + off, by_idx + off, s, k, by_z + off,
                     *reinterpret_cast<GroundSel*>(lds));
   }
@@ -513,7 +767,8 @@ __global__ __launch_bounds__(kGB) void ground_fit_kernel(
   double* out = model + 8 * (size_t)c;
   if (kept_index) {
     // the cell's kept points, in the order used (slots past k hold -1)
-    for (int j = threadIdx.x; j < s; j += kGB) kept_index[off + j] = j < k ? list[j] : -1;
+    if (!listed)
+      for (int j = threadIdx.x; j < s; j += kGB) kept_index[off + j] = j < k ? list[j] : -1;
     if (threadIdx.x == 0) {
       kept_offsets[c] = off;
       if (c == cfg.n_cells - 1) kept_offsets[cfg.n_cells] = off + s;
@@ -528,10 +783,11 @@ __global__ __launch_bounds__(kGB) void ground_fit_kernel(
   }
   // centroid: sequential float sums in list order (the reference's
   // computeCentroid), staged through LDS tiles
-  float sx = 0.f, sy = 0.f, sz = 0.f;
+  float sum = 0.f;  // lane 0: x, 1: y, 2: z
   for (int t0 = 0; t0 < k; t0 += kCentroidTile) {
     const int tn = min(kCentroidTile, k - t0);
     __syncthreads();
+#pragma unroll 4
     for (int j = threadIdx.x; j < tn; j += kGB) {
       const float4 p = pts[list[t0 + j]];
       tile[0][j] = p.x;
@@ -539,22 +795,30 @@ __global__ __launch_bounds__(kGB) void ground_fit_kernel(
       tile[2][j] = p.z;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int j = 0; j < tn; ++j) {
-        sx = sx + tile[0][j];
-        sy = sy + tile[1][j];
-        sz = sz + tile[2][j];
+    if (threadIdx.x < 3) {
+      const float* row = tile[threadIdx.x];
+      const float4* row4 = reinterpret_cast<const float4*>(row);
+      float4 v[4];  // the next sixteen
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = row4[u];
+      int j = 0;
+      for (; j + 16 <= tn; j += 16) {
+        const int ahead = min(j + 16, kCentroidTile - 16) / 4;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float4 q = v[u];
+          v[u] = row4[ahead + u];
+          sum = (((sum + q.x) + q.y) + q.z) + q.w;
+        }
       }
+      for (; j < tn; ++j) sum = sum + row[j];
     }
   }
-  if (threadIdx.x == 0) {
-    cen[0] = (float)((double)sx / (double)k);
-    cen[1] = (float)((double)sy / (double)k);
-    cen[2] = (float)((double)sz / (double)k);
-  }
+  if (threadIdx.x < 3) cen[threadIdx.x] = (float)((double)sum / (double)k);
   __syncthreads();
   const float cx = cen[0], cy = cen[1], cz = cen[2];
   double S[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll 2
   for (int j = threadIdx.x; j < k; j += kGB) {
     const float4 p = pts[list[j]];
     const double x = (double)(p.x - cx), y = (double)(p.y - cy), z = (double)(p.z - cz);
@@ -1214,11 +1478,14 @@ int sloam_ground_planes(sloam_ctx* ctx, const float* d_points, int32_t capacity,
   dc.ox = cfg->origin[0];
   dc.oy = cfg->origin[1];
   const int cap = std::max(capacity, 1);
-  // Partition by cell + selection per cell where the cells are one digit and a
-  // cell of average size keeps at most one round of candidates and is not so
-  // large that one workgroup's passes over it cost more than sorting
-  // (36 cells, 54,000 of 262,144 points, 5 % kept: 31 us in three launches
-  // against 117 in seventeen).
+  // Partition by cell + selection per cell where the cells are one digit and
+  // a cell of average size keeps at most one round of candidates and is not so
+  // large that one workgroup's passes over it cost more than sorting.  36
+  // cells, 5 % kept, 54,000 of 262,144 points: 51 us against 140; all 262,144:
+  // 68 / 156, and with all of them in one cell 352 / 444.  250 cells, all
+  // 500,000 points kept: 128 / 220, with 50,521 in one cell 836 / 1,080; 80
+  // cells, 1,048,576 points in one: 1,633 / 1,628.  (The worst seen: 262,144
+  // points of three heights in one cell, 447 / 421.)
   const bool select = capacity > 0 && n_cells <= kSelCells &&
                       (double)cap <= dc.retain_num * (double)kSelCand * (double)n_cells &&
                       (double)cap <= (double)kSelAvg * (double)n_cells;
@@ -1260,6 +1527,7 @@ int sloam_ground_planes(sloam_ctx* ctx, const float* d_points, int32_t capacity,
     uint8_t* cell = (uint8_t*)kA;
     int32_t* table = (int32_t*)kB;  // (n_cells + 1) rows of stride tiles
     uint32_t* zkey = (uint32_t*)kT;
+    const GroundPairs pairs{zkey + cap, (uint32_t*)kT2, vT, vT2};
     int bits = 1;
     while ((1 << bits) <= n_cells) ++bits;
     const float4* pts = reinterpret_cast<const float4*>(d_points);
@@ -1275,8 +1543,8 @@ int sloam_ground_planes(sloam_ctx* ctx, const float* d_points, int32_t capacity,
     }
     {
       SloamKernelScope ks(ctx, "ground_fit");
-      hipLaunchKernelGGL(ground_fit_kernel<true>, dim3(n_cells), dim3(kGB), 0, ctx->stream, pts,
-                         counts, offs, vA, vB, zkey, dc, reinterpret_cast<int4*>(d_cell_info),
+      hipLaunchKernelGGL(ground_fit_kernel<true>, dim3(n_cells), dim3(kBigB), 0, ctx->stream, pts,
+                         counts, offs, vA, vB, zkey, pairs, dc, reinterpret_cast<int4*>(d_cell_info),
                          d_cell_model, reinterpret_cast<float4*>(d_features), d_kept_index,
                          d_kept_offsets);
     }
@@ -1317,7 +1585,8 @@ int sloam_ground_planes(sloam_ctx* ctx, const float* d_points, int32_t capacity,
                          n_cells, offs);
     hipLaunchKernelGGL(ground_fit_kernel<false>, dim3(n_cells), dim3(kGB), 0, ctx->stream,
                        reinterpret_cast<const float4*>(d_points), counts,
-                       prefix ? offs : nullptr, by_idx, by_z, (const uint32_t*)nullptr, dc,
+                       prefix ? offs : nullptr, by_idx, by_z, (const uint32_t*)nullptr, GroundPairs{},
+                       dc,
                        reinterpret_cast<int4*>(d_cell_info), d_cell_model,
                        reinterpret_cast<float4*>(d_features), d_kept_index, d_kept_offsets);
   }

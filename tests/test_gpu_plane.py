@@ -176,3 +176,79 @@ def test_ground_planes_selection_rounds(ctx, n, retain, ties):
         b, k = g["kept_offsets"][c], o["info"][c, 1]
         assert len(np.unique(idx[b:b + k])) == k and np.all(idx[b:b + k] >= 0)
         assert np.all(idx[b + k:g["kept_offsets"][c + 1]] == -1)
+
+
+@pytest.mark.parametrize("retain", [0.05, 0.5, 1.0])
+@pytest.mark.parametrize("n,share,z", [
+    (4096, 1.0, "normal"), (4097, 1.0, "normal"), (70000, 1.0, "normal"), (70000, 0.9, "ties"),
+    (70000, 1.0, "flat"), (70000, 1.0, "wide"), (262144, 1.0, "normal"), (262144, 0.6, "ties")])
+def test_ground_planes_one_full_cell(ctx, n, share, z, retain):
+    """Clouds with most or all of their points in one cell, around the size up
+    to which a cell's keys are held in LDS and far above it: their selection is
+    a bounded number of passes.  z normal, in many ties, in one tie, and over
+    the floats' whole range (both signs, zeros of both, denormals).  Order and
+    sequential centroid as the oracle's.  (262,144 points at retain 0.5 and 1.0
+    take the radix sorts.)"""
+    rng = np.random.default_rng(n)
+    pts = np.zeros((n, 4), np.float32)
+    r = rng.uniform(16.0, 24.0, n)
+    th = np.where(rng.uniform(0, 1, n) < share, rng.uniform(0.05, 0.3, n),
+                  rng.uniform(-np.pi, np.pi, n))
+    pts[:, 0], pts[:, 1] = r * np.cos(th), r * np.sin(th)
+    pts[:, 2] = {"normal": lambda: rng.normal(-1.5, 0.3, n),
+                 "ties": lambda: np.where(rng.uniform(0, 1, n) < 0.5, -1.5,
+                                          np.round(rng.normal(-1.5, 0.3, n), 2)),
+                 "flat": lambda: np.full(n, -1.5),
+                 "wide": lambda: rng.choice([-1.0, 1.0, 0.0, -0.0], n) *
+                 10.0 ** rng.uniform(-42, 3, n)}[z]()
+    prm = dict(radii_bins=2, theta_bins=18, min_dist=5.0, max_dist=25.0, retain_thresh=retain,
+               num_features=5)
+    print(f"[ground] {n} points, {share} in one cell, z {z}, retain {retain}", flush=True)
+    g = ground_planes(ctx, pts, **prm)
+    o = oracle.ground_planes(pts, **prm)
+    assert np.array_equal(g["info"], o["info"])
+    valid = o["info"][:, 0] == 1
+    assert np.array_equal(g["model"][valid, 4:7], o["model"][valid, 4:7])
+    assert np.array_equal(g["features"][valid], o["features"][valid])
+    if z != "wide":  # of |z| over 45 decades the eigenvectors keep no common digits
+        assert np.allclose(g["model"][valid, :4], o["model"][valid, :4], atol=1e-9, rtol=0)
+    # kept points in increasing z, ties in input order
+    idx, first = g["kept_index"], g["kept_offsets"]
+    for c in np.flatnonzero(valid & (o["info"][:, 1] < o["info"][:, 2])):
+        kept = idx[first[c]:first[c] + o["info"][c, 1]]
+        zk = pts[kept, 2]
+        assert np.all((zk[1:] > zk[:-1]) | ((zk[1:] == zk[:-1]) & (kept[1:] > kept[:-1])))
+        assert np.all(idx[first[c] + len(kept):first[c + 1]] == -1)
+
+
+def test_ground_planes_work_is_bounded(ctx):
+    """262,144 points in one cell cost a small multiple of the same points in
+    36 even cells (5x; a selection that reads the whole cell again for every
+    2,048 kept points took 43x)."""
+    import time
+
+    import torch
+    from sloam_amd.gpu import ground_planes_dev
+    n = 262144
+    rng = np.random.default_rng(0)
+    r = rng.uniform(16.0, 24.0, n)
+    prm = dict(radii_bins=2, theta_bins=18, min_dist=5.0, max_dist=25.0, retain_thresh=0.05,
+               num_features=5)
+    took = {}
+    for name, th in (("even", rng.uniform(-np.pi, np.pi, n)), ("one", rng.uniform(0.05, 0.3, n))):
+        pts = np.zeros((n, 4), np.float32)
+        pts[:, 0], pts[:, 1] = r * np.cos(th), r * np.sin(th)
+        pts[:, 2] = rng.normal(-1.5, 0.3, n)
+        x = torch.as_tensor(pts).to(torch.device("cuda", ctx.device))
+        torch.cuda.synchronize()
+        out = ground_planes_dev(ctx, x, **prm)
+        ctx.sync()
+        ts = []
+        for _ in range(15):
+            t = time.perf_counter()
+            ground_planes_dev(ctx, x, out=out, **prm)
+            ctx.sync()
+            ts.append(time.perf_counter() - t)
+        took[name] = np.median(ts)
+        print(f"[ground] {n} points, {name}: {1e6 * took[name]:.0f} us", flush=True)
+    assert took["one"] < 15 * took["even"]
