@@ -203,7 +203,6 @@ __device__ inline void two_sum(float a, float b, float* s, float* e) {
 // prep: LM state init + landmark tables: FP32 relative to the anchor, or FP64
 // absolute (F64)
 // --------------------------------------------------------------------------
-// Of problem k by one workgroup: its landmarks' entries and its state S.
 struct PoseIn {
   const double* pose;
   const int32_t* free_mask;  // nullable
@@ -213,12 +212,18 @@ struct PoseIn {
   const int32_t* pl_off;
 };
 
+// By one workgroup: the entries of the landmarks listed under problems
+// [m0, m1), and the state S of problem k.
 template <bool F64>
-__device__ inline void pose_prep(int k, const PoseIn& in, const PoseCfgDev& cfg, LMState* S,
-                                 void* cyl_tab, void* pl_tab) {
-  const double* x0 = in.pose + 7 * (size_t)k;
-  const double ax = x0[0], ay = x0[1], az = x0[2];
-  for (int i = in.cyl_off[k] + (int)threadIdx.x; i < in.cyl_off[k + 1]; i += kPBlock) {
+__device__ inline void pose_prep(int k, int m0, int m1, const PoseIn& in, const PoseCfgDev& cfg,
+                                 LMState* S, void* cyl_tab, void* pl_tab) {
+  // anchor of the problem that lists landmark i
+  auto anchor = [&](const int32_t* off, int i) {
+    int m = m0;
+    while (m + 1 < m1 && i >= off[m + 1]) ++m;
+    return in.pose + 7 * (size_t)m;
+  };
+  for (int i = in.cyl_off[m0] + (int)threadIdx.x; i < in.cyl_off[m1]; i += kPBlock) {
     const double* c = in.cyl + 8 * (size_t)i;
     const double rn = sqrt(c[3] * c[3] + c[4] * c[4] + c[5] * c[5]);
     if constexpr (F64) {
@@ -227,30 +232,32 @@ __device__ inline void pose_prep(int k, const PoseIn& in, const PoseCfgDev& cfg,
       t[1] = make_double4(c[3] / rn, c[4] / rn, c[5] / rn, 0.0);
     } else {
       float4* t = static_cast<float4*>(cyl_tab) + 2 * (size_t)i;
-      t[0] = make_float4((float)(c[0] - ax), (float)(c[1] - ay), (float)(c[2] - az), (float)c[6]);
+      const double* a = anchor(in.cyl_off, i);
+      t[0] = make_float4((float)(c[0] - a[0]), (float)(c[1] - a[1]), (float)(c[2] - a[2]),
+                         (float)c[6]);
       t[1] = make_float4((float)(c[3] / rn), (float)(c[4] / rn), (float)(c[5] / rn), 0.f);
     }
   }
-  for (int i = in.pl_off[k] + (int)threadIdx.x; i < in.pl_off[k + 1]; i += kPBlock) {
+  for (int i = in.pl_off[m0] + (int)threadIdx.x; i < in.pl_off[m1]; i += kPBlock) {
     const double* q = in.pl + 4 * (size_t)i;
     const double nn = sqrt(q[0] * q[0] + q[1] * q[1] + q[2] * q[2]);
     if constexpr (F64) {
       static_cast<double4*>(pl_tab)[i] = make_double4(q[0] / nn, q[1] / nn, q[2] / nn, q[3] / nn);
     } else {
-      const double dr = (q[3] + q[0] * ax + q[1] * ay + q[2] * az) / nn;
+      const double* a = anchor(in.pl_off, i);
+      const double dr = (q[3] + q[0] * a[0] + q[1] * a[1] + q[2] * a[2]) / nn;
       static_cast<float4*>(pl_tab)[i] =
           make_float4((float)(q[0] / nn), (float)(q[1] / nn), (float)(q[2] / nn), (float)dr);
     }
   }
   if (threadIdx.x == 0) {
+    const double* x0 = in.pose + 7 * (size_t)k;
     LMState s;
     for (int i = 0; i < 7; ++i) {
       s.x[i] = x0[i];
       s.xe[i] = x0[i];
     }
-    s.anchor[0] = ax;
-    s.anchor[1] = ay;
-    s.anchor[2] = az;
+    for (int i = 0; i < 3; ++i) s.anchor[i] = x0[i];
     s.F0 = s.F = 0.0;
     for (int i = 0; i < 21; ++i) s.A[i] = 0.0;
     for (int i = 0; i < 6; ++i) s.g[i] = 0.0;
@@ -282,7 +289,7 @@ __global__ __launch_bounds__(kPBlock) void pose_prep_kernel(int n_problems, Pose
                                                             void* __restrict__ cyl_tab,
                                                             void* __restrict__ pl_tab) {
   const int k = blockIdx.x;
-  if (k < n_problems) pose_prep<F64>(k, in, cfg, st + k, cyl_tab, pl_tab);
+  if (k < n_problems) pose_prep<F64>(k, k, k + 1, in, cfg, st + k, cyl_tab, pl_tab);
 }
 
 // --------------------------------------------------------------------------
@@ -953,17 +960,19 @@ __global__ __launch_bounds__(64) void pose_solve_kernel(
 // --------------------------------------------------------------------------
 // d_n_problems (nullable): the problem count in device memory (a grid of
 // n_problems workgroups then serves any count up to n_problems).
-// st (nullable): the states pose_prep left, with every problem's landmark
-// tables: residuals may name landmarks listed under another problem.  Without
-// it each workgroup prepares its own problem and reads only that back (no
-// __restrict__): for one problem, or several whose residuals are known to
-// name their own landmarks, where a preparation launch is 4.7 us and the gap
-// after it.
-template <bool F64>
+// A residual may name a landmark listed under another problem, so one problem's
+// table entries alone are not enough.  kPrepared: the preparation launch made
+// the states st and every problem's entries (4.7 us and the gap after it).
+// Else each workgroup makes its own state and tables and reads them back (no
+// __restrict__): of all n_problems, in a copy of its own (copy_cyl, copy_pl
+// bytes; a plan of up to kTableCopies problems), or with own_only of its
+// problem, whose residuals are known to name no other's landmarks.
+template <bool F64, bool kPrepared>
 __global__ __launch_bounds__(kPBlock) void pose_fused_kernel(
     int n_problems, const int32_t* __restrict__ d_n_problems, PoseIn in,
-    const LMState* __restrict__ st, const float4* __restrict__ pts, const int4* __restrict__ work,
-    const int32_t* __restrict__ first_work, void* cyl_tab, void* pl_tab, PoseCfgDev cfg,
+    const float4* __restrict__ pts, const int4* __restrict__ work,
+    const int32_t* __restrict__ first_work, const LMState* __restrict__ st, bool own_only,
+    size_t copy_cyl, size_t copy_pl, void* cyl_tab, void* pl_tab, PoseCfgDev cfg,
     double* __restrict__ pose_out, int32_t* __restrict__ status, double* __restrict__ cost,
     double* __restrict__ params_out) {
   using E = PoseEval<F64>;
@@ -972,10 +981,14 @@ __global__ __launch_bounds__(kPBlock) void pose_fused_kernel(
   __shared__ LMState sS;
   const int k = blockIdx.x;
   if (k >= n_problems || (d_n_problems && k >= *d_n_problems)) return;
-  if (!st)
-    pose_prep<F64>(k, in, cfg, &sS, cyl_tab, pl_tab);
-  else if (threadIdx.x < 64)
-    copy_state(&sS, st + k);
+  if constexpr (kPrepared) {
+    if (threadIdx.x < 64) copy_state(&sS, st + k);
+  } else {
+    cyl_tab = static_cast<char*>(cyl_tab) + copy_cyl * k;
+    pl_tab = static_cast<char*>(pl_tab) + copy_pl * k;
+    pose_prep<F64>(k, own_only ? k : 0, own_only ? k + 1 : n_problems, in, cfg, &sS, cyl_tab,
+                   pl_tab);
+  }
   __syncthreads();
   const int w0 = first_work[k], w1 = first_work[k + 1];
   for (int it = 0; it <= cfg.max_iters; ++it) {
@@ -1016,6 +1029,7 @@ struct sloam_pose_plan {
   double* d_partials = nullptr;
   void* d_cyl_tab = nullptr;  // landmark tables (pose_prep_kernel), bytes
   void* d_pl_tab = nullptr;
+  size_t copy_cyl = 0, copy_pl = 0;  // bytes of one copy of each
   size_t cap_work = 0, cap_first = 0, cap_state = 0, cap_partials = 0, cap_cyl = 0, cap_pl = 0;
 };
 
@@ -1024,6 +1038,11 @@ namespace {
 // a problem set whose largest problem has at most this many chunks is solved
 // by pose_fused in AUTO mode
 constexpr int kFusedAutoChunks = 8;
+// Plans of up to this many problems hold a copy of the landmark tables per
+// problem, which pose_fused fills itself; larger ones share one, made by the
+// preparation launch.  A keyframe's two solves (10 trunks, 36 planes): 41.0 us,
+// with the launch 42.7.
+constexpr int kTableCopies = 4;
 // The evaluations make the LM steps themselves where all their workgroups run
 // at once (four a CU, so the step's latency is paid once) and a problem has
 // few chunks (every workgroup sums its problem's).  10 iterations, joint
@@ -1082,8 +1101,11 @@ int plan_build(sloam_pose_plan* p, const int32_t* h_res_offsets, int32_t n_probl
               sizeof(double));
   // landmark table entries: 2 float4 / 2 double4 per cylinder, 1 per plane
   const size_t tab = p->cfg.precision == 1 ? sizeof(double4) : sizeof(float4);
-  if (!st) st = grow(ctx, &p->d_cyl_tab, &p->cap_cyl, 2 * tab * (size_t)n_cylinders, 1);
-  if (!st) st = grow(ctx, &p->d_pl_tab, &p->cap_pl, tab * (size_t)n_planes, 1);
+  const size_t copies = n_problems <= kTableCopies ? n_problems : 1;
+  p->copy_cyl = 2 * tab * (size_t)n_cylinders;
+  p->copy_pl = tab * (size_t)n_planes;
+  if (!st) st = grow(ctx, &p->d_cyl_tab, &p->cap_cyl, copies * p->copy_cyl, 1);
+  if (!st) st = grow(ctx, &p->d_pl_tab, &p->cap_pl, copies * p->copy_pl, 1);
   if (st) return st;
   // the host vectors stay alive in the plan until the next build, which
   // synchronises the stream first
@@ -1120,14 +1142,18 @@ static PoseCfgDev pose_cfg_dev(const sloam_pose_cfg& c) {
 
 namespace {
 
+// st: what the preparation launch made; null: pose_fused prepares
 template <bool F64>
 void launch_fused(sloam_ctx* ctx, int grid, const int32_t* d_n_problems, const PoseIn& in,
-                  const LMState* st, const float* d_points, const int4* d_work, const int32_t* d_first,
+                  const float* d_points, const int4* d_work, const int32_t* d_first,
+                  const LMState* st, bool own_only, size_t copy_cyl, size_t copy_pl,
                   void* cyl_tab, void* pl_tab, const PoseCfgDev& dc, double* d_pose_out,
                   int32_t* d_status, double* d_cost, double* d_params_out) {
-  hipLaunchKernelGGL(pose_fused_kernel<F64>, dim3(grid), dim3(kPBlock), 0, ctx->stream, grid,
-                     d_n_problems, in, st, reinterpret_cast<const float4*>(d_points), d_work,
-                     d_first, cyl_tab, pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
+  auto kern = st ? pose_fused_kernel<F64, true> : pose_fused_kernel<F64, false>;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(kPBlock), 0, ctx->stream, grid, d_n_problems, in,
+                     reinterpret_cast<const float4*>(d_points), d_work, d_first, st, own_only,
+                     copy_cyl, copy_pl, cyl_tab, pl_tab, dc, d_pose_out, d_status, d_cost,
+                     d_params_out);
 }
 
 }  // namespace
@@ -1145,8 +1171,8 @@ int sloam_pose_fused_device(sloam_ctx* ctx, int max_problems, const int32_t* d_n
   const PoseIn in{d_pose_in, d_free_mask, d_cyl, d_cyl_off, d_planes, d_pl_off};
   const int4* work = reinterpret_cast<const int4*>(d_work);
   auto launch = cfg->precision == 1 ? launch_fused<true> : launch_fused<false>;
-  launch(ctx, max_problems, d_n_problems, in, nullptr, d_points, work, d_first, d_cyl_tab,
-         d_pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
+  launch(ctx, max_problems, d_n_problems, in, d_points, work, d_first, nullptr,
+         /*own_only=*/true, 0, 0, d_cyl_tab, d_pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
   SLOAM_HIP(ctx, hipGetLastError());
   return SLOAM_OK;
 }
@@ -1228,8 +1254,7 @@ int sloam_pose_plan_exec(sloam_pose_plan* p, const float* d_points, const double
   const bool f64 = c.precision == 1;
   const PoseIn in{d_pose_in, d_free_mask, d_cyl, d_cyl_offsets, d_planes, d_plane_offsets};
   const bool fused = sloam_pose_plan_uses_fused(p);
-  // one problem's workgroup prepares itself in the one launch
-  const bool prep = !fused || p->n_problems > 1;
+  const bool prep = !fused || p->n_problems > kTableCopies;
   if (prep) {
     SloamKernelScope ks(ctx, "pose_prep");
     auto kern = f64 ? pose_prep_kernel<true> : pose_prep_kernel<false>;
@@ -1240,8 +1265,9 @@ int sloam_pose_plan_exec(sloam_pose_plan* p, const float* d_points, const double
   if (fused) {
     SloamKernelScope ks(ctx, "pose_fused");
     auto launch = f64 ? launch_fused<true> : launch_fused<false>;
-    launch(ctx, p->n_problems, nullptr, in, prep ? p->d_state : nullptr, d_points, p->d_work,
-           p->d_first, p->d_cyl_tab, p->d_pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
+    launch(ctx, p->n_problems, nullptr, in, d_points, p->d_work, p->d_first,
+           prep ? p->d_state : nullptr, /*own_only=*/false, p->copy_cyl, p->copy_pl, p->d_cyl_tab,
+           p->d_pl_tab, dc, d_pose_out, d_status, d_cost, d_params_out);
     SLOAM_HIP(ctx, hipGetLastError());
     return SLOAM_OK;
   }

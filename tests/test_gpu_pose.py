@@ -143,24 +143,26 @@ def test_fused_matches_batched_bitwise(ctx, name, make, kw, precision):
 
 
 @pytest.mark.parametrize("precision", [0, 1], ids=["fp32", "fp64"])
-def test_landmarks_of_another_problem(ctx, precision):
+@pytest.mark.parametrize("n_prob", [2, 3, 4, 5, 9])
+def test_landmarks_of_another_problem(ctx, n_prob, precision):
     """Problems over one scan and one map whose landmarks are listed under the
-    other problems: both modes read every problem's tables, so the bits are
-    those of three problems solved alone.  One initial translation for all, as
-    precision 0 asks for (landmarks relative to their lister's)."""
+    first and last of them: both modes read every problem's tables (up to four
+    problems a copy each, made in the one launch), so the bits are those of the
+    problems solved alone.  One initial translation for all, as precision 0
+    asks for (landmarks relative to their lister's)."""
     one = synth.make_pose_problems(1, n_cyl=40, n_planes=12, seed=45)
     n, nc, npl = len(one["points"]), len(one["cyl"]), len(one["planes"])
-    pose = np.repeat(one["pose_init"], 3, axis=0)
-    for k in range(3):  # another initial rotation each
+    pose = np.repeat(one["pose_init"], n_prob, axis=0)
+    for k in range(n_prob):  # another initial rotation each
         pose[k, 3:] += 0.01 * k
         pose[k, 3:] /= np.linalg.norm(pose[k, 3:])
-    prob = dict(one, points=np.tile(one["points"], (3, 1)), pose_init=pose,
-                res_offsets=np.arange(4, dtype=np.int32) * n,
-                cyl_offsets=np.array([0, nc // 2, nc // 2, nc], np.int32),
-                plane_offsets=np.array([0, 0, 0, npl], np.int32))
+    prob = dict(one, points=np.tile(one["points"], (n_prob, 1)), pose_init=pose,
+                res_offsets=np.arange(n_prob + 1, dtype=np.int32) * n,
+                cyl_offsets=np.array([0] + [nc // 2] * (n_prob - 1) + [nc], np.int32),
+                plane_offsets=np.array([0] * n_prob + [npl], np.int32))
     kw = dict(max_iters=10, precision=precision)
-    print(f"[pose] shared landmarks, precision {precision}", flush=True)
-    alone = [solve_poses(ctx, dict(one, pose_init=pose[k:k + 1]), **kw) for k in range(3)]
+    print(f"[pose] {n_prob} problems, shared landmarks, precision {precision}", flush=True)
+    alone = [solve_poses(ctx, dict(one, pose_init=pose[k:k + 1]), **kw) for k in range(n_prob)]
     for mode in (1, 2):
         got = solve_poses(ctx, prob, mode=mode, **kw)
         for key in ("pose", "params", "status", "cost"):
