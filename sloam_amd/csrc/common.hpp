@@ -322,10 +322,12 @@ __host__ __device__ inline void sl_basis(const double a[3], double e1[3], double
 // rho = sqrt(x) and inv = 1 / rho, both correctly rounded, from one v_rsq and
 // a Newton step each with exact residuals (Markstein 1990) instead of the
 // compiler's separate square root and divide: 9 instructions and 3 compares
-// for about 25.  Equal to sqrtf(x) and 1.0f / sqrtf(x) at every float of
-// [2^-96, 2^96) where e is not 2^-24 (all 1.6e9 tried on the card; the one
-// exception there is a rho whose mantissa is all ones).  False for the other
-// x, 0, infinity and NaN among them: they take sl_sqrt_inv_any.
+// for about 25.  Equal to sqrtf(x) and 1.0f / sqrtf(x) wherever it returns
+// true, which is at every float of [2^-96, 2^96) but those with e = 2^-24 (37
+// a binade, of which one, the root whose mantissa is all ones, has a wrong
+// reciprocal): tests/cpp/sqrtinv_gpu.hip tries them all, on which this rests.
+// False for the others, 0, infinity and NaN among them: they take
+// sl_sqrt_inv_any.
 __device__ inline bool sl_sqrt_inv(float x, float& rho, float& inv) {
   const float y = __builtin_amdgcn_rsqf(x);
   const float g = x * y;

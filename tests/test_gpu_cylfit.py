@@ -85,11 +85,10 @@ def test_edge_clusters(ctx):
 
 
 def test_large_cluster_takes_per_step_refit(ctx):
-    """A batch holding a 40000-point cluster (20 refit chunks) is refitted
-    with one launch per Gauss-Newton step; without it, the same small batch
-    takes the fused refit (one workgroup per cluster: at most 512 clusters of
-    at most 4 chunks).  Both give the oracle's records bit for bit (the
-    2000-cluster test covers the per-step form at full size)."""
+    """A batch holding a 40000-point cluster (20 refit chunks): its clusters of
+    several chunks are refitted with one launch per Gauss-Newton step; without
+    it, every cluster (at most 4 chunks) has a workgroup that takes all steps.
+    Both give the oracle's records bit for bit."""
     rng = np.random.default_rng(12)
     big, _ = synth.trunk_points(rng, 40000, np.array([4.0, -2.0, 0.0]), np.array([0, 0, 1.0]),
                                 0.3, 8.0, 0.02, 0.2)
@@ -131,6 +130,27 @@ def test_refit_forms_at_their_edges(ctx, sizes):
                       mask=True, best=True)
     o = oracle.cyl_fit_batch(d["xyz"], d["offsets"], 96, samples=True, threads=8)
     assert (o["model"][:, 6] > 0).sum() >= len(pts) - 12 and o["model"][-1, 6] > 0
+    _compare(g, o, d["offsets"][-1])
+
+
+def test_many_clusters_of_many_chunks(ctx):
+    """420 clusters, 90 of them of 2 to 20 refit chunks: from 384 clusters on
+    the seed sums wait for cyl_axis in the memory of the refit's states, which
+    the launch per step then writes; and the chunks of many clusters share a
+    launch."""
+    rng = np.random.default_rng(23)
+    sizes = np.where(rng.uniform(0, 1, 420) < 90 / 420, rng.integers(2049, 40960, 420),
+                     rng.integers(0, 2049, 420))
+    sizes[[3, 200, 419]] = [40960, 8193, 4096]
+    pts = [synth.trunk_points(rng, int(n), np.array([5.0 + k % 9, 1.0, 0.0]),
+                              np.array([0.0, 0.05, 1.0]), 0.1 + 0.3 * (k % 5) / 4, 6.0, 0.02,
+                              0.25)[0] for k, n in enumerate(sizes)]
+    d = {"xyz": np.concatenate(pts).astype(np.float32),
+         "offsets": np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)}
+    _run_both(d, 64)
+    g = fit_cylinders(ctx, d["xyz"], d["offsets"], n_hyp=64, counts=True, mask=True, best=True)
+    o = oracle.cyl_fit_batch(d["xyz"], d["offsets"], 64, threads=16)
+    assert (o["model"][:, 6] > 0).sum() > 380
     _compare(g, o, d["offsets"][-1])
 
 

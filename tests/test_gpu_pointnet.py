@@ -8,6 +8,8 @@ activations to BF16, the oracle sums in FP64 and rounds the same
 activations; a last-bit difference before a BF16 rounding moves that
 activation by one BF16 step (2^-8 relative), so results agree to ~1e-2
 relative, not bit-exactly."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -122,12 +124,53 @@ def test_learned_pipeline_fallback_matches_plain(ctx, verify_rounds):
     flagged cluster ends with exactly the plain fit's model (its 3 refit
     rounds), every other one with exactly the verify-only fit's model
     (verify_rounds refit rounds)."""
-    d = synth.make_clusters(200, seed=13)
+    _learned_against_both(ctx, synth.make_clusters(200, seed=13), verify_rounds)
+
+
+@pytest.mark.parametrize("verify_rounds", [3, 1])
+def test_learned_pipeline_large_clusters(ctx, verify_rounds):
+    """The same on a batch whose clusters of over 8,192 points are refitted with
+    a launch per step (their schedules and hypotheses side by side with the
+    flagged ones'), and by a workgroup each in the rescue: large clusters among
+    the kept, the flagged and the rescued.  From 384 clusters on the seed sums
+    pass through the refit's states."""
+    rng = np.random.default_rng(31)
+    d = synth.make_clusters(360, seed=14, n_max=1500)
+    pts, sizes = [d["xyz"]], list(np.diff(d["offsets"]))
+    for k in range(60):
+        n = int(rng.integers(8193, 16000))
+        if k % 2:
+            # an outlier share around the half that the verification asks for
+            p, _ = synth.trunk_points(rng, n, np.array([5.0 + k % 7, 1.0, 0.0]),
+                                      np.array([0.0, 0.03, 1.0]), 0.25, 6.0, 0.02,
+                                      rng.uniform(0.1, 0.5))
+        else:
+            # two shells 9 cm apart: the band of a good hypothesis takes one
+            # and the edge of the other, and the refit, drawn to the inliers'
+            # mean, may lose some
+            r = np.where(rng.uniform(0, 1, n) < 0.5, 0.25, 0.34) + rng.normal(0, 0.012, n)
+            th = rng.uniform(-math.pi, math.pi, n)
+            p = np.stack([5.0 + r * np.cos(th), r * np.sin(th), rng.uniform(0, 6, n)], axis=1)
+        pts.append(p.astype(np.float32))
+        sizes.append(n)
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    flagged, rescued = _learned_against_both(
+        ctx, {"xyz": np.concatenate(pts), "offsets": off}, verify_rounds, ratio=0.54)
+    big = np.asarray(sizes) > 8192
+    print(f"[pn] large: flagged {int((flagged & big).sum())}, rescued "
+          f"{int((rescued & big).sum())} of {int(big.sum())}", flush=True)
+    assert min((flagged & big).sum(), (rescued & big).sum()) > 0
+    assert (big & ~flagged & ~rescued).sum() > 0
+
+
+def _learned_against_both(ctx, d, verify_rounds, ratio=0.5):
+    S = len(d["offsets"]) - 1
     x = torch.as_tensor(d["xyz"]).cuda()
     o = torch.as_tensor(d["offsets"].astype(np.int32)).cuda()
     net = proposal.ProposalNet(ctx, proposal.init_params(seed=6))
     fit = proposal.LearnedCylinderFit(ctx, net, d["offsets"], n_hyp=16, plain_hyp=256,
-                                      verify_refit_rounds=verify_rounds)
+                                      verify_refit_rounds=verify_rounds,
+                                      min_inlier_ratio=ratio)
     out = fit.alloc()
     fit.exec(x, o, out)
     plain = CylinderFitPlan(ctx, d["offsets"], n_hyp=256, stream_tag=0)
@@ -143,11 +186,12 @@ def test_learned_pipeline_fallback_matches_plain(ctx, verify_rounds):
     nf = int(out["n_fallback"].cpu().numpy()[0])
     n = np.diff(d["offsets"])
     best = vout["counts"].cpu().numpy().max(axis=1)
-    print(f"[pn] fallback {nf} of 200", flush=True)
-    decided = (n >= 3) & (best < 0.5 * n)
+    print(f"[pn] fallback {nf} of {S}", flush=True)
+    ratio = float(np.float32(ratio))  # as the entry takes it
+    decided = (n >= 3) & (best < ratio * n)
     # the rescue: kept by the verify stage, but its refit failed or kept
-    # fewer than half the points
-    rescued = ~decided & (n >= 3) & ~((vm[:, 6] > 0) & (vm[:, 7] >= 0.5 * n))
+    # fewer than that share of the points
+    rescued = ~decided & (n >= 3) & ~((vm[:, 6] > 0) & (vm[:, 7] >= ratio * n))
     print(f"[pn] decided {int(decided.sum())}, rescued {int(rescued.sum())}", flush=True)
     assert nf == act.sum() and nf > 0
     assert np.array_equal(act, decided | rescued)
@@ -156,6 +200,7 @@ def test_learned_pipeline_fallback_matches_plain(ctx, verify_rounds):
     fit.close()
     plain.close()
     verify.close()
+    return decided, rescued
 
 
 def test_two_pass_learned_pipeline_fallback_matches_plain(ctx):

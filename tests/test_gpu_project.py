@@ -71,3 +71,28 @@ def test_empty_and_all_nan(ctx):
     _same(g, o)
     g = project_partition(ctx, np.zeros((0, 4), np.float32), np.zeros(0, np.uint8), H=4, W=16)
     assert int(g["n_ground"][0]) == 0 and np.all(g["mask"] == 0)
+
+
+@pytest.mark.parametrize("n", [1 << 20, (1 << 20) + 1, 1_100_000])
+def test_more_points_than_the_scatter_sums(ctx, n):
+    """Up to 1,024 partition blocks (of 1,024 points) every scatter block adds
+    the counts before its own; above, a scan launch does.  A small image, the
+    points at their pixels' centres (no other pixel within rounding)."""
+    H, W = 32, 256
+    rng = np.random.default_rng(n)
+    row, col = rng.integers(0, H, n), rng.integers(0, W, n)
+    pitch = math.radians(45.0) * (1.0 - (row + 0.5) / H) - math.radians(22.5)
+    yaw = -math.pi * (2.0 * (col + 0.5) / W - 1.0)
+    r = rng.uniform(1.5, 60.0, n)
+    xyzi = np.empty((n, 4), np.float32)
+    xyzi[:, 0] = r * np.cos(pitch) * np.cos(yaw)
+    xyzi[:, 1] = r * np.cos(pitch) * np.sin(yaw)
+    xyzi[:, 2] = r * np.sin(pitch)
+    xyzi[:, 3] = rng.uniform(0, 1, n)
+    xyzi[::1000, 1] = np.nan
+    lab = rng.integers(0, 3, n).astype(np.uint8)
+    print(f"[proj] {n} points on {H}x{W}", flush=True)
+    g = project_partition(ctx, xyzi, lab, H=H, W=W)
+    o = oracle.project_partition(xyzi, lab, H=H, W=W)
+    _same(g, o)
+    assert n // 6 < int(g["n_ground"][0]) < n // 2

@@ -119,6 +119,32 @@ def test_components_across_tiles(ctx, H, W, fill):
     _same(g, o)
 
 
+@pytest.mark.parametrize("n_comps", [1024, 1025, 2049, 7140])
+def test_more_components_than_a_workgroup(ctx, n_comps):
+    """More kept components than the 1,024 that the layout and the assembly
+    take at once: their totals are carried from one part to the next.  Blocks
+    of 2 x 2 pixels, every one a tree of two vertices, with a lone pixel (not
+    kept) between some of them."""
+    H, W = 128, 512
+    rng = np.random.default_rng(n_comps)
+    cloud = np.full((H, W, 4), np.nan, np.float32)
+    r, c = np.divmod(rng.permutation(42 * 170)[:n_comps], 170)
+    for a in (0, 1):
+        for b in (0, 1):
+            cloud[3 * r + a, 3 * c + b, 0] = 5.0 + 0.01 * (3 * c + b)
+            cloud[3 * r + a, 3 * c + b, 1] = rng.normal(0.0, 0.02, n_comps)
+            cloud[3 * r + a, 3 * c + b, 2] = 1.0 - 0.05 * (3 * r + a)
+            cloud[3 * r + a, 3 * c + b, 3] = b
+    cloud[2 + 3 * r[::5], 2 + 3 * c[::5]] = [1.0, 0.0, 0.0, 0.0]  # 4 m from the blocks
+    cloud = cloud.reshape(H * W, 4)
+    kw = dict(min_label_points=2, min_row_points=1, min_vertices=1, max_vertices=40)
+    print(f"[trellis] {n_comps} components of {H}x{W}", flush=True)
+    g = trellis(ctx, cloud, H, W, max_dist_to_centroid=2.0, **kw)
+    o = oracle.trellis(cloud, H, W, max_dist=2.0, **kw)
+    assert len(o["tree_offsets"]) == n_comps + 1
+    _same(g, o)
+
+
 def test_empty_and_overflow(ctx):
     H, W = 8, 64
     cloud = np.full((H * W, 4), np.nan, np.float32)
