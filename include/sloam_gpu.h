@@ -295,10 +295,13 @@ int sloam_pose_plan_reset(sloam_pose_plan* plan, const int32_t* h_res_offsets,
                           const sloam_pose_cfg* cfg);
 /* Execution of sloam_pose_plan_exec:
  *   SLOAM_POSE_MODE_BATCHED: per LM iteration one residual/Jacobian kernel
- *     over 2048-residual chunks of every problem and one LM-step kernel
- *     (2 * (max_iters + 1) launches; for many or large problems);
+ *     over 2048-residual chunks of every problem, which makes the LM step of
+ *     the evaluation before it (max_iters + 3 launches); with more than 1024
+ *     chunks in all or 256 in one problem a kernel of its own makes the step
+ *     (2 * max_iters + 3 launches);
  *   SLOAM_POSE_MODE_FUSED: one workgroup per problem runs every iteration in
- *     one launch (for few small problems, e.g. one keyframe's solve);
+ *     one launch (for few small problems, e.g. one keyframe's solve; more than
+ *     four problems: after a preparation launch);
  *   SLOAM_POSE_MODE_AUTO (default): FUSED when no problem has more than
  *     8 chunks (16384 residuals), else BATCHED.
  * Both modes evaluate the same chunks in the same order and give

@@ -342,11 +342,14 @@ __global__ __launch_bounds__(64) void cyl_axis_kernel(const int32_t* __restrict_
 // and U' the next below U: one VALU instruction and one compare, as two
 // compares are, but one lane mask instead of two, so the scalar unit, shared
 // by the CU's four SIMDs, has two operations per 64 pairs (count, add) instead
-// of three (and).  The loop was bound by those: 19.5 cycles per 64 pairs and
-// SIMD against 15.5 now, 16 being the issue of its four VALU instructions.
-// 2000 clusters x 1024 hypotheses, 2.20e9 pairs: 255 -> 227 us.  (The product
-// on v_mfma_f32_4x4x1_16b, which rounds like fmaf, takes 18.5: it does not
-// overlap the VALU.)
+// of three (and).  2000 clusters x 1024 hypotheses, 2.20e9 pairs: 255 -> 227
+// us.  (The product on v_mfma_f32_4x4x1_16b, which rounds like fmaf, takes a
+// fifth longer: it does not overlap the VALU.)  Bound by VALU issue: the four
+// instructions alone, without scalar or LDS work, take 4.8 ns per 64 pairs and
+// SIMD (an FMA about two cycles, a clamp or compare about four, two waves' at
+// once in part; the clock falls to 2.2 GHz under them).  The whole kernel takes
+// 5.4 to 6.0 on 13.5e6 points, where an eighth of its vector instructions make
+// hypotheses and local coordinates, and 7.5 on 2.0e6 points.
 // work item = {cluster, first hypothesis, hypothesis count, unused}
 // LDS: hyp params [hcap] float4 | counts [hcap] int | u,v,s [tile] float
 // ---------------------------------------------------------------------------
@@ -1811,7 +1814,10 @@ static int plan_layout(sloam_cyl_plan* p, const int32_t* h_offsets, int32_t n_cl
     // no chunk asked for: 256 hypotheses a workgroup (each workgroup takes the
     // cluster's points into the local frame, for all its hypotheses), fewer
     // where that would leave CUs idle, down to one pass of each wave.  12
-    // trees x 1024 hypotheses: 48 workgroups took 34 us, 384 take 8.
+    // trees x 1024 hypotheses: 48 workgroups took 34 us, 384 take 8.  (Counted
+    // plans, laid out for their capacity, keep 256; a chunk that is asked for
+    // stays, as the 128 of the drop-in's tree fits and the autotuner's choices,
+    // of which 64 is the smallest.)
     const int least = kWaves * kHB;
     p->hcap = std::min(256, round_up(cfg.n_hyp, least));
     while (p->hcap > least &&
@@ -1971,10 +1977,6 @@ static int plan_layout(sloam_cyl_plan* p, const int32_t* h_offsets, int32_t n_cl
   if (tb) SLOAM_HIP(ctx, hipMemcpyAsync(p->d_tables, stage, tb, hipMemcpyHostToDevice, ctx->stream));
   return SLOAM_OK;
 }
-
-extern "C" {
-
-}  // extern "C"
 
 // A plan with cfg's launch shapes and no batch yet (nullptr when cfg is
 // invalid; *st says why).

@@ -1027,7 +1027,8 @@ __device__ inline PlFrame plane_frame(const float* __restrict__ box, int R, int 
 // 27,001 points x 200 hypotheses, and the largest patch of a batch set its
 // time (339 us at 300 sets of 40..20,000 points); in chunks of 1,024 points x
 // 64 hypotheses the two take 10.7 us (launch and gather latency) and 29 us
-// (16 us of VALU issue: 3 FMA + 1 compare per point and hypothesis).
+// (17 us of VALU issue, 12 of them the 3 FMA + 1 compare per point and
+// hypothesis).
 __global__ __launch_bounds__(kPlB) void plane_score_kernel(
     const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
     const float* __restrict__ box, const int2* __restrict__ set_chunks,
@@ -1269,11 +1270,6 @@ __device__ inline int plane_sum_int(int v, int* red) {
   return t;
 }
 
-// What the refit's kernels hand on for a set of several chunks.
-struct PlState {
-  PlHyp h;  // the best hypothesis
-};
-
 // model: plane[4] (unit normal, z >= 0 orientation), centroid[3], inliers of
 // the refitted plane.
 //
@@ -1285,7 +1281,7 @@ __global__ __launch_bounds__(kPlB) void plane_refit_kernel(
     const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
     const PlFrame* __restrict__ frames, const PlChunk* __restrict__ chunks,
     const int32_t* __restrict__ counts, int n_hyp, float thr, uint32_t k0, uint32_t k1,
-    uint32_t tag, double* __restrict__ part, PlState* __restrict__ state,
+    uint32_t tag, double* __restrict__ part, PlHyp* __restrict__ best_hyp,
     uint32_t* __restrict__ mask, int32_t* __restrict__ best_out, double* __restrict__ model) {
   __shared__ double red[kPlW * 6];
   __shared__ long long redk[kPlW];
@@ -1311,7 +1307,7 @@ __global__ __launch_bounds__(kPlB) void plane_refit_kernel(
     }
     if (ck.index() == 0) {
       if (best_out) best_out[c] = best;
-      state[c].h = best_h;
+      best_hyp[c] = best_h;
     }
   }
   __syncthreads();
@@ -1381,7 +1377,7 @@ __global__ __launch_bounds__(kPlB) void plane_refit_kernel(
 __global__ __launch_bounds__(kPlB) void plane_finish_kernel(
     const float* __restrict__ xyz, const int32_t* __restrict__ offsets,
     const PlFrame* __restrict__ frames, const int2* __restrict__ set_chunks,
-    const PlChunk* __restrict__ chunks, float thr, const PlState* __restrict__ state,
+    const PlChunk* __restrict__ chunks, float thr, const PlHyp* __restrict__ best_hyp,
     const double* __restrict__ part, int2* __restrict__ arrived, double* __restrict__ model) {
   __shared__ double red[kPlW * 6];
   __shared__ int redi[kPlW];
@@ -1399,7 +1395,7 @@ __global__ __launch_bounds__(kPlB) void plane_finish_kernel(
   for (int i = 0; i < 6; ++i) S[i] = mine ? sp[4 + i] : 0.0;
   plane_sum<4>(acc, red);
   const double k = acc[3];
-  if (k < 3.0 || !state[ck.set].h.valid) {
+  if (k < 3.0 || !best_hyp[ck.set].valid) {
     if (ck.index() == 0 && threadIdx.x == 0) {
       for (int i = 0; i < 7; ++i) out[i] = 0.0;
       out[7] = k;
@@ -1445,7 +1441,7 @@ struct sloam_plane_plan {
   int2* d_sets = nullptr;        // per set {first refit chunk, refit chunks}
   float* d_box = nullptr;        // 6 per refit chunk
   double* d_part = nullptr;      // 10 per refit chunk: centroid sums, covariance
-  PlState* d_state = nullptr;
+  PlHyp* d_best_hyp = nullptr;   // per set, what the refit hands to the finish
   int2* d_arrived = nullptr;     // per set {inliers, chunks done}
   PlFrame* d_frames = nullptr;
   int32_t* d_counts = nullptr;
@@ -1647,7 +1643,7 @@ int sloam_plane_plan_create(sloam_ctx* ctx, const int32_t* h_offsets, int32_t n_
   auto al = [](size_t x) { return (x + 255) / 256 * 256; };
   const size_t sb = al(sizeof(PlChunk) * score.size()), rb = al(sizeof(PlChunk) * refit.size()),
                tb = al(sizeof(int2) * sets.size()), bb = al(sizeof(float) * 6 * refit.size()),
-               pb = al(sizeof(double) * 10 * refit.size()), hb = al(sizeof(PlState) * n_sets),
+               pb = al(sizeof(double) * 10 * refit.size()), hb = al(sizeof(PlHyp) * n_sets),
                ab = al(sizeof(int2) * n_sets), fb = al(sizeof(PlFrame) * n_sets),
                cb = al(sizeof(int32_t) * (size_t)n_sets * cfg->n_hyp);
   int st = sloam_dev_alloc(ctx, &p->d_mem, sb + rb + tb + bb + pb + hb + ab + fb + cb);
@@ -1674,7 +1670,7 @@ int sloam_plane_plan_create(sloam_ctx* ctx, const int32_t* h_offsets, int32_t n_
   p->d_sets = (int2*)take(tb);
   p->d_box = (float*)take(bb);
   p->d_part = (double*)take(pb);
-  p->d_state = (PlState*)take(hb);
+  p->d_best_hyp = (PlHyp*)take(hb);
   p->d_arrived = (int2*)take(ab);
   p->d_frames = (PlFrame*)take(fb);
   p->d_counts = (int32_t*)take(cb);
@@ -1719,10 +1715,10 @@ int sloam_plane_plan_exec(sloam_plane_plan* p, const float* d_xyz, const int32_t
     SloamKernelScope ks(ctx, "plane_refit");
     hipLaunchKernelGGL(plane_refit_kernel, chunks, block, 0, ctx->stream, d_xyz, d_offsets,
                        p->d_frames, p->d_refit, counts, H, thr, k0, k1, tag, p->d_part,
-                       p->d_state, d_mask, d_best, d_model);
+                       p->d_best_hyp, d_mask, d_best, d_model);
     if (p->multi)
       hipLaunchKernelGGL(plane_finish_kernel, chunks, block, 0, ctx->stream, d_xyz, d_offsets,
-                         p->d_frames, p->d_sets, p->d_refit, thr, p->d_state, p->d_part,
+                         p->d_frames, p->d_sets, p->d_refit, thr, p->d_best_hyp, p->d_part,
                          p->d_arrived, d_model);
   }
   SLOAM_HIP(ctx, hipGetLastError());

@@ -22,7 +22,7 @@
 //               partials in chunk order, then the same LM step in its first
 //               wave, so its results are bit-identical to the loop's.  It
 //               serves small problems (a keyframe's solve), where the loop's
-//               max_iters + 2 launches cost more than the work.
+//               max_iters + 3 launches cost more than the work.
 // Coordinates are evaluated relative to a per-problem anchor (the initial
 // translation) so that FP32 residuals keep sub-micrometre resolution.
 //
@@ -333,8 +333,10 @@ __device__ inline void eval_frame(const LMState& s, int param, EvalFrame& F) {
 // kPBlock threads: thread t takes residuals b + j * kPBlock + t.  Returns the
 // chunk's 28 sums as FP64 (sum + compensation) in threads 0..27.
 //
-// The kernel is bound by VALU issue (~160 instructions per residual against
-// 16 bytes of HBM).  kSub false (the quaternion parametrization, all
+// VALU work is the largest part (~125 instructions per residual and ~410 per
+// wave for the frame and the sums: 7 us of issue in 12.5 at 64 problems of
+// 31000 residuals; the rest is the loads' and the reduction's latency; 16 bytes
+// of HBM per residual are 6.5).  kSub false (the quaternion parametrization, all
 // parameters free) drops the left-Jacobian map and the masks, whose identity
 // and unit factors change no bit.  The divides and the square root stay
 // correctly rounded (a root and its reciprocal from one v_rsq): the hardware
@@ -1035,8 +1037,12 @@ struct sloam_pose_plan {
 
 namespace {
 
-// a problem set whose largest problem has at most this many chunks is solved
-// by pose_fused in AUTO mode
+// A problem set whose largest problem has at most this many chunks is solved
+// by pose_fused in AUTO mode.  The line was drawn when an iteration of the
+// batched form was two launches; with the joint form below it lies at two
+// chunks (10 iterations of 1, 2, 3, 5, 8 chunks in FP32: fused 66, 100, 143,
+// 231, 392 us against batched 87, 104, 109, 111, 113; FP64 74, 126, 199, 343,
+// 616 against 101, 136, 142, 144, 147; the same from 1 to 16 problems).
 constexpr int kFusedAutoChunks = 8;
 // Plans of up to this many problems hold a copy of the landmark tables per
 // problem, which pose_fused fills itself; larger ones share one, made by the
