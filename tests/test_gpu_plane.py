@@ -113,10 +113,11 @@ def test_plane_ransac_chunks(ctx, sizes, n_hyp):
 @pytest.mark.parametrize("n,bins", [(3000, (1, 1)), (30000, (1, 4)), (40000, (1, 1))],
                          ids=["3000-one-cell", "30000-four-cells", "40000-one-cell"])
 def test_ground_planes_bottom_k_order(ctx, n, bins):
-    """The bottom-k order by (z, input order) of the (cell, z) radix sort.  z
-    is quantised to 1 cm so that many points tie, -0 and +0 among them (equal
-    under <, so input order decides); the kept points and the features must
-    come out in the oracle's order."""
+    """The bottom-k order by (z, input order) of the selection per cell, and of
+    the (cell, z) radix sort (40,000 points in one cell).  z is quantised to 1
+    cm so that many points tie, -0 and +0 among them (equal under <, so input
+    order decides); the kept points and the features must come out in the
+    oracle's order."""
     rng = np.random.default_rng(n)
     r = 25.0 * np.sqrt(rng.uniform(0.0, 1.0, n))
     th = rng.uniform(-np.pi, np.pi, n)
@@ -143,11 +144,10 @@ def test_ground_planes_bottom_k_order(ctx, n, bins):
 @pytest.mark.parametrize("ties", ["none", "some", "most"])
 def test_ground_planes_selection_rounds(ctx, n, retain, ties):
     """The per-cell selection (few cells) where one cell holds most of the
-    points: cells larger than the keys held in LDS (4,096), more kept points
-    than one round sorts (2,048), more ties of one z than that, and scans of a
-    few points.  At retain 1.0 the larger clouds take the radix sorts.  The
-    float centroid is a sequential sum, so it is equal only if every kept
-    point comes in the oracle's order."""
+    points: cells up to the keys held in LDS (4,096) in rounds, with more kept
+    points than one round sorts (2,048) and more ties of one z than that;
+    larger cells; and scans of a few points.  The float centroid is a sequential
+    sum, so it is equal only if every kept point comes in the oracle's order."""
     rng = np.random.default_rng(n)
     r = rng.uniform(6.0, 24.0, n)
     th = np.where(rng.uniform(0, 1, n) < 0.85, rng.uniform(0.05, 0.3, n),
@@ -180,8 +180,9 @@ def test_ground_planes_selection_rounds(ctx, n, retain, ties):
 
 @pytest.mark.parametrize("retain", [0.05, 0.5, 1.0])
 @pytest.mark.parametrize("n,share,z", [
-    (4096, 1.0, "normal"), (4097, 1.0, "normal"), (70000, 1.0, "normal"), (70000, 0.9, "ties"),
-    (70000, 1.0, "flat"), (70000, 1.0, "wide"), (262144, 1.0, "normal"), (262144, 0.6, "ties")])
+    (4096, 1.0, "normal"), (4096, 1.0, "flat"), (4096, 1.0, "ties"), (4097, 1.0, "normal"),
+    (70000, 1.0, "normal"), (70000, 0.9, "ties"), (70000, 1.0, "flat"), (70000, 1.0, "wide"),
+    (262144, 1.0, "normal"), (262144, 0.6, "ties")])
 def test_ground_planes_one_full_cell(ctx, n, share, z, retain):
     """Clouds with most or all of their points in one cell, around the size up
     to which a cell's keys are held in LDS and far above it: their selection is

@@ -130,8 +130,8 @@ FUSED_CASES = [
 @pytest.mark.parametrize("name,make,kw", FUSED_CASES, ids=[c[0] for c in FUSED_CASES])
 def test_fused_matches_batched_bitwise(ctx, name, make, kw, precision):
     """The one-launch LM kernel evaluates the same chunks in the same order and
-    runs the same step: every output equals the two-kernel loop's bit for bit,
-    in either evaluation precision."""
+    runs the same step: every output equals the batched loop's bit for bit, in
+    either evaluation precision."""
     prob = make()
     print(f"[pose] fused vs batched: {name}, precision {precision}, "
           f"{len(prob['res_offsets']) - 1} problems, {prob['res_offsets'][-1]} residuals",
